@@ -386,7 +386,7 @@ def train_bench(args) -> int:
     probe, nprobe = eng.read_probe_backward()
     eng.set_probe(-1)
     # Roofline kernel: layer 1's QKV weight-gradient GEMM (dWqkv += dqkv^T . n1,
-    # 2 * 2304 * 768 flop per token; 2304 x 768 output in 64 x 192 tiles, run
+    # 2 * 2304 * 768 flop per token; 2304 x 768 output in 64 x 128 tiles, run
     # unsplit over the tokens), timed with HIP events on
     # the weight-gradient stream; it shares the GPU with the main stream's
     # kernels while it runs.
@@ -417,8 +417,8 @@ def train_bench(args) -> int:
         "loss_first_last": [round(losses[0], 5), round(losses[-1], 5)],
         "backward_probe_ms_per_launch": {k: round(v / max(nprobe, 1), 5) for k, v in probe.items()},
         "dgrad_qkv_tflops": round(qkv_flop / dg_s / 1e12, 2) if dg_s > 0 else None,
-        "roofline": {"kernel": "gemm_nt_kernel<bf16,64,192,128,4,EPI_F32> accumulating into the gradient (one "
-                               "split: 144 tiles): layer 1 dWqkv (weight-gradient stream, concurrent with the main "
+        "roofline": {"kernel": "gemm_nt_kernel<bf16,64,128,128,5,EPI_F32> accumulating into the gradient (one "
+                               "split: 216 tiles): layer 1 dWqkv (weight-gradient stream, concurrent with the main "
                                "stream)",
                      "bound": "mfma", "achieved": round(qkv_flop / wg_s / 1e12, 2) if wg_s > 0 else None,
                      "peak": PEAK[args.precision] / 1e12, "unit": "TFLOP/s",
@@ -1028,7 +1028,7 @@ def summarize_traffic(fetch_dir: str, write_dir: str, out_path: str) -> int:
         m = re.findall(r"Li(\d+)E", tail)
         if not m:
             m = re.findall(r"(?<=[<,\s])(\d+)(?=[,>])", tail.split(">")[0] + ">")
-        return tuple(int(x) for x in m)
+        return tuple(int(x) for x in m)[:8]  # the main-loop form and the statistics' columns follow
 
     fetch, write = per_dispatch(fetch_dir, "FETCH_SIZE"), per_dispatch(write_dir, "WRITE_SIZE")
     copy_bytes = 512 << 20

@@ -226,13 +226,11 @@ bool fold_geometry(const dn_ctx *c) {
 
 bool fold_eligible(const dn_ctx *c, int T) {
   const Config &g = c->cfg;
-  return c->ln_fold && c->fold_cs.p && !g.generic && gemm_ln_fold_ok(g.precision, T, g.hidden, g.inter);
+  return (c->ln_fold || T <= kFoldSwitchTokens) && c->fold_cs.p && !g.generic &&
+         gemm_ln_fold_ok(g.precision, T, g.hidden, g.inter);
 }
 
-size_t fold_bytes_per_token(const dn_ctx *c) {
-  if (!fold_geometry(c)) return 0;
-  return sizeof(float) * 2 * (c->cfg.hidden / kLnPartCols) + sizeof(float) * 2;
-}
+size_t fold_bytes_per_token(const dn_ctx *c) { return fold_geometry(c) ? sizeof(float) * 2 : 0; }
 
 // The consumer GEMMs' column sums of layer l: QKV's (attn_norm, layers >= 1)
 // at fold_cs + l * (3H + 2I), Wi's (mlp_norm) 3H further.
@@ -246,23 +244,33 @@ int ensure_fold_cs(dn_ctx *c, hipStream_t s) {
   if (!c->fold_cs.p || c->fold_gen == c->wgen) return DN_OK;
   const Config &g = c->cfg;
   const int H = g.hidden, I = g.inter;
+  FoldJobs jobs{};
+  jobs.K = H;
+  auto flush = [&]() -> int {
+    HIPCHK(c, "fold_colsum", launch_fold_colsum(g.precision, jobs, s));
+    jobs.n = 0;
+    return DN_OK;
+  };
   for (int l = 0; l < g.layers; l++) {
     const std::string pf = layer_prefix(l);
+    if (jobs.n + 2 > kFoldJobs) {
+      const int rc = flush();
+      if (rc) return rc;
+    }
     if (l > 0)
-      HIPCHK(c, "fold_colsum", launch_fold_colsum(g.precision, W(c, pf + "attn.Wqkv.weight"), 3 * H, H,
-                                                  (const float *)W(c, pf + "attn_norm.weight"), fold_cs_qkv(c, l), s));
-    HIPCHK(c, "fold_colsum", launch_fold_colsum(g.precision, W(c, pf + "mlp.Wi.weight"), 2 * I, H,
-                                                (const float *)W(c, pf + "mlp_norm.weight"), fold_cs_wi(c, l), s));
+      jobs.job[jobs.n++] = {W(c, pf + "attn.Wqkv.weight"), (const float *)W(c, pf + "attn_norm.weight"),
+                            fold_cs_qkv(c, l), 3 * H};
+    jobs.job[jobs.n++] = {W(c, pf + "mlp.Wi.weight"), (const float *)W(c, pf + "mlp_norm.weight"), fold_cs_wi(c, l),
+                          2 * I};
   }
+  const int rc = flush();
+  if (rc) return rc;
   c->fold_gen = c->wgen;
   return DN_OK;
 }
 
-// The folded LayerNorm's statistics buffers for T tokens (none when this
-// context never folds).
+// The folded LayerNorm's row means for T tokens.
 int ensure_fold_buffers(dn_ctx *c, size_t T) {
-  if (!fold_geometry(c) || !c->ln_fold) return DN_OK;
-  HIPCHK(c, "hipMalloc", ensure(c->fold_part, sizeof(float) * 2 * (c->cfg.hidden / kLnPartCols) * T));
   HIPCHK(c, "hipMalloc", ensure(c->fold_mean, sizeof(float) * 2 * T));
   return DN_OK;
 }
@@ -325,7 +333,6 @@ int ctx_workspace(dn_ctx *c, int nseq, const int32_t *seq_len, int R, Workspace 
   if (fold_eligible(c, (int)T)) {
     const int rc = ensure_fold_buffers(c, T);
     if (rc) return rc;
-    o.lpart = (float *)c->fold_part.p;
     o.lmean1 = (float *)c->fold_mean.p;
     o.lmean2 = (float *)c->fold_mean.p + T;
   }
@@ -397,9 +404,11 @@ struct Pass {
   // a large batch); every other forward, training included, uses ATTN_QUERIES
   // items for all layers.
   bool wide_global = false;
-  // The folded LayerNorm (the workspace has its buffers and the pass more
-  // than 1024 tokens).
+  // The folded LayerNorm (the workspace has its buffers), and its statistics'
+  // columns per part: by the whole batch's tokens, also for the parts of a
+  // split forward.
   bool fold = false;
+  int ln_cols = kLnPartWide;
   Workspace w;
   const int32_t *ids, *pos, *opt;
   hipStream_t s;
@@ -479,10 +488,14 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
   const std::string pf = layer_prefix(l);
   const bool sliding = g.sliding[l] != 0;
   const bool split = w.part && !S && !g.generic && h1 == in && out == in;
-  const bool fold = p.fold && w.lpart && !S && !split && !g.generic && h1 == in && out == in;
+  const bool fold = p.fold && w.lmean1 && !S && !split && !g.generic && h1 == in && out == in;
   fold_in = fold_in && fold && l > 0;
   fold_out = fold_out && fold && l + 1 < g.layers;
-  const int lparts = H / kLnPartCols;
+  // The statistics' parts live in buffers that are free from the GEMM that
+  // writes them to the one that reads them: mlp_norm's (Wo to Wi) in qkv,
+  // attn_norm's (MlpWo to the next layer's QKV) in ctx.
+  const int lparts = kLnHidden / p.ln_cols;
+  float *const mlp_part = (float *)w.qkv, *const attn_part = (float *)w.ctx;
   if (l > 0) {
     x1 = S ? S->n1.p : w.xn;
     if (fold_in) {
@@ -508,7 +521,7 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
   q.n_store = 3 * H;
   LnFold qf{};
   if (fold_in) {
-    qf.lpart = w.lpart;
+    qf.lpart = attn_part;
     qf.lparts = lparts;
     qf.mprev = w.lmean2;  // what the previous MlpWo subtracted: its layer's mlp_norm means
     qf.mean_out = w.lmean1;
@@ -580,7 +593,7 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
     LnFold of{};
     of.fx = x2;
     of.lw = (const float *)W(c, pf + "mlp_norm.weight");
-    of.lpart = w.lpart;
+    of.lpart = mlp_part;
     of.lparts = lparts;
     of.mprev = mlp_mprev;
     PROBED(ev, DN_PROBE_WO, "gemm(Wo)", layer_gemm(g, EPI_F32_LN, o, s, &of));
@@ -610,7 +623,7 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
     wi.ldc = I;
     LnFold wf{};
     if (fold) {
-      wf.lpart = w.lpart;
+      wf.lpart = mlp_part;
       wf.lparts = lparts;
       wf.mprev = mlp_mprev;
       wf.mean_out = w.lmean2;
@@ -640,7 +653,7 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
   if (fold_out) {
     mf.fx = w.xn;
     mf.lw = (const float *)W(c, layer_prefix(l + 1) + "attn_norm.weight");
-    mf.lpart = w.lpart;
+    mf.lpart = attn_part;
     mf.lparts = lparts;
     mf.mprev = w.lmean2;
   }
@@ -1011,11 +1024,11 @@ int forward_split(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_
     w.act = (char *)c->act.p + es * t0 * I;
     w.kinfo = (int *)c->kinfo.p + t0;
     if (fold) {
-      w.lpart = (float *)c->fold_part.p + t0 * 2 * (H / kLnPartCols);
       w.lmean1 = (float *)c->fold_mean.p + t0;
       w.lmean2 = (float *)c->fold_mean.p + T + t0;
     }
     ps[k].fold = fold;
+    ps[k].ln_cols = T_total <= kLnNarrowTokens ? kLnPartNarrow : kLnPartWide;
     ps[k].ids = d_ids + t0;
     ps[k].pos = d_pos + t0;
     ps[k].opt = d_opt ? d_opt + t0 : nullptr;
@@ -1125,7 +1138,8 @@ int forward_core(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_i
   ps.pos = d_pos;
   ps.opt = d_opt;
   ps.s = c->stream;
-  ps.fold = !train && w.lpart && fold_eligible(c, T);
+  ps.fold = !train && w.lmean1 && fold_eligible(c, T);
+  ps.ln_cols = T <= kLnNarrowTokens ? kLnPartNarrow : kLnPartWide;
   if (ps.fold) {
     rc = ensure_fold_cs(c, ps.s);
     if (rc) return rc;
@@ -1417,7 +1431,7 @@ void dn_close(dn_ctx *c) {
                     &c->rope,     &c->kinfo, &c->io,
                     &c->logits,   &c->err_flag, &c->gA,    &c->gB,          &c->gC,       &c->d_seq_off, &c->head_s1, &c->head_d,
                     &c->d_seq_len, &c->d_chunk_off, &c->d_chunk_desc, &c->d_work, &c->d_chunks,
-                    &c->d_codes,   &c->d_first, &c->calib, &c->smallpart, &c->fold_cs, &c->fold_part,
+                    &c->d_codes,   &c->d_first, &c->calib, &c->smallpart, &c->fold_cs,
                     &c->fold_mean};
   for (DevBuf *b : bufs) release(*b);
   if (c->pin) (void)hipHostFree(c->pin);

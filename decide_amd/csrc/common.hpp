@@ -118,6 +118,18 @@ __device__ __forceinline__ uint32_t pack16<f16>(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// A lane exchange within a row of 16 lanes as a DPP move (no LDS round trip).
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp_u32(unsigned x) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const unsigned long long u = __double_as_longlong(v);
+  const unsigned lo = dpp_u32<CTRL>((unsigned)u), hi = dpp_u32<CTRL>((unsigned)(u >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // GELU, exact erf form: 0.5*x*(1 + erf(x/sqrt2)) (internal/nn/ops.go:140-142).
 // The fp32 validation build evaluates erf in double as the reference does.
 template <class T>
@@ -234,8 +246,6 @@ struct GemmArgs {
   int M, N, K, lda, ldb, ldc;
   int n_store;    // columns actually stored (fp32 epilogue)
   int accumulate; // fp32 epilogue: C += result
-  int ngroups;    // N-tile groups per XCD sweep (set by launch_gemm)
-  int order;      // workgroup -> tile order (0: XCD-aware groups)
   size_t c_split; // split-K: elements between the partial outputs of blockIdx.y (0: one split)
   const float *res; // EPI_F32 with accumulate: C = res + result (res has C's layout); null: C += result
   void *C2;         // EPI_GEGLU_KEEP: the GeGLU output (ldc2), C receives the plain product
@@ -250,8 +260,8 @@ struct GemmArgs {
 // larger kernel arguments cost every launch ~0.6 us, which the small-batch
 // forwards' ~160 launches feel). The residual GEMM (EPI_F32_LN) also writes
 // fx = (x - mprev[row]) * lw[col] in the operand type, of the new residual x (row stride
-// ldc) and, per row and 192-column N-tile, the tile's (mean, M2) of x to
-// lpart (lparts float pairs per row). The GEMM that takes fx as A (EPI_STORE_LN,
+// ldc) and, per row and part of 768 / lparts columns, the part's (mean, M2) of
+// x to lpart (lparts float pairs per row). The GEMM that takes fx as A (EPI_STORE_LN,
 // EPI_GEGLU_LN) merges them into the row's mean and rstd = 1/sqrt(M2/K +
 // eps) and computes rstd * (A.B^T - (mean - mprev[row]) * lcs[col]) with
 // lcs[n] = sum_k lw[k] B[n][k], i.e. LayerNorm(x).B^T with the LayerNorm
@@ -272,12 +282,14 @@ struct LnFold {
 // output (M x N), and C (M x 2N, operand type, the interleaved Wi layout)
 // receives the gradients of its value and gate inputs, read from gin.
 enum { EPI_F32 = 0, EPI_STORE = 1, EPI_GEGLU = 2, EPI_GEGLU_KEEP = 3, EPI_GEGLU_BWD = 4 };
-// The folded-LayerNorm forms (LnFold; bf16 or fp16, M > 1024): the
+// The folded-LayerNorm forms (LnFold; bf16 or fp16, M > 128): the
 // residual GEMM that produces the LayerNorm's input, and the store / GeGLU
 // GEMMs that consume its output.
 enum { EPI_F32_LN = 5, EPI_STORE_LN = 6, EPI_GEGLU_LN = 7 };
-// Columns per LayerNorm statistics part written by EPI_F32_LN.
-constexpr int kLnPartCols = 192;
+// The folded LayerNorm's row width, and the columns per statistics part
+// written by EPI_F32_LN (LnFold::lparts tells which): narrow for forwards of
+// up to kLnNarrowTokens tokens.
+constexpr int kLnHidden = 768, kLnPartNarrow = 64, kLnPartWide = 192, kLnNarrowTokens = 5376;
 // Whether the folded LayerNorm runs for a 16-bit model of this geometry at M
 // rows (the configurations launch_gemm tiles for EPI_*_LN).
 bool gemm_ln_fold_ok(int precision, int M, int hidden, int inter);
@@ -404,10 +416,20 @@ hipError_t launch_prologue(int precision, const int *pos, const int *opt, const 
                            int *kinfo, ChunkInfo *chunks, const int *ids, int Tn, const float *tok, int vocab,
                            const float *w, float eps, int H, float *h, void *xn, int *err, hipStream_t s,
                            float *mean = nullptr, float *rstd = nullptr);
-// Column sums of a LayerNorm-weighted bf16 or fp16 projection for the folded
-// LayerNorm: cs[n] = sum_k lw[k] * B[n][k] (fp64 sums), B N x K.
-hipError_t launch_fold_colsum(int precision, const void *B, int N, int K, const float *lw, float *cs,
-                              hipStream_t s);
+// Column sums of LayerNorm-weighted bf16 or fp16 projections for the folded
+// LayerNorm: cs[n] = sum_k lw[k] * B[n][k] (fp64 sums), B N x K; n jobs in one
+// launch.
+constexpr int kFoldJobs = 48;
+struct FoldJobs {
+  struct {
+    const void *B;
+    const float *lw;
+    float *cs;
+    int N;
+  } job[kFoldJobs];
+  int n, K;
+};
+hipError_t launch_fold_colsum(int precision, const FoldJobs &j, hipStream_t s);
 // LayerNorm launchers; mean / rstd (optional, [rows]) receive the row statistics.
 hipError_t launch_ln(int precision, const float *x, int rows, int H, const float *w, float eps, void *y, hipStream_t s,
                      float *mean = nullptr, float *rstd = nullptr);

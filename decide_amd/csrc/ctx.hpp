@@ -105,10 +105,8 @@ struct Workspace {
   // [kSmallSplitParts x T x H] split-K partial products of the residual
   // GEMMs for batches of at most kSmallSplitMaxTokens tokens; null otherwise.
   float *part = nullptr;
-  // Folded LayerNorm (bf16 / fp16, more than 1024 tokens): per row the residual
-  // GEMM's (mean, M2) pairs over each 192 columns ([T x H/192]), and the
-  // row means of a layer's attn_norm and mlp_norm ([T] each); null: no fold.
-  float *lpart = nullptr;
+  // Folded LayerNorm (bf16 / fp16, more than 128 tokens): the row means of a
+  // layer's attn_norm and mlp_norm ([T] each); null: no fold.
   float *lmean1 = nullptr, *lmean2 = nullptr;
   int *seq_off = nullptr, *seq_len = nullptr, *chunk_off = nullptr, *first = nullptr;
   int4 *chunk_desc = nullptr, *work = nullptr;
@@ -175,7 +173,7 @@ struct dn_ctx {
   // weighted QKV and Wi weights per layer ([L x (3H + 2I)] floats, allocated
   // by dn_set_config), rebuilt when the weights' generation (bumped by every
   // upload and optimizer step) has moved; the forwards' statistics buffers.
-  DevBuf fold_cs, fold_part, fold_mean;
+  DevBuf fold_cs, fold_mean;
   uint64_t wgen = 1, fold_gen = 0;
   bool ln_fold = true;
   // Forwards of large batches run in two parts of whole sequences, one per
@@ -211,6 +209,9 @@ struct dn_ctx {
 
 namespace dnh {
 
+// dn_set_ln_fold applies to forwards of more tokens than this; smaller ones
+// (above the small-M kernels' 128) always fold.
+constexpr int kFoldSwitchTokens = 1024;
 constexpr int kPositions = 65536;  // RoPE table rows: positions are validated / flagged to this range
 
 int fail(dn_ctx *c, int code, const std::string &msg);

@@ -22,9 +22,9 @@
 //     (row >> 1) & 7, so the 16 rows read by a quarter-wave fall in distinct
 //     banks (the swizzle is applied on the global side of the DMA).
 //   * Workgroup -> tile order is XCD-aware: consecutive workgroup ids go
-//     round-robin over the 8 XCDs; each XCD owns a contiguous range of M
-//     panels and sweeps the N tiles in groups small enough that the group's
-//     slice of B stays in that XCD's 4 MB L2 while its A panels stream.
+//     round-robin over the 8 XCDs; each XCD owns a contiguous range of the
+//     tiles in row order, so an A panel is read into one XCD's L2 (two at a
+//     range's ends) and B (at most 3.5 MB here) stays in it.
 //   * The epilogue stages the finished tile through LDS so global stores are
 //     full 16-byte-per-lane rows.
 #include <type_traits>
@@ -85,24 +85,19 @@ __device__ __forceinline__ void lds_read8x16(const char *const (&p)[8], uint4 (&
   o[6] = __builtin_bit_cast(uint4, v6), o[7] = __builtin_bit_cast(uint4, v7);
 }
 
+// Workgroup -> tile: XCD x (workgroup ids congruent to x mod 8) takes the x-th
+// of eight contiguous ranges of the row-ordered tiles, for any tile count.
+// Row order over all workgroups, which ragged row counts took before, spread
+// each A panel over every XCD (3,840 x 768 x 2304, 128 x 128 tiles: 25.9 ->
+// 23.4 us; 3,840 x 2304 x 768: 25.7 -> 24.3 us).
 template <int BM, int BN>
 struct TileOrder {
   int m0, n0;
-  __device__ __forceinline__ TileOrder(int bid, int tiles_m, int tiles_n, int ngroups, int order) {
-    int tm, tn;
-    const int nt = tiles_m * tiles_n;
-    if (order != 1 && tiles_m % 8 == 0 && tiles_n % ngroups == 0 && nt == (int)gridDim.x) {
-      const int xcd = order == 2 ? bid / (nt / 8) : bid % 8, j = order == 2 ? bid % (nt / 8) : bid / 8;
-      const int pm = tiles_m / 8, gn = tiles_n / ngroups;
-      const int grp = j / (pm * gn), rem = j % (pm * gn);
-      tm = xcd * pm + rem / gn;
-      tn = grp * gn + rem % gn;
-    } else {
-      tm = bid / tiles_n;
-      tn = bid % tiles_n;
-    }
-    m0 = tm * BM;
-    n0 = tn * BN;
+  __device__ __forceinline__ TileOrder(int bid, int tiles_n) {
+    const int nt = (int)gridDim.x, q = nt >> 3, r = nt & 7, xcd = bid & 7;
+    const int t = xcd * q + min(xcd, r) + (bid >> 3);
+    m0 = (t / tiles_n) * BM;
+    n0 = (t % tiles_n) * BN;
   }
 };
 
@@ -153,31 +148,28 @@ __device__ __forceinline__ void store_staged(const T *st, T *C, int ldc, int m0,
 // two-pass statistics, and returns (rstd, mean - mprev) with mean and rstd
 // rounded to float as that kernel rounds them; write_mean also stores the
 // row's mean.
-constexpr int kLnMaxParts = 8;  // launch_gemm checks lparts <= 8
-__device__ __forceinline__ void ln_fold_load(const GemmArgs &g, const LnFold &lf, int row, float2 (&v)[kLnMaxParts],
-                                             float &mp) {
-  const int rr = min(row, g.M - 1), np = lf.lparts;
-  const float2 *pp = (const float2 *)lf.lpart + (size_t)rr * np;
+// NP parts of PC columns (launch_gemm checks lparts == NP, NP PC == K).
+template <int NP>
+__device__ __forceinline__ void ln_fold_load(const GemmArgs &g, const LnFold &lf, int row, float2 (&v)[NP], float &mp) {
+  const int rr = min(row, g.M - 1);
+  const float2 *pp = (const float2 *)lf.lpart + (size_t)rr * NP;
 #pragma unroll
-  for (int t = 0; t < kLnMaxParts; t++)
-    if (t < np) v[t] = pp[t];
+  for (int t = 0; t < NP; t++) v[t] = pp[t];
   mp = lf.mprev ? lf.mprev[rr] : 0.0f;
 }
-__device__ __forceinline__ float2 ln_fold_merge(const GemmArgs &g, const LnFold &lf, int row,
-                                                const float2 (&v)[kLnMaxParts], float mp, bool write_mean) {
-  const int np = lf.lparts;
+template <int NP, int PC>
+__device__ __forceinline__ float2 ln_fold_merge(const GemmArgs &g, const LnFold &lf, int row, const float2 (&v)[NP],
+                                                float mp, bool write_mean) {
   double sum = 0;
 #pragma unroll
-  for (int t = 0; t < kLnMaxParts; t++)
-    if (t < np) sum += (double)v[t].x;
-  const double mu = sum / np;
+  for (int t = 0; t < NP; t++) sum += (double)v[t].x;
+  const double mu = sum / NP;
   double m2 = 0;
 #pragma unroll
-  for (int t = 0; t < kLnMaxParts; t++)
-    if (t < np) {
-      const double d = (double)v[t].x - mu;
-      m2 += (double)v[t].y + (double)kLnPartCols * d * d;
-    }
+  for (int t = 0; t < NP; t++) {
+    const double d = (double)v[t].x - mu;
+    m2 += (double)v[t].y + (double)PC * d * d;
+  }
   const float mean = (float)mu;
   if (write_mean && row < g.M) lf.mean_out[row] = mean;
   return make_float2((float)(1.0 / sqrt(m2 / (double)g.K + (double)lf.eps)), mean - mp);
@@ -185,8 +177,9 @@ __device__ __forceinline__ float2 ln_fold_merge(const GemmArgs &g, const LnFold 
 
 // WGM x WGN waves tile the BM x BN block; each wave owns a WM x WN sub-tile.
 // The body of gemm_nt_kernel and gemm_nt_ln_kernel (lf: the folded
-// LayerNorm's arguments, used by the EPI_*_LN forms only).
-template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM, int WGN>
+// LayerNorm's arguments, used by the EPI_*_LN forms only; PC: its statistics'
+// columns per part). PF: the main loop for small wave tiles (below).
+template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM, int WGN, bool PF, int PC>
 __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf) {
   using MF = Mfma<T>;
   typedef typename MF::frag frag;
@@ -198,12 +191,13 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
   constexpr int TM = WM / 32, TN = WN / 32;
   constexpr int STAGE = (BM + BN) * RB;
   constexpr int LOADS = (BM + BN) * CPR / NT;  // 16-byte DMA loads per thread per stage
+  constexpr bool LNC = EPI == EPI_STORE_LN || EPI == EPI_GEGLU_LN;  // folded LayerNorm consumer
   static_assert(LOADS * NT == (BM + BN) * CPR, "tile rows must fill whole DMA instructions");
+  static_assert(!LNC || (BM <= NT && BN <= NT), "one thread per row and column of the folded LayerNorm's terms");
   static_assert(EPI == EPI_F32 || EPI == EPI_F32_LN || EPI == EPI_GEGLU_BWD || TN % 2 == 0,
                 "paired epilogues need 64-column wave tiles");
   constexpr bool F32OUT = EPI == EPI_F32 || EPI == EPI_F32_LN;
   constexpr bool GATED = EPI == EPI_GEGLU || EPI == EPI_GEGLU_LN;
-  constexpr bool LNC = EPI == EPI_STORE_LN || EPI == EPI_GEGLU_LN;  // folded LayerNorm consumer
   static_assert(NSTAGE >= 2 && LOADS * (NSTAGE - 2) < 64, "pipeline depth");
   // fp32 epilogue staged in WGM passes of WM rows; the others in one pass.
   constexpr int EPI_BYTES = (F32OUT || EPI == EPI_GEGLU_BWD) ? WM * (BN + 4) * 4
@@ -221,7 +215,7 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
   const int wm = wave / WGN, wn = wave % WGN;
   const int lr = lane & 31, lh = lane >> 5;
 
-  const TileOrder<BM, BN> to(blockIdx.x, (g.M + BM - 1) / BM, g.N / BN, g.ngroups, g.order);
+  const TileOrder<BM, BN> to(blockIdx.x, g.N / BN);
   const int m0 = to.m0, n0 = to.n0;
   // Folded LayerNorm consumer: thread t < BM takes block row t's statistics
   // and thread t < BN column n0 + t's lcs (loaded here; merged after the
@@ -230,10 +224,11 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
   // mprev) of its rows from ln_st and its columns' lcs from ln_cs.
   float2 *const ln_st = (float2 *)(smem + SMEM_RING);
   float *const ln_cs = (float *)(smem + SMEM_RING + BM * 8);
-  float2 ln_v[LNC ? kLnMaxParts : 1];
+  constexpr int NP = LNC ? kLnHidden / PC : 1;
+  float2 ln_v[NP];
   float ln_mp = 0.0f, ln_c = 0.0f;
   if constexpr (LNC) {
-    if (threadIdx.x < BM) ln_fold_load(g, lf, m0 + (int)threadIdx.x, ln_v, ln_mp);
+    if (threadIdx.x < BM) ln_fold_load<NP>(g, lf, m0 + (int)threadIdx.x, ln_v, ln_mp);
     if (threadIdx.x < BN) ln_c = lf.lcs[n0 + threadIdx.x];
   }
   // Split-K: blockIdx.y takes K elements [y*K, (y+1)*K) of A and B and writes
@@ -285,69 +280,152 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
   constexpr int PER_KS = (LOADS + NKS - 1) / NKS;      // next-stage loads issued per k step
   static_assert(NKS % 2 == 0, "operand double buffering alternates per k step");
 
-  // MFMA operands are double buffered across k steps: the fragments of step
-  // ks+1 (or of the next stage's step 0) are read from LDS while the MFMAs of
-  // step ks run. The next stage's readiness (vmcnt + barrier) is established
-  // at the end of each stage, after the last MFMAs of the stage are issued.
-  frag fa[2][TM], fb[2][TN];
-  auto load_frags = [&](int buf, int stage, int ks) {
-    const char *sa = smem + stage * STAGE;
-    const char *sb = sa + BM * RB;
-    const int ke = ks * MF::KSTEP + lh * MF::SLOTS;  // first k element of this lane's operand
-    const int chunk = ke * (int)sizeof(T) / 16, within = ke * (int)sizeof(T) % 16;
+  if constexpr (PF) {
+    // Small wave tiles (one or two MFMAs a k step, fewer cycles than an LDS
+    // read takes): a stage's operands are all in registers before its first
+    // MFMA, and each k step's fragments are replaced by the next stage's right
+    // after the MFMAs that used them. The loop below with its one k step of
+    // lookahead spends ~550 cycles a stage on LDS latency there, this one about
+    // half (512 x 768 x 768 on 64 x 64 tiles 6.9 -> 5.9 us, K = 2304 13.2 ->
+    // 10.2 us; the same MFMAs in the same order). A stage is read into
+    // registers one stage ahead, so one DMA stage fewer is in flight; past the
+    // last one nothing is issued, and the last NSTAGE - 1 stages run unrolled
+    // with their own waits.
+    frag fa[NKS][TM], fb[NKS][TN];
+    auto load_step = [&](int slot, int ks) {
+      const char *sa = smem + slot * STAGE;
+      const char *sb = sa + BM * RB;
+      const int ke = ks * MF::KSTEP + lh * MF::SLOTS;
+      const int chunk = ke * (int)sizeof(T) / 16, within = ke * (int)sizeof(T) % 16;
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-      const int r = wm * WM + i * 32 + lr;
-      fa[buf][i] = *(const frag *)(sa + r * RB + ((chunk ^ swz<RB>(r)) << 4) + within);
-    }
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-      const int r = wn * WN + j * 32 + lr;
-      fb[buf][j] = *(const frag *)(sb + r * RB + ((chunk ^ swz<RB>(r)) << 4) + within);
-    }
-  };
-  // Waits until stage kt has landed for every wave: NSTAGE-2 later stages'
-  // loads may still be in flight.
-  auto stage_ready = [&]() {
-    wait_vmcnt<LOADS * (NSTAGE - 2)>();
-    __builtin_amdgcn_s_barrier();
-  };
-
-  stage_ready();
-  load_frags(0, 0, 0);
-  for (int kt = 0; kt < nk; kt++) {
-    // Refill the buffer of stage kt-1 (every wave finished reading it before
-    // the barrier that made stage kt visible) with stage kt + NSTAGE - 1.
-    const int rstage = (kt + NSTAGE - 1) % NSTAGE, rk = min(kt + NSTAGE - 1, nk - 1) * KT;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ks++) {
-      const int cur = ks & 1;
-      // Program order: next step's operand reads, this step's share of the
-      // DMA refill (the DMA writes LDS, so reads placed after it could not be
-      // hoisted above it), then this step's MFMAs.
-      if (ks + 1 < NKS) load_frags(cur ^ 1, kt % NSTAGE, ks + 1);
-      {
-        const int i0 = ks * PER_KS < LOADS ? ks * PER_KS : LOADS;
-        const int i1 = (ks + 1) * PER_KS < LOADS ? (ks + 1) * PER_KS : LOADS;
-        issue_part(rstage, rk, i0, i1);
+      for (int i = 0; i < TM; i++) {
+        const int r = wm * WM + i * 32 + lr;
+        fa[ks][i] = *(const frag *)(sa + r * RB + ((chunk ^ swz<RB>(r)) << 4) + within);
       }
-      // B is the MFMA's first operand: acc[i][j] holds the transposed
-      // 32x32 block, so lane l owns token row l%32 and four runs of four
-      // consecutive output columns (vector stores in the epilogue).
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const int r = wn * WN + j * 32 + lr;
+        fb[ks][j] = *(const frag *)(sb + r * RB + ((chunk ^ swz<RB>(r)) << 4) + within);
+      }
+    };
+    auto mfmas = [&](int ks) {
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = MF::mma(fb[cur][j], fa[cur][i], acc[i][j]);
-      // One MFMA, then all of the next step's operand reads (they get the
-      // rest of the step to land), then the DMA issues, then the MFMAs.
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (ks + 1 < NKS) __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x020, PER_KS, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, TM * TN - 2, 0);
-      if (ks + 1 == NKS && kt + 1 < nk) {
-        stage_ready();
-        load_frags(cur ^ 1, (kt + 1) % NSTAGE, 0);
+        for (int j = 0; j < TN; j++) acc[i][j] = MF::mma(fb[ks][j], fa[ks][i], acc[i][j]);
+    };
+    wait_vmcnt<LOADS * (NSTAGE - 2)>();
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int ks = 0; ks < NKS; ks++) load_step(0, ks);
+    // No scalar load in flight past here, so the compiler's waits in the loop
+    // count LDS reads exactly.
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    int kt = 0, slot = 0;
+    for (; kt + NSTAGE - 1 < nk; kt++) {
+      const int nslot = slot + 1 == NSTAGE ? 0 : slot + 1, pslot = slot == 0 ? NSTAGE - 1 : slot - 1;
+      wait_vmcnt<LOADS * (NSTAGE - 3)>();
+      __builtin_amdgcn_s_barrier();
+#pragma unroll
+      for (int ks = 0; ks < NKS; ks++) {
+        mfmas(ks);
+        load_step(nslot, ks);
+        const int i0 = ks * PER_KS < LOADS ? ks * PER_KS : LOADS;
+        const int i1 = (ks + 1) * PER_KS < LOADS ? (ks + 1) * PER_KS : LOADS;
+        issue_part(pslot, (kt + NSTAGE - 1) * KT, i0, i1);
+        __builtin_amdgcn_sched_group_barrier(0x008, TM * TN, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, PER_KS, 0);
+      }
+      slot = nslot;
+    }
+    auto tail = [&](auto tc) {
+      constexpr int TT = decltype(tc)::value;  // 0 .. NSTAGE - 2
+      if (kt + NSTAGE - 1 - TT == nk) {
+        const int nslot = slot + 1 == NSTAGE ? 0 : slot + 1;
+        if constexpr (TT < NSTAGE - 2) {
+          wait_vmcnt<LOADS * (NSTAGE - 3 - TT > 0 ? NSTAGE - 3 - TT : 0)>();
+          __builtin_amdgcn_s_barrier();
+        }
+#pragma unroll
+        for (int ks = 0; ks < NKS; ks++) {
+          mfmas(ks);
+          if constexpr (TT < NSTAGE - 2) load_step(nslot, ks);
+        }
+        slot = nslot;
+        kt++;
+      }
+    };
+    static_assert(NSTAGE >= 3 && NSTAGE <= 5, "unrolled tail");
+    tail(std::integral_constant<int, 0>{});
+    tail(std::integral_constant<int, 1>{});
+    if constexpr (NSTAGE > 3) tail(std::integral_constant<int, 2>{});
+    if constexpr (NSTAGE > 4) tail(std::integral_constant<int, 3>{});
+  } else {
+    // MFMA operands are double buffered across k steps: the fragments of step
+    // ks+1 (or of the next stage's step 0) are read from LDS while the MFMAs of
+    // step ks run. The next stage's readiness (vmcnt + barrier) is established
+    // at the end of each stage, after the last MFMAs of the stage are issued.
+    frag fa[2][TM], fb[2][TN];
+    auto load_frags = [&](int buf, int stage, int ks) {
+      const char *sa = smem + stage * STAGE;
+      const char *sb = sa + BM * RB;
+      const int ke = ks * MF::KSTEP + lh * MF::SLOTS;  // first k element of this lane's operand
+      const int chunk = ke * (int)sizeof(T) / 16, within = ke * (int)sizeof(T) % 16;
+#pragma unroll
+      for (int i = 0; i < TM; i++) {
+        const int r = wm * WM + i * 32 + lr;
+        fa[buf][i] = *(const frag *)(sa + r * RB + ((chunk ^ swz<RB>(r)) << 4) + within);
+      }
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const int r = wn * WN + j * 32 + lr;
+        fb[buf][j] = *(const frag *)(sb + r * RB + ((chunk ^ swz<RB>(r)) << 4) + within);
+      }
+    };
+    // Waits until stage kt has landed for every wave: NSTAGE-2 later stages'
+    // loads may still be in flight.
+    auto stage_ready = [&]() {
+      wait_vmcnt<LOADS * (NSTAGE - 2)>();
+      __builtin_amdgcn_s_barrier();
+    };
+
+    stage_ready();
+    load_frags(0, 0, 0);
+    for (int kt = 0; kt < nk; kt++) {
+      // Refill the buffer of stage kt-1 (every wave finished reading it before
+      // the barrier that made stage kt visible) with stage kt + NSTAGE - 1.
+      const int rstage = (kt + NSTAGE - 1) % NSTAGE, rk = min(kt + NSTAGE - 1, nk - 1) * KT;
+#pragma unroll
+      for (int ks = 0; ks < NKS; ks++) {
+        const int cur = ks & 1;
+        // Program order: next step's operand reads, this step's share of the
+        // DMA refill (the DMA writes LDS, so reads placed after it could not be
+        // hoisted above it), then this step's MFMAs.
+        if (ks + 1 < NKS) load_frags(cur ^ 1, kt % NSTAGE, ks + 1);
+        {
+          const int i0 = ks * PER_KS < LOADS ? ks * PER_KS : LOADS;
+          const int i1 = (ks + 1) * PER_KS < LOADS ? (ks + 1) * PER_KS : LOADS;
+          issue_part(rstage, rk, i0, i1);
+        }
+        // B is the MFMA's first operand: acc[i][j] holds the transposed
+        // 32x32 block, so lane l owns token row l%32 and four runs of four
+        // consecutive output columns (vector stores in the epilogue).
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int j = 0; j < TN; j++) acc[i][j] = MF::mma(fb[cur][j], fa[cur][i], acc[i][j]);
+        // One MFMA, then all of the next step's operand reads (they get the
+        // rest of the step to land), then the DMA issues, then the MFMAs.
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (ks + 1 < NKS) __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, PER_KS, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, TM * TN - 2, 0);
+        if (ks + 1 == NKS && kt + 1 < nk) {
+          stage_ready();
+          load_frags(cur ^ 1, (kt + 1) % NSTAGE, 0);
+        }
       }
     }
   }
@@ -357,7 +435,7 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
     // The folded LayerNorm's row statistics (loaded at the start, landed
     // with the last stage) and column sums, for every wave's epilogue: the
     // barrier must also wait for these LDS writes.
-    if (threadIdx.x < BM) ln_st[threadIdx.x] = ln_fold_merge(g, lf, m0 + (int)threadIdx.x, ln_v, ln_mp, n0 == 0);
+    if (threadIdx.x < BM) ln_st[threadIdx.x] = ln_fold_merge<NP, PC>(g, lf, m0 + (int)threadIdx.x, ln_v, ln_mp, n0 == 0);
     if (threadIdx.x < BN) ln_cs[threadIdx.x] = ln_c;
     __syncthreads();
   } else {
@@ -434,10 +512,14 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
     constexpr int V = BN / 4;  // float4 per row
     constexpr int ITER = HM * V / NT;
     static_assert(ITER * NT == HM * V, "epilogue shape");
-    // Folded LayerNorm: TPR threads per row of a pass (8 on 256-row tiles).
-    constexpr int TPR = NT / HM, CW = 4 * TPR;
-    static_assert(!LN || (BN == kLnPartCols && TPR * HM == NT && (TPR == 4 || TPR == 8) && BN % CW == 0),
-                  "LayerNorm statistics: 4 or 8 threads per 192-column row");
+    // Folded LayerNorm: TPR threads per row of a pass, TPP per row and part
+    // of PC columns. The sums of a part are associated as eight lanes' sums
+    // whatever TPP is (16: a lane's chunks are split over two threads), so
+    // the statistics do not depend on the tile.
+    constexpr int TPR = NT / HM, PCC = LN ? PC : BN, TPP = TPR / (BN / PCC), CW = 4 * TPP;
+    static_assert(!LN || (BN % PCC == 0 && TPR * HM == NT && TPP * (BN / PCC) == TPR && (TPP == 8 || TPP == 16) &&
+                          PCC % CW == 0),
+                  "LayerNorm statistics: 8 or 16 threads per row and part");
     const bool vec = (g.ldc & 3) == 0;
     // The residual loads of a pass are issued together (one HBM round trip
     // per pass): pass 0's before its staging, so that their latency overlaps
@@ -456,15 +538,17 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
       }
     };
     load_old(0);
-    // Folded LayerNorm: thread (row tid / TPR of the pass, part tid % TPR)
-    // takes the 4-column chunks 4 part + CW q (q < NQ) of the row, so that
-    // the TPR threads of a row store 8 TPR contiguous bytes of the bf16
-    // operand per instruction; the LayerNorm weight at them.
-    constexpr int NQ = BN / CW;
+    // Folded LayerNorm: thread (row tid / TPR of the pass, thread tid % TPP of
+    // part tid % TPR / TPP) takes the 4-column chunks CW q (q < NQ) after
+    // column lnc, so that the TPP threads of a row and part store 8 TPP
+    // contiguous bytes of the 16-bit operand per instruction; the LayerNorm
+    // weight at them.
+    constexpr int NQ = PCC / CW;
+    const int lnc = tid % TPR / TPP * PCC + 4 * (tid % TPP);
     float4 lw4[LN ? NQ : 1];
     if constexpr (LN) {
 #pragma unroll
-      for (int q = 0; q < NQ; q++) lw4[q] = *(const float4 *)(lf.lw + n0 + 4 * (tid % TPR) + CW * q);
+      for (int q = 0; q < NQ; q++) lw4[q] = *(const float4 *)(lf.lw + n0 + lnc + CW * q);
     }
 #pragma unroll
     for (int pass = 0; pass < WGM; pass++) {
@@ -492,22 +576,22 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
         }
       }
       if constexpr (LN) {
-        // The pass's rows from the staging area: TPR threads per row, the
-        // chunks above. The next LayerNorm's operand (x - mprev) * w in T,
-        // one 8-byte store per chunk; the statistics over this tile's 192
-        // columns: fp32 partial sums, the TPR reduced in fp64 in a fixed
-        // order, then the squared deviations from the tile mean the same way,
-        // stored as an fp32 pair (their fp32 rounding, ~1e-6 relative, is far
-        // below the bf16 operand's).
+        // The pass's rows from the staging area, the chunks above. The next
+        // LayerNorm's operand (x - mprev) * w in T, one 8-byte store per chunk;
+        // the statistics over each part's PC columns: fp32 sums of eight
+        // lanes (lane v: the 4-column chunks 32 q + 4 v, in order), the eight
+        // reduced in fp64 in a fixed order, then the squared deviations from
+        // the part's mean the same way, stored as an fp32 pair (their fp32
+        // rounding, ~1e-6 relative, is far below the 16-bit operand's).
         __syncthreads();
-        const int r = tid / TPR, part = tid % TPR;
+        const int r = tid / TPR;
         float4 xv[NQ];
 #pragma unroll
-        for (int q = 0; q < NQ; q++) xv[q] = *(const float4 *)(st + r * LD + 4 * part + CW * q);
+        for (int q = 0; q < NQ; q++) xv[q] = *(const float4 *)(st + r * LD + lnc + CW * q);
         {
           const int row = m0 + pass * HM + r;
           if (row < g.M) {
-            T *f = (T *)lf.fx + (size_t)row * g.ldc + n0 + 4 * part;
+            T *f = (T *)lf.fx + (size_t)row * g.ldc + n0 + lnc;
 #pragma unroll
             for (int q = 0; q < NQ; q++) {
               const float4 a = xv[q], wa = lw4[q];
@@ -516,26 +600,46 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
             }
           }
         }
-        float s32 = 0.0f;
+        // A lane's chunk sums, added in column order: with 16 threads the
+        // chunks alternate between threads v (even) and v + 8 (odd).
+        const bool odd = TPP == 16 && (tid & 8);
+        auto lane_sum = [&](const float (&c)[NQ]) {
+          float t = 0.0f;
 #pragma unroll
-        for (int q = 0; q < NQ; q++) s32 += (xv[q].x + xv[q].y) + (xv[q].z + xv[q].w);
-        double sum = s32;
+          for (int q = 0; q < NQ; q++) {
+            if constexpr (TPP == 16) {
+              const float o = __uint_as_float(dpp_u32<0x128>(__float_as_uint(c[q])));  // row_ror:8
+              t += odd ? o : c[q];
+              t += odd ? c[q] : o;
+            } else {
+              t += c[q];
+            }
+          }
+          return t;
+        };
+        float cs[NQ];
 #pragma unroll
-        for (int o = 1; o < TPR; o <<= 1) sum += __shfl_xor(sum, o);
-        const double mu = sum / BN;
+        for (int q = 0; q < NQ; q++) cs[q] = (xv[q].x + xv[q].y) + (xv[q].z + xv[q].w);
+        // Over eight lanes: lane ^ 1, lane ^ 2 and, the quads' lanes now being
+        // equal, the half row mirrored for lane ^ 4.
+        auto sum8 = [](double v) {
+          v += dpp_f64<0xB1>(v);
+          v += dpp_f64<0x4E>(v);
+          v += dpp_f64<0x141>(v);
+          return v;
+        };
+        const double sum = sum8(lane_sum(cs));
+        const double mu = sum / PCC;
         const float muf = (float)mu;
-        float q32 = 0.0f;
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
           const float a = xv[q].x - muf, b = xv[q].y - muf, c = xv[q].z - muf, d = xv[q].w - muf;
-          q32 += (a * a + b * b) + (c * c + d * d);
+          cs[q] = (a * a + b * b) + (c * c + d * d);
         }
-        double m2 = q32;
-#pragma unroll
-        for (int o = 1; o < TPR; o <<= 1) m2 += __shfl_xor(m2, o);
+        const double m2 = sum8(lane_sum(cs));
         const int row = m0 + pass * HM + r;
-        if (part == 0 && row < g.M)
-          ((float2 *)lf.lpart)[(size_t)row * lf.lparts + n0 / BN] = make_float2((float)mu, (float)m2);
+        if (tid % TPP == 0 && row < g.M)
+          ((float2 *)lf.lpart)[(size_t)row * lf.lparts + (n0 + lnc) / PCC] = make_float2((float)mu, (float)m2);
       }
       if (pass + 1 < WGM) {
         load_old(pass + 1);
@@ -630,71 +734,42 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
   }
 }
 
-template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM, int WGN>
+template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM, int WGN, bool PF>
 __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm_nt_kernel(GemmArgs g) {
   static_assert(EPI < EPI_F32_LN, "the folded-LayerNorm forms run as gemm_nt_ln_kernel");
-  gemm_nt_tile<T, BM, BN, RB, NSTAGE, EPI, WPE, WGM, WGN>(g, LnFold{});
+  gemm_nt_tile<T, BM, BN, RB, NSTAGE, EPI, WPE, WGM, WGN, PF, 0>(g, LnFold{});
 }
-template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM, int WGN>
+template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM, int WGN, bool PF, int PC>
 __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm_nt_ln_kernel(GemmArgs g,
                                                                                                             LnFold lf) {
   static_assert(EPI >= EPI_F32_LN, "plain forms run as gemm_nt_kernel");
-  gemm_nt_tile<T, BM, BN, RB, NSTAGE, EPI, WPE, WGM, WGN>(g, lf);
+  gemm_nt_tile<T, BM, BN, RB, NSTAGE, EPI, WPE, WGM, WGN, PF, PC>(g, lf);
 }
 
-template <class T, int BM, int BN, int RB, int NSTAGE, int WPE, int WGM = 2, int WGN = 2>
-hipError_t launch_cfg(int epi, const GemmArgs &a, hipStream_t s, int splits = 1) {
-  const int tiles = ((a.M + BM - 1) / BM) * (a.N / BN);
-  dim3 grid(tiles, splits), block(64 * WGM * WGN);
-  // bf16 256-row tiles serve only the operand-type epilogues (the fp32 ones
-  // take 128 x 192 or 128 x 128 tiles): the fp32 epilogue is not built there.
-  constexpr bool f32_epi = !(sizeof(T) == 2 && BM == 256);
-  // The fp16 mode is inference only: no training epilogues.
-  constexpr bool train_epi = !std::is_same<T, f16>::value;
-  if (!train_epi && (epi == EPI_GEGLU_BWD || epi == EPI_GEGLU_KEEP)) return hipErrorInvalidValue;
-  switch (epi) {
-    case EPI_F32:
-      if constexpr (f32_epi)
-        hipLaunchKernelGGL((gemm_nt_kernel<T, BM, BN, RB, NSTAGE, EPI_F32, WPE, WGM, WGN>), grid, block, 0, s, a);
-      else
-        return hipErrorInvalidValue;
-      break;
-    case EPI_STORE:
-      hipLaunchKernelGGL((gemm_nt_kernel<T, BM, BN, RB, NSTAGE, EPI_STORE, WPE, WGM, WGN>), grid, block, 0, s, a);
-      break;
-    case EPI_GEGLU:
-      hipLaunchKernelGGL((gemm_nt_kernel<T, BM, BN, RB, NSTAGE, EPI_GEGLU, WPE, WGM, WGN>), grid, block, 0, s, a);
-      break;
-    case EPI_GEGLU_BWD:
-      if constexpr (train_epi)
-        hipLaunchKernelGGL((gemm_nt_kernel<T, BM, BN, RB, NSTAGE, EPI_GEGLU_BWD, WPE, WGM, WGN>), grid, block, 0, s, a);
-      break;
-    default:
-      if constexpr (train_epi)
-        hipLaunchKernelGGL((gemm_nt_kernel<T, BM, BN, RB, NSTAGE, EPI_GEGLU_KEEP, WPE, WGM, WGN>), grid, block, 0, s, a);
-      break;
-  }
-  return hipGetLastError();
-}
+// A tile configuration: block tile, K stage bytes, stages, workgroups per CU
+// (waves per SIMD), waves, and the small-wave-tile main loop.
+template <int BM_, int BN_, int RB_, int NSTAGE_, int WPE_, int WGM_, int WGN_, bool PF_ = false>
+struct Tile {
+  static constexpr int BM = BM_, BN = BN_, RB = RB_, NSTAGE = NSTAGE_, WPE = WPE_, WGM = WGM_, WGN = WGN_;
+  static constexpr bool PF = PF_;
+  static int count(const GemmArgs &a) { return (a.M + BM - 1) / BM * (a.N / BN); }
+};
 
-// One epilogue alone (the fp32 one or the GeGLU backward), for tiles whose
-// wave columns (BN / 2 = 96) do not pair up for the operand-type epilogues.
-// WGM rows of waves (64-row wave tiles when BM = 256 and WGM = 4).
-template <class T, int BM, int BN, int RB, int NSTAGE, int WPE, int EPI = EPI_F32, int WGM = 2>
-hipError_t launch_cfg_one(const GemmArgs &a, hipStream_t s, int splits = 1, const LnFold *ln = nullptr) {
-  static_assert(EPI == EPI_F32 || EPI == EPI_F32_LN || EPI == EPI_GEGLU_BWD, "epilogues that take 96-column wave tiles");
-  constexpr int WGN = BN / 96;  // 96-column wave tiles: 2 x 2 waves for 192 columns, 2 x 4 for 384
-  static_assert(WGN * 96 == BN && (WGN == 2 || WGN == 4), "96-column wave tiles");
-  static_assert(WGM * WGN <= 8, "at most 8 waves per workgroup");
-  const int tiles = ((a.M + BM - 1) / BM) * (a.N / BN);
-  if constexpr (EPI == EPI_F32_LN)
-    hipLaunchKernelGGL((gemm_nt_ln_kernel<T, BM, BN, RB, NSTAGE, EPI, WPE, WGM, WGN>), dim3(tiles, splits),
-                       dim3(64 * WGM * WGN), 0, s, a, *ln);
+template <class T, class C, int EPI, int PC = 0>
+hipError_t launch_tile(const GemmArgs &a, hipStream_t s, const LnFold *ln = nullptr, int splits = 1) {
+  if (a.N % C::BN || a.K % (C::RB / (int)sizeof(T))) return hipErrorInvalidValue;
+  const dim3 grid(C::count(a), splits), block(64 * C::WGM * C::WGN);
+  if constexpr (EPI >= EPI_F32_LN)
+    hipLaunchKernelGGL((gemm_nt_ln_kernel<T, C::BM, C::BN, C::RB, C::NSTAGE, EPI, C::WPE, C::WGM, C::WGN, C::PF, PC>),
+                       grid, block, 0, s, a, *ln);
   else
-    hipLaunchKernelGGL((gemm_nt_kernel<T, BM, BN, RB, NSTAGE, EPI, WPE, WGM, WGN>), dim3(tiles, splits),
-                       dim3(64 * WGM * WGN), 0, s, a);
+    hipLaunchKernelGGL((gemm_nt_kernel<T, C::BM, C::BN, C::RB, C::NSTAGE, EPI, C::WPE, C::WGM, C::WGN, C::PF>), grid,
+                       block, 0, s, a);
   return hipGetLastError();
 }
+
+// Workgroups of a launch that runs in one round on 256 CUs.
+constexpr int kCUs = 256;
 
 // Small-M GEMM (M <= 128 in bf16: one request; M <= 1024 in fp32: the
 // scorer's dense layer over every [MASK] row of a batch). Such
@@ -1204,12 +1279,8 @@ hipError_t launch_gemm_splitk(int precision, const GemmArgs &a0, int splits, flo
   a.n_store = a0.N;
   a.accumulate = 0;
   a.c_split = (size_t)a0.M * a0.N;
-  a.ngroups = 1;
-  a.order = 1;  // row-major tile order: the grid is (tiles, splits)
-  // bf16: 64 x 128 tiles with 128-byte K stages (the long-K weight-gradient
-  // shapes run best on them, unsplit or lightly split).
-  hipError_t e = precision == 1 ? launch_cfg<bf16, 64, 128, 128, 4, 1>(EPI_F32, a, s, splits)
-                                : launch_cfg<float, 128, 128, 128, 3, 1>(EPI_F32, a, s, splits);
+  const hipError_t e = precision == PREC_BF16 ? launch_tile<bf16, Tile<64, 128, 128, 5, 1, 2, 4, true>, EPI_F32>(a, s, nullptr, splits)
+                                              : launch_tile<float, Tile<128, 128, 128, 3, 1, 2, 2>, EPI_F32>(a, s, nullptr, splits);
   if (e != hipSuccess) return e;
   const size_t n = (size_t)a0.M * a0.N;
   hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, partial, splits,
@@ -1233,14 +1304,13 @@ bool gemm_shape_ok(int precision, int N, int K) {
 }
 
 bool gemm_epi_ok(int precision, int epi, int M) {
-  if (epi >= EPI_F32_LN) return prec16(precision) && M > 1024;
+  if (epi >= EPI_F32_LN) return prec16(precision) && M > 128;
   if (epi != EPI_GEGLU_BWD) return true;
   return prec16(precision) ? M > 128 : M > 1024;
 }
 
 bool gemm_ln_fold_ok(int precision, int M, int hidden, int inter) {
-  return prec16(precision) && M > 1024 && hidden % kLnPartCols == 0 && hidden / kLnPartCols <= 8 &&
-         3 * hidden > 1024 && (3 * hidden) % 128 == 0 && (2 * inter) % 128 == 0 && inter % 64 == 0;
+  return prec16(precision) && M > 128 && hidden == kLnHidden && inter > 0 && inter % 64 == 0;
 }
 
 // Any-shape GEMM (model geometries the MFMA kernels do not tile): thread n of
@@ -1293,127 +1363,141 @@ hipError_t launch_gemm_generic(int precision, int epi, const GemmArgs &a, hipStr
                                  : launch_gemm_generic_t<float>(epi, a, s);
 }
 
-// The tiled kernel's configuration for 16-bit operands (bf16 or fp16; the
-// same tiles, measured on bf16).
-template <class T>
-hipError_t launch_gemm16(int epi, const GemmArgs &a, hipStream_t s, const LnFold *ln);
+// fp32-output tiles (the residual GEMMs, input and weight gradients): the
+// smallest tile whose grid is one round of the 256 CUs, since a launch takes
+// about as long as one workgroup and that is its K loop's length times its
+// tile. Measured on isolated launches with weights rotated past L2 (us, K =
+// 768 / 1152 / 2304, N = 768), each beside the tile it replaced there:
+//   64 x 64   600 rows   5.8 /  7.1 / 10.2  (64 x 128, four waves:  8.2 /  9.6 / 14.4)
+//   64 x 128  2,046      8.1 /  9.4 / 16.2  (64 x 192:             11.5 / 13.7 / 22.8)
+//   128 x 128 3,840     11.6 / 13.7 / 23.4  (64 x 192:             12.8 / 15.3 / 24.7)
+//   64 x 256  5,400     13.9 / 17.0 / 29.5  (256 x 192:            25.1 / 31.8 / 56.5)
+//   128 x 192 8,192     18.6 / 22.6 / 36.0  (256 x 192:            26.2 / 33.2 / 60.2)
+//   256 x 192 16,000    33.3 / 42.8 / 73.6  (128 x 192, two rounds: 34.3 / 45.7 / 74.8)
+// The first four hold a stage's operands in registers (PF): without it 64 x
+// 64 took 6.9 / 8.7 / 13.2 us at 512 rows. 256 x 192 (eight waves of 64 x 96,
+// one workgroup per CU) stages the fewest operand bytes per output.
+typedef Tile<64, 64, 128, 5, 2, 2, 2, true> F64x64;
+typedef Tile<64, 128, 128, 5, 1, 2, 4, true> F64x128;
+typedef Tile<128, 128, 128, 4, 1, 4, 2, true> F128x128;
+typedef Tile<64, 256, 128, 4, 1, 2, 4, true> F64x256;
+typedef Tile<128, 192, 128, 3, 1, 4, 2> F128x192;
+typedef Tile<256, 192, 128, 2, 2, 4, 2> F256x192;
+typedef Tile<128, 128, 64, 3, 3, 2, 2> F128x128s;  // large outputs of other widths
 
-hipError_t launch_gemm(int precision, int epi, const GemmArgs &a0, hipStream_t s, const LnFold *ln) {
-  if (a0.M <= 0) return hipSuccess;
-  if (!gemm_epi_ok(precision, epi, a0.M) || (epi == EPI_GEGLU_BWD && (!a0.gin || a0.ldc % 8))) return hipErrorInvalidValue;
-  // Small M goes to the whole-K kernel (grid: N/32 x M/64 workgroups). In
-  // fp32 (the scorer's dense layer over all [MASK] rows, the fp32 validation
-  // build) that pays up to M = 1024: the 64 x 128 tiles below would leave
-  // most CUs idle with a 24-step fp32 K loop each.
-  if (a0.M <= 128)
-    return precision == PREC_BF16  ? launch_skinny<bf16>(epi, a0, s)
-           : precision == PREC_F16 ? launch_skinny<f16>(epi, a0, s)
-                                   : launch_skinny<float>(epi, a0, s);
-  if (precision == PREC_F32 && a0.M <= 1024) return launch_skinny<float>(epi, a0, s);
-  GemmArgs a = a0;
-  // N groups per XCD sweep: keep the group's slice of B (N/groups rows of
-  // K elements) within about 2 MB of L2.
-  const size_t b_bytes = (size_t)a.N * a.K * (prec16(precision) ? 2 : 4);
-  const int tiles_n = a.N / 128;
-  int groups = 1;
-  while (b_bytes / groups > (2u << 20) && groups < tiles_n) {
-    groups++;
-    while (tiles_n % groups) groups++;
+template <class T>
+hipError_t launch_f32(const GemmArgs &a, hipStream_t s) {
+  if (F64x64::count(a) <= kCUs) return launch_tile<T, F64x64, EPI_F32>(a, s);
+  if (F64x128::count(a) <= kCUs) return launch_tile<T, F64x128, EPI_F32>(a, s);
+  if (F128x128::count(a) <= kCUs) return launch_tile<T, F128x128, EPI_F32>(a, s);
+  if (a.N % 256 == 0 && F64x256::count(a) <= kCUs) return launch_tile<T, F64x256, EPI_F32>(a, s);
+  if (a.N % 192) return launch_tile<T, F128x128s, EPI_F32>(a, s);
+  if (F128x192::count(a) <= kCUs) return launch_tile<T, F128x192, EPI_F32>(a, s);
+  return launch_tile<T, F256x192, EPI_F32>(a, s);
+}
+
+// Operand-type outputs (store, GeGLU and their folded-LayerNorm forms), by
+// the same rule; past one round of 128 x 128, 256 x 128 tiles at two
+// workgroups per CU, whose epilogues and DMA stalls overlap the other's
+// MFMAs. N = 2304, K = 768, store / GeGLU, isolated launches as above (us):
+//   64 x 64 (two waves)  208 rows  5.8 /  6.1  (64 x 128:  6.8 /  7.1)
+//   128 x 64             600       7.0 /  7.4  (64 x 128:  8.1 /  8.5)
+//   128 x 128, 8 waves 1,500       9.4 /  9.8  (128 x 128, 64-byte stages: 12.5 / 13.0)
+//   256 x 128, 8 waves 3,000      15.8 / 16.2  (128 x 128, 64-byte stages: 18.3 / 18.5)
+// At 64 x 64 the line lies at 160 workgroups: 252 of them (448 rows) took
+// 7.2 us against 6.8 for 128 x 64.
+typedef Tile<64, 64, 128, 5, 1, 2, 1, true> S64x64;
+typedef Tile<128, 64, 128, 4, 1, 4, 1, true> S128x64;
+typedef Tile<128, 128, 128, 4, 1, 4, 2, true> S128x128;
+typedef Tile<256, 128, 128, 3, 1, 4, 2> S256x128;
+typedef Tile<128, 128, 64, 3, 3, 2, 2> S128x128s;
+typedef Tile<256, 128, 64, 3, 2, 2, 2> S256x128s;
+
+template <class T, int EPI, int PC = 0>
+hipError_t launch_store(const GemmArgs &a, hipStream_t s, const LnFold *ln = nullptr) {
+  constexpr bool gated = EPI == EPI_GEGLU || EPI == EPI_GEGLU_KEEP || EPI == EPI_GEGLU_LN;
+  if constexpr (PC != kLnPartWide) {
+    if (S64x64::count(a) <= 160) return launch_tile<T, S64x64, EPI, PC>(a, s, ln);
+    if (S128x64::count(a) <= kCUs) return launch_tile<T, S128x64, EPI, PC>(a, s, ln);
+    if (S128x128::count(a) <= kCUs) return launch_tile<T, S128x128, EPI, PC>(a, s, ln);
+    if (S256x128::count(a) <= kCUs) return launch_tile<T, S256x128, EPI, PC>(a, s, ln);
   }
-  a.ngroups = groups;
-  a.order = 0;
-  // Tile configs (measured on cfg3 shapes, 2304- and 768-wide outputs):
-  //  * M <= 1024: 64 x 128, 128-byte K stages, 4 stages, 1 workgroup per CU;
-  //  * paired / store epilogues (N = 2304): 256 x 128, 64-byte stages x 3
-  //    (72 KB LDS), two workgroups per CU so one tile's epilogue and DMA
-  //    stalls overlap the other's MFMAs;
-  //  * fp32 epilogue with N a multiple of 192 (the 768-wide Wo / MlpWo and
-  //    dX GEMMs): 192-column tiles (below); other fp32 outputs and the GeGLU
-  //    backward (training): 128 x 128, 64-byte stages x 3 (48 KB), three
-  //    workgroups per CU.
-  //  * medium M (the trainer's micro-batches: a few thousand rows) has too
-  //    few large tiles to fill 256 CUs: up to 4096 rows the fp32 and the
-  //    narrow (N <= 1024) store epilogues take 64 x 128 tiles and the wide
-  //    store 128 x 128; the GeGLU epilogues keep 128 x 128 up to 8192 rows
-  //    (isolated launches on the training shapes, 3840 rows: Wi + GeGLU 36.4
-  //    -> 31.3 us, dX GEMMs N = 768 K = 2304 32.3 -> 30.4 us, dctx 16.0 ->
-  //    12.6 us).
-  if (precision == PREC_BF16) return launch_gemm16<bf16>(epi, a, s, ln);
-  if (precision == PREC_F16) return launch_gemm16<f16>(epi, a, s, ln);
-  if (a.M <= 1024) return launch_cfg<float, 64, 128, 128, 4, 1>(epi, a, s);
-  return launch_cfg<float, 256, 128, 128, 3, 1>(epi, a, s);
+  if (a.M <= (gated ? 8192 : 4096)) return launch_tile<T, S128x128s, EPI, PC>(a, s, ln);
+  return launch_tile<T, S256x128s, EPI, PC>(a, s, ln);
 }
 
-// The folded-LayerNorm forms on the tiles launch_gemm16 gives their plain
-// counterparts at M > 1024 (the 192-column residual tiles; the store and
-// GeGLU tiles of N > 1024).
-template <class T, int BM, int BN, int RB, int NSTAGE, int WPE, int EPI>
-hipError_t launch_fold_cfg(const GemmArgs &a, const LnFold &ln, hipStream_t s) {
-  const int tiles = ((a.M + BM - 1) / BM) * (a.N / BN);
-  hipLaunchKernelGGL((gemm_nt_ln_kernel<T, BM, BN, RB, NSTAGE, EPI, WPE, 2, 2>), dim3(tiles), dim3(256), 0, s, a, ln);
-  return hipGetLastError();
-}
-
+// The folded-LayerNorm forms. The statistics' parts are kLnPartNarrow columns
+// for forwards of up to kLnNarrowTokens tokens (the residual tiles of one
+// round there are 64 and 128 columns wide), else kLnPartWide (192-column
+// tiles, a third of the pairs for the consumers' 18 N-tiles to re-read).
 template <class T>
-hipError_t launch_gemm_fold(int epi, const GemmArgs &a, const LnFold *ln, hipStream_t s) {
-  const bool medium = a.M <= 4096;
-  if (!ln) return hipErrorInvalidValue;
+hipError_t launch_fold(int epi, const GemmArgs &a, const LnFold *ln, hipStream_t s) {
+  if (!ln || !ln->lpart) return hipErrorInvalidValue;
+  const bool narrow = ln->lparts == kLnHidden / kLnPartNarrow;
+  if (!narrow && ln->lparts != kLnHidden / kLnPartWide) return hipErrorInvalidValue;
   if (epi == EPI_F32_LN) {
-    if (a.N % kLnPartCols || ln->lparts != a.N / kLnPartCols || !a.accumulate || a.ldc % 4 || a.n_store != a.N ||
-        !ln->fx || !ln->lw || !ln->lpart)
+    if (a.N != kLnHidden || !a.accumulate || a.ldc % 4 || a.n_store != a.N || !ln->fx || !ln->lw)
       return hipErrorInvalidValue;
-    if (medium) return launch_cfg_one<T, 64, 192, 128, 4, 1, EPI_F32_LN>(a, s, 1, ln);
-    return launch_cfg_one<T, 256, 192, 128, 2, 2, EPI_F32_LN, 4>(a, s, 1, ln);
+    if (narrow) {
+      if (F64x64::count(a) <= kCUs) return launch_tile<T, F64x64, EPI_F32_LN, kLnPartNarrow>(a, s, ln);
+      if (F64x128::count(a) <= kCUs) return launch_tile<T, F64x128, EPI_F32_LN, kLnPartNarrow>(a, s, ln);
+      return launch_tile<T, F128x128, EPI_F32_LN, kLnPartNarrow>(a, s, ln);
+    }
+    if (F128x192::count(a) <= kCUs) return launch_tile<T, F128x192, EPI_F32_LN, kLnPartWide>(a, s, ln);
+    return launch_tile<T, F256x192, EPI_F32_LN, kLnPartWide>(a, s, ln);
   }
-  if (ln->lparts < 1 || ln->lparts > 8 || ln->lparts * kLnPartCols != a.K || !ln->lpart || !ln->lcs ||
-      !ln->mean_out || (epi == EPI_STORE_LN && a.N <= 1024))
-    return hipErrorInvalidValue;
-  if (epi == EPI_STORE_LN) {
-    if (medium) return launch_fold_cfg<T, 128, 128, 64, 3, 3, EPI_STORE_LN>(a, *ln, s);
-    return launch_fold_cfg<T, 256, 128, 64, 3, 2, EPI_STORE_LN>(a, *ln, s);
-  }
-  if (a.M <= 8192) return launch_fold_cfg<T, 128, 128, 64, 3, 3, EPI_GEGLU_LN>(a, *ln, s);
-  return launch_fold_cfg<T, 256, 128, 64, 3, 2, EPI_GEGLU_LN>(a, *ln, s);
+  if (a.K != kLnHidden || !ln->lcs || !ln->mean_out) return hipErrorInvalidValue;
+  if (epi == EPI_STORE_LN)
+    return narrow ? launch_store<T, EPI_STORE_LN, kLnPartNarrow>(a, s, ln)
+                  : launch_store<T, EPI_STORE_LN, kLnPartWide>(a, s, ln);
+  return narrow ? launch_store<T, EPI_GEGLU_LN, kLnPartNarrow>(a, s, ln)
+                : launch_store<T, EPI_GEGLU_LN, kLnPartWide>(a, s, ln);
 }
 
 template <class T>
 hipError_t launch_gemm16(int epi, const GemmArgs &a, hipStream_t s, const LnFold *ln) {
-  if (epi >= EPI_F32_LN) return launch_gemm_fold<T>(epi, a, ln, s);
-  const bool small = a.M <= 1024;
-  {
-    if (small) return launch_cfg<T, 64, 128, 128, 4, 1>(epi, a, s);
-    const bool medium = a.M <= 4096;
-    if (epi == EPI_F32 && a.N % 192 == 0) {
-      // 768-wide outputs in 192-column tiles: 3,840 rows make 240 tiles of
-      // 64 x 192 for 256 CUs where 64 x 128 made 360 (dX GEMM N = 768,
-      // K = 2304: 30.6 -> 24.2 us isolated; Wo 16.2 -> 12.7 us). Above 4096
-      // rows, 256 x 192 tiles of 8 waves (64 x 96 each) at one workgroup per
-      // CU (112 KB of LDS: 2 stages of 64 K elements). These GEMMs are bound
-      // by the vector memory path (TA/TD), not by HBM or the matrix cores:
-      // every byte staged into LDS and every fp32 residual byte passes it.
-      // Per output element the main loop stages (1/BN + 1/BM) K operand
-      // elements: 0.0091 K for 256 x 192 against 0.0104 K for 128 x 384
-      // (-12.5%), and the residual read + write is the same. Alternating
-      // runs on one box, cfg3: Wo 80.7 -> 75.7 us, MlpWo 90.5 -> 83.8 us per
-      // launch, forward 2.80 -> 2.82M tokens/s; TA busy 0.64 -> 0.38, TD
-      // 0.77 -> 0.71 (128 x 384 tiles of 8 waves with 3 stages of 32 K
-      // elements before; 128 x 192 at two workgroups per CU was 2-4% slower
-      // still).
-      if (medium) return launch_cfg_one<T, 64, 192, 128, 4, 1>(a, s);
-      return launch_cfg_one<T, 256, 192, 128, 2, 2, EPI_F32, 4>(a, s);
-    }
-    // GeGLU backward (N = 1152) at medium M: 64 x 192 at two workgroups per
-    // CU (3840 rows: 30.2 -> 25.8 us isolated). Training only (bf16).
-    if constexpr (!std::is_same<T, f16>::value)
-      if (epi == EPI_GEGLU_BWD && medium && a.N % 192 == 0)
-        return launch_cfg_one<T, 64, 192, 64, 4, 2, EPI_GEGLU_BWD>(a, s);
-    if (epi == EPI_F32 || (epi == EPI_STORE && a.N <= 1024 && a.M <= 16384)) {
-      if (medium) return launch_cfg<T, 64, 128, 128, 4, 1>(epi, a, s);
-      return launch_cfg<T, 128, 128, 64, 3, 3>(epi, a, s);
-    }
-    if (epi == EPI_GEGLU_BWD || (epi == EPI_STORE && medium) ||
-        ((epi == EPI_GEGLU || epi == EPI_GEGLU_KEEP) && a.M <= 8192))
-      return launch_cfg<T, 128, 128, 64, 3, 3>(epi, a, s);
-    return launch_cfg<T, 256, 128, 64, 3, 2>(epi, a, s);
+  switch (epi) {
+    case EPI_F32: return launch_f32<T>(a, s);
+    case EPI_STORE: return launch_store<T, EPI_STORE>(a, s);
+    case EPI_GEGLU: return launch_store<T, EPI_GEGLU>(a, s);
+    case EPI_F32_LN: case EPI_STORE_LN: case EPI_GEGLU_LN: return launch_fold<T>(epi, a, ln, s);
   }
+  if constexpr (std::is_same<T, bf16>::value) {  // training: bf16 only
+    if (epi == EPI_GEGLU_KEEP) return launch_store<T, EPI_GEGLU_KEEP>(a, s);
+    // GeGLU backward (N = 1152) at medium M: 64 x 192 at two workgroups per
+    // CU (3840 rows: 30.2 -> 25.8 us isolated).
+    if (a.M <= 1024) return launch_tile<T, Tile<64, 128, 128, 4, 1, 2, 2>, EPI_GEGLU_BWD>(a, s);
+    if (a.M <= 4096 && a.N % 192 == 0) return launch_tile<T, Tile<64, 192, 64, 4, 2, 2, 2>, EPI_GEGLU_BWD>(a, s);
+    return launch_tile<T, F128x128s, EPI_GEGLU_BWD>(a, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+template <class C>
+hipError_t launch_gemm_f32_tile(int epi, const GemmArgs &a, hipStream_t s) {
+  switch (epi) {
+    case EPI_F32: return launch_tile<float, C, EPI_F32>(a, s);
+    case EPI_STORE: return launch_tile<float, C, EPI_STORE>(a, s);
+    case EPI_GEGLU: return launch_tile<float, C, EPI_GEGLU>(a, s);
+    case EPI_GEGLU_KEEP: return launch_tile<float, C, EPI_GEGLU_KEEP>(a, s);
+    case EPI_GEGLU_BWD: return launch_tile<float, C, EPI_GEGLU_BWD>(a, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_gemm(int precision, int epi, const GemmArgs &a, hipStream_t s, const LnFold *ln) {
+  if (a.M <= 0) return hipSuccess;
+  if (!gemm_epi_ok(precision, epi, a.M) || (epi == EPI_GEGLU_BWD && (!a.gin || a.ldc % 8))) return hipErrorInvalidValue;
+  // Small M goes to the whole-K kernel (grid: N/32 x M/64 workgroups). In
+  // fp32 (the scorer's dense layer over all [MASK] rows, the fp32 validation
+  // build) that pays up to M = 1024: the 64 x 128 tiles below would leave
+  // most CUs idle with a 24-step fp32 K loop each.
+  if (a.M <= 128)
+    return precision == PREC_BF16  ? launch_skinny<bf16>(epi, a, s)
+           : precision == PREC_F16 ? launch_skinny<f16>(epi, a, s)
+                                   : launch_skinny<float>(epi, a, s);
+  if (precision == PREC_BF16) return launch_gemm16<bf16>(epi, a, s, ln);
+  if (precision == PREC_F16) return launch_gemm16<f16>(epi, a, s, ln);
+  if (a.M <= 1024) return launch_skinny<float>(epi, a, s);
+  return launch_gemm_f32_tile<Tile<256, 128, 128, 3, 1, 2, 2>>(epi, a, s);
 }

@@ -19,16 +19,6 @@ namespace {
 // l % 8 only); quad_perm [2,3,0,1] and [1,0,3,2] are lane ^ 2 and lane ^ 1.
 // Floating-point addition is commutative, so every lane ends with the same
 // bits as the shuffle butterfly v += __shfl_xor(v, o).
-template <int CTRL>
-__device__ __forceinline__ unsigned dpp_u32(unsigned x) {
-  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-  const unsigned long long u = __double_as_longlong(v);
-  const unsigned lo = dpp_u32<CTRL>((unsigned)u), hi = dpp_u32<CTRL>((unsigned)(u >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
 __device__ __forceinline__ double wave_sum(double v) {
   {
     const unsigned long long u = __double_as_longlong(v);
@@ -470,24 +460,28 @@ hipError_t launch_prologue(int precision, const int *pos, const int *opt, const 
 // cs[n] = sum_k lw[k] * B[n][k] (B bf16 or fp16, N x K), summed in fp64 and rounded
 // to float: the column sums of the LayerNorm-weighted projection that a
 // folded LayerNorm's consumer GEMM subtracts. One wave per row n.
+// blockIdx.y: the job.
 template <class T>
-__global__ __launch_bounds__(256) void fold_colsum_kernel(const T *B, int N, int K, const float *lw, float *cs) {
+__global__ __launch_bounds__(256) void fold_colsum_kernel(FoldJobs j) {
+  const auto &job = j.job[blockIdx.y];
   const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (n >= N) return;
-  const T *b = B + (size_t)n * K;
+  if (n >= job.N) return;
+  const T *b = (const T *)job.B + (size_t)n * j.K;
   double acc = 0;
-  for (int k = lane; k < K; k += 64) acc += (double)lw[k] * (double)(float)b[k];
+  for (int k = lane; k < j.K; k += 64) acc += (double)job.lw[k] * (double)(float)b[k];
   acc = wave_sum(acc);
-  if (lane == 0) cs[n] = (float)acc;
+  if (lane == 0) job.cs[n] = (float)acc;
 }
 
-hipError_t launch_fold_colsum(int precision, const void *B, int N, int K, const float *lw, float *cs,
-                              hipStream_t s) {
+hipError_t launch_fold_colsum(int precision, const FoldJobs &j, hipStream_t s) {
+  int N = 0;
+  for (int i = 0; i < j.n; i++) N = N > j.job[i].N ? N : j.job[i].N;
   if (N <= 0) return hipSuccess;
+  const dim3 grid((N + 3) / 4, j.n), block(256);
   if (precision == PREC_BF16)
-    hipLaunchKernelGGL(fold_colsum_kernel<bf16>, dim3((N + 3) / 4), dim3(256), 0, s, (const bf16 *)B, N, K, lw, cs);
+    hipLaunchKernelGGL(fold_colsum_kernel<bf16>, grid, block, 0, s, j);
   else if (precision == PREC_F16)
-    hipLaunchKernelGGL(fold_colsum_kernel<f16>, dim3((N + 3) / 4), dim3(256), 0, s, (const f16 *)B, N, K, lw, cs);
+    hipLaunchKernelGGL(fold_colsum_kernel<f16>, grid, block, 0, s, j);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

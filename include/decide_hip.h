@@ -207,18 +207,21 @@ int dn_set_stream_split(dn_ctx *ctx, int min_tokens);
  * (forward.go:212-243 runs every layer over all tokens, then gathers). */
 int dn_set_row_tail(dn_ctx *ctx, int min_tokens);
 
-/* bf16 and fp16 inference forwards of more than 1024 tokens (or parts of a two-stream
- * forward) run attn_norm and mlp_norm folded into the GEMMs around them: the
+/* bf16 and fp16 inference forwards of more than 128 tokens (hidden 768) run
+ * attn_norm and mlp_norm folded into the GEMMs around them: the
  * residual GEMM before a LayerNorm (Wo, MlpWo) also writes the norm's operand
  * ((x - m) * w in the operand type) of the new residual row x, with m the row mean of the
- * previous LayerNorm and w the norm weight, and per 192 columns the row's
+ * previous LayerNorm and w the norm weight, and per part of 64 columns (192 in
+ * forwards of more than 5,376 tokens) the row's
  * (mean, M2) as an fp32 pair (reduced in fp64); the GEMM after it (QKV, Wi)
  * merges those (in fp64) into the row's
  * mean and rstd and computes rstd * (A.B^T - (mean - m) * sum_k w[k] B[n][k]),
  * i.e. LayerNorm(x).B^T, so the LayerNorm launches (a read of the fp32
  * residual stream each) disappear. The logits move by the bf16 rounding of
  * the operand (x - m) * w instead of the normalised row, the same size of
- * error. on = 0 runs the LayerNorm kernels; the default is on. No
+ * error. on = 0 runs the LayerNorm kernels in forwards (or parts of a
+ * two-stream forward) of more than 1024 tokens; smaller ones always fold. The
+ * default is on. No
  * counterpart in the reference (forward.go:289-294, :324 normalise, then
  * project). */
 int dn_set_ln_fold(dn_ctx *ctx, int on);

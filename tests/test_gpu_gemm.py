@@ -156,6 +156,43 @@ def test_gemm_16bit_device_store(eng, prec, M, N, K):
     assert float((err / (1e-5 * bound + half_ulp * 1.0001)).max()) <= 1.0
 
 
+@pytest.mark.parametrize("prec,M,N,K,store", [
+    # fp32 output, N = 768: 64 x 64 from its first row count to the last of one
+    # round (21 x 12 workgroups), 64 x 128, 128 x 128, 64 x 256, 128 x 192
+    ("bf16", 129, 768, 64, False), ("bf16", 129, 768, 192, False), ("fp16", 1344, 768, 320, False),
+    ("bf16", 1345, 768, 1152, False), ("bf16", 2689, 768, 768, False), ("fp16", 5377, 768, 768, False),
+    ("bf16", 5441, 768, 1152, False), ("bf16", 8193, 768, 768, False), ("bf16", 200, 128, 256, False),
+    # stored outputs, N = 2304: 64 x 64, 128 x 64, 128 x 128, 256 x 128
+    ("bf16", 129, 2304, 64, True), ("fp16", 256, 2304, 256, True), ("bf16", 257, 2304, 768, True),
+    ("bf16", 897, 2304, 128, True), ("fp16", 1793, 2304, 768, True), ("bf16", 3585, 2304, 192, True),
+    ("bf16", 4097, 128, 768, True)])
+def test_gemm_tile_boundaries(eng, prec, M, N, K, store):
+    """Row counts on both sides of each tile rule and K from one stage up
+    (fewer stages than the ring holds): every output against float64, at the
+    fp32 bound (stored outputs: plus half an ulp of the operand type), and rows
+    past M untouched."""
+    import torch
+
+    dt = torch.bfloat16 if prec == "bf16" else torch.float16
+    g = torch.Generator().manual_seed(M + K)
+    A = torch.randn(M, K, generator=g).to(dt)
+    B = (torch.randn(N, K, generator=g) * 0.02).to(dt)
+    dA, dB = A.cuda(), B.cuda()
+    dC = torch.full((M + 1, N), 7.0, dtype=dt if store else torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    if store:
+        eng.gemm_device_store(prec, M, N, K, dA.data_ptr(), dB.data_ptr(), dC.data_ptr())
+    else:
+        eng.gemm_device(prec, M, N, K, dA.data_ptr(), dB.data_ptr(), dC.data_ptr())
+    eng.synchronize()
+    exact = dA.double() @ dB.double().T
+    bound = 1e-5 * (dA.double().abs() @ dB.double().abs().T)
+    if store:
+        bound += exact.abs() * (2.0 ** -8 if prec == "bf16" else 2.0 ** -11) * 1.0001 + 2.0 ** -25
+    assert bool(((dC[:M].double() - exact).abs() <= bound + 1e-30).all())
+    assert bool((dC[M] == 7.0).all())
+
+
 @pytest.mark.parametrize("prec", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("M,N,K", [(1, 2304, 768), (31, 768, 1152), (33, 384, 768), (64, 2304, 768),
                                    (65, 768, 768), (112, 768, 1152), (128, 2304, 64), (100, 128, 4096)])

@@ -93,3 +93,24 @@ def test_small_m_operand_paths_agree(base_small, prec):
             assert np.array_equal(lds, regs), (total, float(np.max(np.abs(lds - regs))))
     finally:
         eng.set_small_m_loads(1)
+
+
+@pytest.mark.parametrize("total", [129, 256, 257, 897, 1000, 1024, 1345])
+def test_folded_small_batch_matches_oracle(base_small, total):
+    """Batches above the small-M kernels (129 tokens up) on both sides of the
+    folded GEMMs' tile rules: attn_norm and mlp_norm run inside the GEMMs around
+    them, statistics in 64-column parts; the switch applies above 1,024 tokens
+    only."""
+    cfg, orc, engs = base_small
+    rng = np.random.default_rng(2000 + total)
+    batch = batch_with_total(total, cfg.vocab, rng)
+    oracle.set_workers(WORKERS)
+    want = orc.forward(batch)
+    for prec in ("bf16", "fp16"):
+        got = engs[prec].forward(batch)
+        compare(got, want, batch, prec)
+        try:
+            engs[prec].set_ln_fold(False)
+            assert np.array_equal(engs[prec].forward(batch), got) == (total <= 1024)
+        finally:
+            engs[prec].set_ln_fold(True)
