@@ -409,10 +409,19 @@ struct Pass {
   // split forward.
   bool fold = false;
   int ln_cols = kLnPartWide;
+  // Attention with the keys split over waves (attn_key_split), by the whole
+  // batch too.
+  bool key_split = false;
   Workspace w;
   const int32_t *ids, *pos, *opt;
   hipStream_t s;
 };
+
+// Whether attention splits a query chunk's keys over waves: batches of few work
+// items (attention.hip has both sides' times).
+bool attn_key_split(const Config &g, int nwork) {
+  return !g.generic && nwork <= (prec16(g.precision) ? kKeySplitItems16 : kKeySplitItems32);
+}
 
 // Token info, 32-token chunk summaries, attention tile classes of both layer
 // types, and the embedding gather + emb norm into cur (fp32) and xn0.
@@ -549,6 +558,7 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
   at.codes = w.codes + (sliding ? (size_t)w.nwork * ATTN_MAXKT : 0);
   at.first = w.first + (sliding ? w.nwork : 0);
   at.qt = ATTN_QT;
+  at.key_split = p.key_split ? 1 : 0;
   if (!sliding && p.wide_global && w.nwork2 > 0) {  // global layer of the two-stream forward: 256-query items
     at.work = w.work2;
     at.nwork = w.nwork2;
@@ -1033,8 +1043,14 @@ int forward_split(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_
     ps[k].pos = d_pos + t0;
     ps[k].opt = d_opt ? d_opt + t0 : nullptr;
     ps[k].s = st[k];
-    ps[k].wide_global = true;
-    rc = enqueue_prologue(c, ps[k], w.h, w.xn, nullptr, nullptr);
+  }
+  const bool key_split = attn_key_split(g, ps[0].w.nwork + ps[1].w.nwork);
+  for (Pass &p : ps) {
+    p.key_split = key_split;
+    p.wide_global = !key_split;
+  }
+  for (Pass &p : ps) {
+    rc = enqueue_prologue(c, p, p.w.h, p.w.xn, nullptr, nullptr);
     if (rc) return rc;
   }
   const bool rows_tail = tail_on_rows(c, T_total, R, false);
@@ -1140,6 +1156,7 @@ int forward_core(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_i
   ps.s = c->stream;
   ps.fold = !train && w.lmean1 && fold_eligible(c, T);
   ps.ln_cols = T <= kLnNarrowTokens ? kLnPartNarrow : kLnPartWide;
+  ps.key_split = attn_key_split(g, w.nwork);
   if (ps.fold) {
     rc = ensure_fold_cs(c, ps.s);
     if (rc) return rc;

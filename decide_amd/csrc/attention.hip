@@ -270,12 +270,6 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
   constexpr int NT = 64 * QW, R = QW >= 4 ? 1 : 4 / QW;
   static_assert(QW == 1 || QW == 2 || QW == 4 || QW == 8, "waves per workgroup");
   static_assert(QT * QW <= 8, "tile codes hold 8 query chunks");
-  // Workgroups of fewer than ATTN_WAVES waves (fp32 batches of few work
-  // items) take ATTN_WAVES / QW turns at one work item of ATTN_WAVES 32-query
-  // chunks: part `sub` of the item computes chunks sub * QW .. sub * QW + QW - 1.
-  constexpr int SUB = LIST ? 1 : ATTN_WAVES / QW;
-  static_assert(SUB * QW == ATTN_WAVES || SUB == 1, "work item parts");
-  static_assert(SUB == 1 || QT == 1, "parted work items have one query tile per wave");
   using MF = Mfma<T>;
   typedef typename MF::frag frag;
   constexpr int ROWK = D * sizeof(T) + 16;       // K tile row bytes (key-major)
@@ -301,14 +295,11 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
   // (work item, head) with the q blocks of one sequence and its 12 heads
   // adjacent: the K/V rows, RoPE factors and chunk summaries they share are
   // reused out of that XCD's L2.
-  const int total = a.nwork * a.heads * SUB;
+  const int total = a.nwork * a.heads;
   const int bid = blockIdx.x;
   int logical = bid;
   if (total % 8 == 0) logical = (bid % 8) * (total / 8) + bid / 8;
-  const int sub = logical % SUB;
-  logical /= SUB;
   const int wi = logical / a.heads, head = logical % a.heads;
-  const int wq = sub * QW + wave;  // this wave's chunk of the work item (QT query tiles each)
   int s, q0 = 0, slot0 = 0, cnt = 0, n, base;
   if constexpr (LIST) {
     if (wi >= *a.nitems) return;  // the grid is sized by an upper bound on the items
@@ -361,7 +352,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
     int qq;
     const T *qrow;
     if constexpr (LIST) {
-      const int idx = (wq * QT + t) * 32 + lr;
+      const int idx = (wave * QT + t) * 32 + lr;
       qvalid[t] = idx < cnt;
       const int r = a.rows[slot0 + (qvalid[t] ? idx : 0)];
       qrow_r[t] = r;
@@ -369,7 +360,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
       qq = min(max(a.row_tok[r] - base, 0), n - 1);
       qrow = (const T *)a.q_rows + (size_t)r * H + head * D;
     } else {
-      const int q = q0 + (wq * QT + t) * 32 + lr;
+      const int q = q0 + (wave * QT + t) * 32 + lr;
       qvalid[t] = q < n;
       qq = qvalid[t] ? q : n - 1;
       qrow = qkv + (size_t)(base + qq) * ld + head * D;
@@ -452,7 +443,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
     // This wave's classes: per query tile t and 32-key half i (uniform
     // across the wave).
     const int mycode =
-        __builtin_amdgcn_readfirstlane((sCode[kt] >> (4 * QT * wq)) & ((1u << (4 * QT)) - 1));
+        __builtin_amdgcn_readfirstlane((sCode[kt] >> (4 * QT * wave)) & ((1u << (4 * QT)) - 1));
     int hcls[QT][2];
 #pragma unroll
     for (int t = 0; t < QT; t++) {
@@ -609,11 +600,11 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
     const float l_tot = l_run[t] + __shfl_xor(l_run[t], 32);
     const float inv = 1.0f / l_tot;
     if (!LIST && a.lse && qvalid[t] && lh == 0) {
-      const int q = q0 + (wq * QT + t) * 32 + lr;
+      const int q = q0 + (wave * QT + t) * 32 + lr;
       a.lse[(size_t)(base + q) * a.heads + head] = m_run[t] * a.scale_log2 + log2f(l_tot);
     }
     if (qvalid[t]) {
-      const int q = q0 + (wq * QT + t) * 32 + lr;
+      const int q = q0 + (wave * QT + t) * 32 + lr;
       T *out = (T *)a.ctx + (size_t)(LIST ? qrow_r[t] : base + q) * H + head * D;
 #pragma unroll
       for (int i = 0; i < 2; i++)
@@ -629,6 +620,370 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
           }
         }
     }
+  }
+}
+
+// ---- few work items: the keys split over a workgroup's waves ---------------
+//
+// A batch of few work items leaves most CUs idle above, and its
+// time is the chain of key tiles one workgroup walks (one 512-token bf16
+// request: 48 workgroups, 8 tiles, 14.9 us on sliding and 19.5 us on global
+// layers; 203 tokens in fp32: 30.8 us). Here a workgroup takes one 32-query
+// chunk, and its eight waves take every eighth unit of 32 keys (the halves the
+// tile classes describe), each with its own softmax state and its own LDS
+// slab: no barrier until the end, where the partial results are merged in wave
+// order (512 tokens: 7.7 and 10.3 us; fp32, 203 tokens: 11.5 us). What is left
+// is the chain of dependent loads (work item, classes, key info, RoPE rows),
+// one or two units and the merge. The chunk's Q rows are loaded and rotated
+// once for all waves: each wave loading its own fragments, scattered over 32
+// rows, kept the CU's address unit busy (fp32 20.3 us instead of 11.5).
+// K, V and RoPE rows are read once per chunk instead of once per four. Whole
+// 22-layer forwards, keys split against the tile walk: bf16 4 x 128 tokens
+// 886 against 979 us, 1,024 tokens 1,262 / 1,337, 4 x 256 tokens (8 work items)
+// 1,159 / 1,161, 8 x 184 (16 items) 1,390 / 1,284; fp32 8 x 184 11.18 / 11.32
+// ms, 2,044 tokens (16 items) 12.3 / 13.1 ms, 4 x 1024 17.0 / 17.1 ms: hence the
+// lines at 8 and 16 items.
+
+// One unit (32 keys) of a wave's staging, the items of Staging above spread
+// over 64 lanes.
+template <class T>
+struct UnitStage {  // 16-bit: 128 (key, chunk pair) K items, 128 (key pair, 8-d group) V items
+  static constexpr int KI = 2, VI = 2;
+  uint4 k_lo[KI], k_hi[KI], v0[VI], v1[VI];
+  float4 c_lo[KI], c_hi[KI], s_lo[KI], s_hi[KI];
+};
+template <>
+struct UnitStage<float> {  // 256 (key, 4-element chunk pair) K items, 512 (key, 4-d group) V items
+  static constexpr int KI = 4, VI = 8;
+  uint4 k_lo[KI], k_hi[KI], v[VI];
+  float4 c[KI], s[KI];
+};
+
+template <class T>
+struct UnitInfo {  // per-token info of a lane's K items' keys and of key lane % 32
+  int pk[UnitStage<T>::KI];
+  int pi;
+};
+
+template <class T>
+__device__ __forceinline__ void unit_info(UnitInfo<T> &f, const int *kinfo, int base, int n, int k0, int lane) {
+  constexpr int SH = sizeof(T) == 2 ? 2 : 3;
+#pragma unroll
+  for (int j = 0; j < UnitStage<T>::KI; j++) f.pk[j] = kinfo[base + min(k0 + ((lane + 64 * j) >> SH), n - 1)];
+  f.pi = kinfo[base + min(k0 + (lane & 31), n - 1)];
+}
+
+template <class T>
+__device__ __forceinline__ void unit_load(UnitStage<T> &st, const T *qkv, int ld, int H, int head, int base, int n,
+                                          int k0, const float *cos_t, const float *sin_t, const UnitInfo<T> &f,
+                                          int lane) {
+  typedef UnitStage<T> U;
+  constexpr int SH = sizeof(T) == 2 ? 2 : 3, CH = 16 / sizeof(T);  // chunks per key 1 << SH, elements per chunk
+  // Keys past the sequence end read the last key's row; unit_store zeroes them.
+  auto row = [&](int k) { return qkv + (size_t)(unsigned)(base + min(k, n - 1)) * (unsigned)ld + head * D; };
+#pragma unroll
+  for (int j = 0; j < U::KI; j++) {
+    const int it = lane + 64 * j, key = it >> SH, c = it & ((1 << SH) - 1);
+    const T *r = row(k0 + key) + H;
+    st.k_lo[j] = *(const uint4 *)(r + CH * c);
+    st.k_hi[j] = *(const uint4 *)(r + 32 + CH * c);
+    const size_t p = (size_t)(f.pk[j] & 0xffff) * 32 + CH * c;
+    if constexpr (sizeof(T) == 2) {
+      st.c_lo[j] = *(const float4 *)(cos_t + p);
+      st.c_hi[j] = *(const float4 *)(cos_t + p + 4);
+      st.s_lo[j] = *(const float4 *)(sin_t + p);
+      st.s_hi[j] = *(const float4 *)(sin_t + p + 4);
+    } else {
+      st.c[j] = *(const float4 *)(cos_t + p);
+      st.s[j] = *(const float4 *)(sin_t + p);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < U::VI; j++) {
+    const int it = lane + 64 * j;
+    if constexpr (sizeof(T) == 2) {
+      const int k = k0 + 2 * (it & 15), g = it >> 4;
+      st.v0[j] = *(const uint4 *)(row(k) + 2 * H + 8 * g);
+      st.v1[j] = *(const uint4 *)(row(k + 1) + 2 * H + 8 * g);
+    } else {
+      st.v[j] = *(const uint4 *)(row(k0 + (it >> 4)) + 2 * H + 4 * (it & 15));
+    }
+  }
+}
+
+// K rotated and key-major, V transposed (d-major; 16-bit: key pairs packed and
+// ordered as in stage_store), and the keys' mask fields.
+template <class T, int ROWK, int ROWV>
+__device__ __forceinline__ void unit_store(const UnitStage<T> &st, char *sK, char *sV, int *sKo, int *sKw, int n,
+                                           int k0, int info, int half_window, int lane) {
+  typedef UnitStage<T> U;
+  constexpr int SH = sizeof(T) == 2 ? 2 : 3;
+#pragma unroll
+  for (int j = 0; j < U::KI; j++) {
+    const int it = lane + 64 * j, key = it >> SH, c = it & ((1 << SH) - 1);
+    const bool ok = k0 + key < n;
+    const uint4 kl = keep_if(ok, st.k_lo[j]), kh = keep_if(ok, st.k_hi[j]);
+    if constexpr (sizeof(T) == 2) {
+      const uint32_t klo[4] = {kl.x, kl.y, kl.z, kl.w}, khi[4] = {kh.x, kh.y, kh.z, kh.w};
+      const float cs[8] = {st.c_lo[j].x, st.c_lo[j].y, st.c_lo[j].z, st.c_lo[j].w,
+                           st.c_hi[j].x, st.c_hi[j].y, st.c_hi[j].z, st.c_hi[j].w};
+      const float sn[8] = {st.s_lo[j].x, st.s_lo[j].y, st.s_lo[j].z, st.s_lo[j].w,
+                           st.s_hi[j].x, st.s_hi[j].y, st.s_hi[j].z, st.s_hi[j].w};
+      uint32_t po[4], ph[4];
+#pragma unroll
+      for (int w = 0; w < 4; w++) {
+        float a0 = lo16<T>(klo[w]), a1 = hi16<T>(klo[w]), b0 = lo16<T>(khi[w]), b1 = hi16<T>(khi[w]);
+        rope1(a0, b0, cs[2 * w], sn[2 * w]);
+        rope1(a1, b1, cs[2 * w + 1], sn[2 * w + 1]);
+        po[w] = pack16<T>(a0, a1);
+        ph[w] = pack16<T>(b0, b1);
+      }
+      *(uint4 *)(sK + key * ROWK + 16 * c) = make_uint4(po[0], po[1], po[2], po[3]);
+      *(uint4 *)(sK + key * ROWK + 64 + 16 * c) = make_uint4(ph[0], ph[1], ph[2], ph[3]);
+    } else {
+      float4 lo = *(const float4 *)&kl, hi = *(const float4 *)&kh;
+      rope1(lo.x, hi.x, st.c[j].x, st.s[j].x);
+      rope1(lo.y, hi.y, st.c[j].y, st.s[j].y);
+      rope1(lo.z, hi.z, st.c[j].z, st.s[j].z);
+      rope1(lo.w, hi.w, st.c[j].w, st.s[j].w);
+      *(float4 *)(sK + key * ROWK + 16 * c) = lo;
+      *(float4 *)(sK + key * ROWK + 128 + 16 * c) = hi;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < U::VI; j++) {
+    const int it = lane + 64 * j;
+    if constexpr (sizeof(T) == 2) {
+      const int p = it & 15, g = it >> 4, lp = p & 7, q4 = lp >> 1;
+      const int pw = (p & ~7) + ((((q4 & 1) << 1) | (q4 >> 1)) << 1) + (lp & 1);
+      const uint4 v0 = keep_if(k0 + 2 * p < n, st.v0[j]), v1 = keep_if(k0 + 2 * p + 1 < n, st.v1[j]);
+      const uint32_t va[4] = {v0.x, v0.y, v0.z, v0.w}, vb[4] = {v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+      for (int w = 0; w < 4; w++) {
+        *(uint32_t *)(sV + (8 * g + 2 * w) * ROWV + 4 * pw) = __builtin_amdgcn_perm(vb[w], va[w], 0x05040100u);
+        *(uint32_t *)(sV + (8 * g + 2 * w + 1) * ROWV + 4 * pw) = __builtin_amdgcn_perm(vb[w], va[w], 0x07060302u);
+      }
+    } else {
+      const int key = it >> 4, g = it & 15;
+      const uint4 v = keep_if(k0 + key < n, st.v[j]);
+      *(uint32_t *)(sV + (4 * g + 0) * ROWV + 4 * key) = v.x;
+      *(uint32_t *)(sV + (4 * g + 1) * ROWV + 4 * key) = v.y;
+      *(uint32_t *)(sV + (4 * g + 2) * ROWV + 4 * key) = v.z;
+      *(uint32_t *)(sV + (4 * g + 3) * ROWV + 4 * key) = v.w;
+    }
+  }
+  if (lane < 32) {
+    const int inf = k0 + lane < n ? info : (int)0xffff0000u;
+    sKo[lane] = (inf >> 16) - 1;
+    sKw[lane] = (inf & 0xffff) + half_window;
+  }
+}
+
+template <class T, bool LOCAL>
+__global__ __launch_bounds__(512) void attention_ks_kernel(AttnArgs a) {
+  using MF = Mfma<T>;
+  typedef typename MF::frag frag;
+  constexpr int QW = 8;
+  static_assert(ATTN_MAXKT * 2 <= 64 * QW, "a wave's units fit its lanes");
+  constexpr int NKS = D / MF::KSTEP, NPV = 32 / MF::KSTEP;
+  constexpr int ROWK = D * sizeof(T) + 16, ROWV = 32 * sizeof(T) + 16;
+  constexpr int ROWO = D + 4;  // floats per row of a wave's partial output
+  constexpr int SLAB = 32 * ROWK + D * ROWV + 256;
+  static_assert(32 * ROWO * 4 + 256 <= SLAB, "a wave's partial result fits its slab");
+  __shared__ __attribute__((aligned(16))) char smem[QW * SLAB];
+  __shared__ __attribute__((aligned(16))) char sQ[32 * ROWK];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 31, lh = lane >> 5;
+  // (work item, head, chunk), XCD-aware as above; a work item holds
+  // ATTN_WAVES chunks of 32 queries.
+  const int total = a.nwork * a.heads * ATTN_WAVES;
+  int logical = blockIdx.x;
+  if (total % 8 == 0) logical = (logical % 8) * (total / 8) + logical / 8;
+  const int chunk = logical % ATTN_WAVES, wi = logical / ATTN_WAVES / a.heads, head = logical / ATTN_WAVES % a.heads;
+  const int4 wk = a.work[wi];
+  const int q0 = wk.y + 32 * chunk, base = wk.z, n = wk.w;
+  if (q0 >= n) return;  // the whole workgroup
+  const int H = a.H, ld = 3 * H;
+  const T *qkv = (const T *)a.qkv;
+
+  // This wave's units: wave + QW * l for lane l, with their classes (read
+  // beside the work item, not after its length).
+  const int u0 = wave + QW * lane;
+  const uint32_t code = a.codes[(size_t)wi * ATTN_MAXKT + min(u0 >> 1, ATTN_MAXKT - 1)];
+  // The chunk's Q rows, rotated once for every wave: thread t takes two
+  // element pairs (i, i + 32) of row t / 16 (or four of row t / 8).
+  constexpr int QE = 32 * 32 / (64 * QW);  // pairs per thread
+  const int qr = tid / (32 / QE), qi = tid % (32 / QE) * QE, qq = min(q0 + qr, n - 1);
+  const T *qrow = qkv + (size_t)(base + qq) * ld + head * D + qi;
+  typedef T QV __attribute__((ext_vector_type(QE)));
+  typedef float FV __attribute__((ext_vector_type(QE)));
+  QV qlo = *(const QV *)qrow, qhi = *(const QV *)(qrow + 32);
+  const size_t qp = (size_t)(a.kinfo[base + qq] & 0xffff) * 32 + qi;
+  const FV qc = *(const FV *)(a.cos_t + qp), qs = *(const FV *)(a.sin_t + qp);
+  const int qinfo = a.kinfo[base + min(q0 + lr, n - 1)];
+  const int cls = u0 < (n + 31) / 32 ? (code >> (4 * chunk + 2 * (u0 & 1))) & 3 : 0;
+  uint64_t todo = __ballot(cls != 0);
+  auto take = [&]() {  // the next unit's lane index, or -1
+    if (!todo) return -1;
+    const int l = __builtin_ctzll(todo);
+    todo &= todo - 1;
+    return l;
+  };
+  int cur = take(), nxt = take();
+  UnitStage<T> st;
+  UnitInfo<T> f;
+  if (cur >= 0) {
+    unit_info<T>(f, a.kinfo, base, n, 32 * (wave + QW * cur), lane);
+    unit_load<T>(st, qkv, ld, H, head, base, n, 32 * (wave + QW * cur), a.cos_t, a.sin_t, f, lane);
+  }
+  int info = f.pi;
+  if (nxt >= 0) unit_info<T>(f, a.kinfo, base, n, 32 * (wave + QW * nxt), lane);
+#pragma unroll
+  for (int e = 0; e < QE; e++) {
+    float x = (float)qlo[e], y = (float)qhi[e];
+    rope1(x, y, qc[e], qs[e]);
+    qlo[e] = to_elem<T>(x);
+    qhi[e] = to_elem<T>(y);
+  }
+  *(QV *)(sQ + qr * ROWK + qi * sizeof(T)) = qlo;
+  *(QV *)(sQ + qr * ROWK + (32 + qi) * sizeof(T)) = qhi;
+  const int qopt = (qinfo >> 16) - 1, qpos = qinfo & 0xffff;
+  __syncthreads();
+  frag qf[NKS];
+#pragma unroll
+  for (int ks = 0; ks < NKS; ks++)
+    qf[ks] = *(const frag *)(sQ + lr * ROWK + (ks * MF::KSTEP + lh * MF::SLOTS) * (int)sizeof(T));
+
+  char *const slab = smem + wave * SLAB, *const sK = slab, *const sV = slab + 32 * ROWK;
+  int *const sKo = (int *)(sV + D * ROWV), *const sKw = sKo + 32;
+  f32x16 ot[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) ot[i][e] = 0.0f;
+  float m_run = -INFINITY, l_run = 0.0f;
+  const unsigned win2 = (unsigned)(2 * a.half_window);
+  while (cur >= 0) {
+    const int k0 = 32 * (wave + QW * cur), kc = __builtin_amdgcn_readlane(cls, cur);
+    unit_store<T, ROWK, ROWV>(st, sK, sV, sKo, sKw, n, k0, info, a.half_window, lane);
+    // The next unit's loads run under this one's arithmetic.
+    const int nn = take();
+    if (nxt >= 0) {
+      unit_load<T>(st, qkv, ld, H, head, base, n, 32 * (wave + QW * nxt), a.cos_t, a.sin_t, f, lane);
+      info = f.pi;
+      if (nn >= 0) unit_info<T>(f, a.kinfo, base, n, 32 * (wave + QW * nn), lane);
+    }
+    // Other lanes' rows: written and read by this wave alone, in order.
+    __builtin_amdgcn_wave_barrier();
+    f32x16 sT = {};
+#pragma unroll
+    for (int ks = 0; ks < NKS; ks++)
+      sT = MF::mma(*(const frag *)(sK + lr * ROWK + (ks * MF::KSTEP + lh * MF::SLOTS) * (int)sizeof(T)), qf[ks], sT);
+    if (kc == 2) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const int kl = 8 * g + 4 * lh;
+        const int4 ko4 = *(const int4 *)(sKo + kl), kw4 = *(const int4 *)(sKw + kl);
+        const int kos[4] = {ko4.x, ko4.y, ko4.z, ko4.w}, kws[4] = {kw4.x, kw4.y, kw4.z, kw4.w};
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          bool ok = (kos[u] == -1) | (kos[u] == qopt);
+          if constexpr (LOCAL) ok = ok & ((unsigned)(kws[u] - qpos) <= win2);
+          sT[4 * g + u] = ok ? sT[4 * g + u] : -INFINITY;
+        }
+      }
+    }
+    float mx = sT[0];
+#pragma unroll
+    for (int e = 1; e < 16; e++) mx = fmaxf(mx, sT[e]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(m_run, mx), m_use = m_new == -INFINITY ? 0.0f : m_new;
+    const float c = a.scale_log2, mc = -m_use * c;
+    const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * c);
+    float psum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      const float p = __builtin_amdgcn_exp2f(fmaf(sT[e], c, mc));
+      sT[e] = p;
+      psum += p;
+    }
+    l_run = l_run * alpha + psum;
+    m_run = m_new;
+    if (__ballot(alpha != 1.0f)) {
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) ot[i][e] *= alpha;
+    }
+#pragma unroll
+    for (int ks = 0; ks < NPV; ks++) {
+      frag pf;
+      if constexpr (sizeof(T) == 2) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) pf[u] = to_elem<T>(sT[8 * ks + u]);
+      } else {
+        pf = sT[ks];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const char *vrow = sV + (i * 32 + lr) * ROWV;
+        frag vf;
+        if constexpr (sizeof(T) == 2) vf = *(const frag *)(vrow + 32 * ks + 16 * lh);
+        else vf = *(const float *)(vrow + (8 * (ks >> 2) + 4 * lh + (ks & 3)) * 4);
+        ot[i] = MF::mma(vf, pf, ot[i]);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    cur = nxt;
+    nxt = nn;
+  }
+
+  // The waves' partial outputs, each in its own slab, merged in wave order.
+  float *const sO = (float *)slab, *const sM = sO + 32 * ROWO, *const sL = sM + 32;
+  const float l_tot = l_run + __shfl_xor(l_run, 32);
+  if (lh == 0) {
+    sM[lr] = m_run;
+    sL[lr] = l_tot;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+      *(float4 *)(sO + lr * ROWO + i * 32 + 8 * g + 4 * lh) =
+          make_float4(ot[i][4 * g], ot[i][4 * g + 1], ot[i][4 * g + 2], ot[i][4 * g + 3]);
+  __syncthreads();
+  constexpr int DPT = 32 * D / (64 * QW);  // outputs per thread: 4 or 8 of one query
+  const int mq = tid / (D / DPT), d0 = tid % (D / DPT) * DPT;
+  if (q0 + mq >= n) return;
+  float m = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < QW; w++) m = fmaxf(m, ((const float *)(smem + w * SLAB))[32 * ROWO + mq]);
+  float lsum = 0.0f, o[DPT];
+#pragma unroll
+  for (int d = 0; d < DPT; d++) o[d] = 0.0f;
+#pragma unroll
+  for (int w = 0; w < QW; w++) {
+    const float *pO = (const float *)(smem + w * SLAB);
+    const float mw = pO[32 * ROWO + mq];
+    // a wave without a unit (or whose units this query does not see): weight 0
+    const float al = mw == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((mw - m) * a.scale_log2);
+    lsum += pO[32 * ROWO + 32 + mq] * al;
+#pragma unroll
+    for (int d = 0; d < DPT; d += 4) {
+      const float4 v = *(const float4 *)(pO + mq * ROWO + d0 + d);
+      o[d] += v.x * al, o[d + 1] += v.y * al, o[d + 2] += v.z * al, o[d + 3] += v.w * al;
+    }
+  }
+  const float inv = 1.0f / lsum;
+  if (a.lse && d0 == 0) a.lse[(size_t)(base + q0 + mq) * a.heads + head] = m * a.scale_log2 + log2f(lsum);
+  T *out = (T *)a.ctx + (size_t)(base + q0 + mq) * H + head * D + d0;
+#pragma unroll
+  for (int d = 0; d < DPT; d += 4) {
+    if constexpr (sizeof(T) == 2)
+      *(uint2 *)(out + d) = make_uint2(pack16<T>(o[d] * inv, o[d + 1] * inv), pack16<T>(o[d + 2] * inv, o[d + 3] * inv));
+    else
+      *(float4 *)(out + d) = make_float4(o[d] * inv, o[d + 1] * inv, o[d + 2] * inv, o[d + 3] * inv);
   }
 }
 
@@ -1391,18 +1746,11 @@ hipError_t launch_attention_generic(int precision, const AttnArgs &a, hipStream_
 
 template <class T>
 void launch_attention_t(const AttnArgs &a, hipStream_t s) {
-  // fp32 launches of at most 256 (work item, head) pairs (the certification
-  // twin's few sequences, fp32 validation of small requests) leave most CUs
-  // idle: each work item runs as two workgroups of two waves (the same
-  // per-query arithmetic; one 512-token fp32 forward 3.81 -> 3.37 ms, bit-
-  // identical; one-wave parts measured the same).
-  if constexpr (std::is_same<T, float>::value) {
-    if (a.qt == ATTN_QT && a.nwork * a.heads <= 256) {
-      dim3 grid(a.nwork * a.heads * (ATTN_WAVES / 2)), block(128);
-      if (a.sliding) hipLaunchKernelGGL((attention_kernel<T, 2, ATTN_QT, true>), grid, block, 0, s, a);
-      else hipLaunchKernelGGL((attention_kernel<T, 2, ATTN_QT, false>), grid, block, 0, s, a);
-      return;
-    }
+  if (a.key_split) {
+    const dim3 grid(a.nwork * a.heads * ATTN_WAVES), block(512);
+    if (a.sliding) hipLaunchKernelGGL((attention_ks_kernel<T, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((attention_ks_kernel<T, false>), grid, block, 0, s, a);
+    return;
   }
   dim3 grid(a.nwork * a.heads), block(64 * ATTN_WAVES);
   if (a.sliding)
@@ -1427,6 +1775,7 @@ hipError_t launch_attention(int precision, const AttnArgs &a, hipStream_t s) {
   // Sliding-window layers take ATTN_QT; global layers ATTN_QT or (their
   // inference layout) ATTN_QT_GLOBAL.
   if (a.qt != ATTN_QT && (a.sliding || a.qt != ATTN_QT_GLOBAL)) return hipErrorInvalidValue;
+  if (a.key_split && a.qt != ATTN_QT) return hipErrorInvalidValue;
   if (precision == PREC_BF16) launch_attention_t<bf16>(a, s);
   else if (precision == PREC_F16) launch_attention_t<f16>(a, s);
   else launch_attention_t<float>(a, s);

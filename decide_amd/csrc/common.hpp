@@ -345,6 +345,7 @@ struct AttnArgs {
   float *lse;         // training: per (token, head) log2 of the softmax denominator of the
                       // scaled scores, lse[t*heads + head] = max*scale_log2 + log2(sum); null otherwise
   int qt;                       // query tiles per wave of the work items (ATTN_QT or ATTN_QT_GLOBAL)
+  int key_split;                // few work items: each 32-query chunk's keys split over a workgroup's waves
   int nseq, max_len, head_dim;  // the any-geometry kernel: sequences, longest one, head width,
   float scale;                  // and the softmax scale float32(1 / sqrt(head_dim))
   // Option-row attention (launch_attention_rows): work items and slots from

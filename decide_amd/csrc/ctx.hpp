@@ -93,6 +93,10 @@ struct TrainState {
 // the parts into the residual stream.
 constexpr int kSmallSplitMaxTokens = 128, kSmallSplitParts = 6, kSplitMaxWorkgroups = 256;
 
+// Batches of at most this many 128-query work items split the attention's keys
+// over waves (attention_ks_kernel, with the measurements at 12 heads).
+constexpr int kKeySplitItems16 = 8, kKeySplitItems32 = 16;
+
 // Device memory one forward works in beyond the weights: the activations,
 // the batch layout and the head's scratch. forward_core takes it from the
 // context's own buffers unless a caller hands one in

@@ -114,3 +114,21 @@ def test_folded_small_batch_matches_oracle(base_small, total):
             assert np.array_equal(engs[prec].forward(batch), got) == (total <= 1024)
         finally:
             engs[prec].set_ln_fold(True)
+
+
+@pytest.mark.parametrize("prec,lens", [("bf16", (31,)), ("fp32", (32, 33)), ("bf16", (257, 225, 30)),
+                                       ("fp16", (1024,)), ("bf16", (1025,)), ("fp32", (2048,)), ("fp32", (2049,))])
+def test_key_split_attention_matches_oracle(base_small, prec, lens):
+    """Attention with each query chunk's keys split over a workgroup's waves:
+    sequences of one unit (32 keys), ragged last units and chunks, more units
+    than waves, and both sides of the item limits (1,024 tokens in 16 bits, 2,048
+    in fp32). Independent options and plain sequences."""
+    from decide_amd.nn import build_sequence
+    from decide_amd.synth import MASK_ID, pack_request
+
+    cfg, orc, engs = base_small
+    rng = np.random.default_rng(sum(lens))
+    batch = [build_sequence(pack_request(rng, n - 3 * 5, [5] * 3, cfg.vocab), MASK_ID, independent=i % 2 == 0)
+             for i, n in enumerate(lens)]
+    oracle.set_workers(WORKERS)
+    compare(engs[prec].forward(batch), orc.forward(batch), batch, prec)
