@@ -412,6 +412,7 @@ struct Pass {
   // Attention with the keys split over waves (attn_key_split), by the whole
   // batch too.
   bool key_split = false;
+  int rows = 0;  // the whole batch's tokens
   Workspace w;
   const int32_t *ids, *pos, *opt;
   hipStream_t s;
@@ -528,6 +529,7 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
   q.N = 3 * H;
   q.K = H;
   q.n_store = 3 * H;
+  q.rows = p.rows;
   LnFold qf{};
   if (fold_in) {
     qf.lpart = attn_part;
@@ -589,6 +591,7 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
   o.K = H;
   o.n_store = H;
   o.accumulate = 1;
+  o.rows = p.rows;
   void *x2 = S ? S->n2.p : w.xn;
   // The row value the folded mlp_norm's operand is taken relative to: this
   // layer's attn_norm means when its QKV folded too (0 otherwise).
@@ -622,6 +625,7 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
   wi.N = 2 * I;
   wi.K = H;
   wi.n_store = 2 * I;
+  wi.rows = p.rows;
   if (S) {  // training keeps the pre-activation as well as the GeGLU output
     wi.C = S->wi.p;
     wi.ldc = 2 * I;
@@ -656,6 +660,7 @@ int enqueue_layer(dn_ctx *c, const Pass &p, int l, float *in, float *h1, float *
   mo.K = I;
   mo.n_store = H;
   mo.accumulate = 1;
+  mo.rows = p.rows;
   const int parts = split && mo_parts ? small_split_parts(prec, T, H, I) : 1;
   if (mo_parts) *mo_parts = parts > 1 ? parts : 0;
   mo.skinny_regs = g.skinny_regs ? 1 : 0;
@@ -1047,6 +1052,7 @@ int forward_split(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_
   const bool key_split = attn_key_split(g, ps[0].w.nwork + ps[1].w.nwork);
   for (Pass &p : ps) {
     p.key_split = key_split;
+    p.rows = T_total;
     p.wide_global = !key_split;
   }
   for (Pass &p : ps) {
@@ -1156,7 +1162,10 @@ int forward_core(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_i
   ps.s = c->stream;
   ps.fold = !train && w.lmean1 && fold_eligible(c, T);
   ps.ln_cols = T <= kLnNarrowTokens ? kLnPartNarrow : kLnPartWide;
-  ps.key_split = attn_key_split(g, w.nwork);
+  // Training keeps the tile walk in bf16: its gradients cancel over a
+  // question's options, so another order of attention's sums, rounded to
+  // bf16, moves them by as much as their own error (5% at a few examples).
+  ps.key_split = !(train && prec16(g.precision)) && attn_key_split(g, w.nwork);
   if (ps.fold) {
     rc = ensure_fold_cs(c, ps.s);
     if (rc) return rc;

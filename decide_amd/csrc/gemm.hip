@@ -85,6 +85,26 @@ __device__ __forceinline__ void lds_read8x16(const char *const (&p)[8], uint4 (&
   o[6] = __builtin_bit_cast(uint4, v6), o[7] = __builtin_bit_cast(uint4, v7);
 }
 
+// The same with four reads.
+__device__ __forceinline__ void lds_read4x16(const char *const (&p)[4], uint4 (&o)[4]) {
+  typedef int i32x4 __attribute__((ext_vector_type(4)));
+  uint32_t a[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) a[i] = (uint32_t)(size_t)(const __attribute__((address_space(3))) char *)p[i];
+  i32x4 v0, v1, v2, v3;
+  asm volatile(
+      "ds_read_b128 %0, %4\n\t"
+      "ds_read_b128 %1, %5\n\t"
+      "ds_read_b128 %2, %6\n\t"
+      "ds_read_b128 %3, %7\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3])
+      : "memory");
+  o[0] = __builtin_bit_cast(uint4, v0), o[1] = __builtin_bit_cast(uint4, v1);
+  o[2] = __builtin_bit_cast(uint4, v2), o[3] = __builtin_bit_cast(uint4, v3);
+}
+
 // Workgroup -> tile: XCD x (workgroup ids congruent to x mod 8) takes the x-th
 // of eight contiguous ranges of the row-ordered tiles, for any tile count.
 // Row order over all workgroups, which ragged row counts took before, spread
@@ -821,15 +841,20 @@ __global__ __launch_bounds__(64 * W) void gemm_skinny_kernel(GemmArgs g) {
   using MF = Mfma<T>;
   typedef typename MF::frag frag;
   static_assert(!F16 || sizeof(T) == 2, "16 x 16 blocks: 16-bit operands");
-  static_assert(!DMA || (F16 && MB == 1 && NB == 1 && W == 8), "LDS operand path: 16-bit 32 x 32 tiles, 8 waves");
-  // DMA: each wave stages its K groups through a private two-slot LDS slab.
+  static_assert(!DMA || (W == 8 && (sizeof(T) == 4 || (F16 && MB == 1 && NB == 1))),
+                "LDS operand path: 8 waves, fp32 or 16-bit 32 x 32 tiles");
+  // DMA: each wave stages its K groups through a private LDS slab of two
+  // slots, in fp32 one (a group's 16 MFMAs of 64 cycles cover the next one's
+  // arrival, and at 64 KB two workgroups share a CU).
   // A group's 32 A rows and 32 B rows (128 bytes each) arrive by eight
   // wave-wide global->LDS loads, lane l carrying 16 bytes of row 8j + l/8, so
   // every row is read as one whole 128-byte segment (the register path's
   // lanes read 64-byte pieces of 16 rows per instruction); the fragments are
   // then read from LDS in the same layout the register path loads them in,
   // so both paths feed the MFMAs the same operands in the same order.
-  constexpr int SLAB = 64 * 128;  // bytes of one group (64 rows x 128 bytes)
+  constexpr int TR = 32 * MB, TC = 32 * NB, TE = TR * TC;
+  constexpr int SLAB = (TR + TC) * 128;  // bytes of one group (its rows x 128 bytes)
+  constexpr int SLOTS = sizeof(T) == 2 ? 2 : 1;
   // F16: the tile as 16 x 16 blocks of the 16 x 16 x 32 MFMA, whose operand
   // lanes read 64 contiguous bytes of a row (four lanes x 16 bytes) where the
   // 32 x 32 x 16 form reads 32 (two lanes): half the cache-line sectors per
@@ -842,7 +867,6 @@ __global__ __launch_bounds__(64 * W) void gemm_skinny_kernel(GemmArgs g) {
   constexpr int NT = 64 * W;
   constexpr int VPL = 16 / (int)sizeof(T);  // elements per 16-byte load
   constexpr int GK = 8 * VPL;               // k elements per group
-  constexpr int TR = 32 * MB, TC = 32 * NB, TE = TR * TC;
   static_assert(EPI != EPI_GEGLU_KEEP || NB == 2, "the kept pre-activation tile is 32 value + 32 gate columns");
   static_assert(EPI != EPI_GEGLU || NB <= 2, "GeGLU tiles");
   static_assert(W == 4 || W == 8, "wave count");
@@ -853,8 +877,8 @@ __global__ __launch_bounds__(64 * W) void gemm_skinny_kernel(GemmArgs g) {
   // thread one item; NQ items per thread.
   constexpr int FV = TE <= 2 * NT ? 2 : 4, TEV = TE / FV, NQ = (TEV + NT - 1) / NT;
   // The partial tiles; in DMA mode the same memory first holds the waves'
-  // slabs (W x 2 groups), and a barrier separates the two uses.
-  constexpr int RED = DMA && W * 2 * SLAB / 4 > NP * TE ? W * 2 * SLAB / 4 : NP * TE;
+  // slabs (W x SLOTS groups), and a barrier separates the two uses.
+  constexpr int RED = DMA && W * SLOTS * SLAB / 4 > NP * TE ? W * SLOTS * SLAB / 4 : NP * TE;
   __shared__ __attribute__((aligned(1024))) float red[RED];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 31, lh = lane >> 5;
@@ -904,109 +928,8 @@ __global__ __launch_bounds__(64 * W) void gemm_skinny_kernel(GemmArgs g) {
         XB[j][q] = *(const uint4 *)(bp[j] + k_ + (GK / NS) * q);                                   \
   } while (0)
 
-  const int ngrp = g.K / GK;
-  uint4 la[RB][NS], lb[CB][NS];
-  int grp = wave;
-  if (!DMA && grp < ngrp) SKINNY_LOAD(la, lb, grp);
-  // The fp32 epilogue's residual input, loaded now (behind the first operand
-  // group) so its latency overlaps the main loop instead of following the
-  // reduction; each element is read and then written by this thread only.
-  fvec<FV> pre[NQ];
-  const bool vec = (g.ldc & (FV - 1)) == 0;
-  if constexpr (EPI == EPI_F32) {
-    const float *R = g.res ? g.res : (const float *)g.C;
-#pragma unroll
-    for (int k = 0; k < NQ; k++) {
-      pre[k] = 0.0f;
-      const int q = tid + NT * k;
-      const int r = q / (TC / FV), col = n0 + (q % (TC / FV)) * FV;
-      if (g.accumulate && vec && q < TEV && m0 + r < g.M && col + FV <= g.n_store)
-        pre[k] = *(const fvec<FV> *)(R + (size_t)(m0 + r) * g.ldc + col);
-    }
-  }
-  if constexpr (DMA) {
-    // Slab row r < 32 is A row m0 + r, r >= 32 the B row of tile column
-    // r - 32 (the mapping of bp above). DMA load j of a group fills slab
-    // rows 8j .. 8j+7; lane l brings the 16-byte chunk (l % 8) ^ swz(row) of
-    // row 8j + l / 8 into LDS slot l % 8 of that row, so a row's logical
-    // chunk c sits in slot c ^ swz(row) (the XOR swizzle spreads the 16 rows
-    // a quarter-wave reads over distinct banks).
-    const int wv = __builtin_amdgcn_readfirstlane(wave);
-    const char *dsrc[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int r = 8 * j + (lane >> 3);
-      const int c = (lane & 7) ^ swz<128>(r);
-      const T *row;
-      if (r < 32) {
-        row = (const T *)g.A + (size_t)min(m0 + r, g.M - 1) * g.lda;
-      } else {
-        const int cc = r - 32;
-        const int br = EPI == EPI_GEGLU ? (n0 & ~63) + (cc < 16 ? 0 : 32) + ((n0 >> 5) & 1) * 16 + (cc & 15) : n0 + cc;
-        row = (const T *)g.B + (size_t)br * g.ldb;
-      }
-      dsrc[j] = (const char *)(row + kz) + c * 16;
-    }
-    // The LDS reads are opaque to the compiler (lds_read8x16), so it adds no
-    // waits of its own for the DMA: the vmcnt waits below are the only ones.
-    auto issue = [&](int gi, int slot) {
-      char *dst = (char *)red + (wv * 2 + slot) * SLAB;
-      const size_t kb = (size_t)gi * GK * sizeof(T);
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        __builtin_amdgcn_global_load_lds((gbl_void *)(dsrc[j] + kb), (lds_void *)(dst + j * 1024), 16, 0, 0);
-    };
-    // This wave's groups: wv, wv + W, ... (the register path's order).
-    const int myn = wv < ngrp ? (ngrp - 1 - wv) / W + 1 : 0;
-    if (myn > 0) issue(wv, 0);
-    if (myn > 1) issue(wv + W, 1);
-    for (int i = 0; i < myn; i++) {
-      // Group i has landed once at most the next group's eight loads are
-      // outstanding (the residual loads above are older and count as done).
-      if (i + 1 < myn) wait_vmcnt<8>();
-      else wait_vmcnt<0>();
-      const char *sl = (const char *)red + (wv * 2 + (i & 1)) * SLAB;
-      const char *fp[8];
-      uint4 fr[8];
-#pragma unroll
-      for (int q = 0; q < NS; q++) {
-        const int c = (lane >> 4) + 4 * q;  // the register path's k chunk for this lane
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-          const int ra = 16 * b + (lane & 15), rb = 32 + ra;
-          fp[4 * q + b] = sl + ra * 128 + ((c ^ swz<128>(ra)) << 4);
-          fp[4 * q + 2 + b] = sl + rb * 128 + ((c ^ swz<128>(rb)) << 4);
-        }
-      }
-      // The fragments are in registers when this returns: the MFMAs may use
-      // them and the slot can be refilled with group i + 2.
-      lds_read8x16(fp, fr);
-#pragma unroll
-      for (int q = 0; q < NS; q++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-          la[b][q] = fr[4 * q + b];
-          lb[b][q] = fr[4 * q + 2 + b];
-        }
-      if (i + 2 < myn) issue(wv + (i + 2) * W, i & 1);
-#pragma unroll
-      for (int q = 0; q < NS; q++)
-#pragma unroll
-        for (int a = 0; a < RB; a++)
-#pragma unroll
-          for (int b = 0; b < CB; b++)
-            acc[a][b] = mma16x16<T>(__builtin_bit_cast(frag, la[a][q]), __builtin_bit_cast(frag, lb[b][q]), acc[a][b]);
-    }
-    // Every load has landed and every wave is done with its slab before the
-    // partial tiles reuse the memory.
-    wait_vmcnt<0>();
-    __syncthreads();
-    grp = ngrp;  // the register loop below does nothing
-  }
-  for (; grp < ngrp; grp += W) {
-    uint4 na[RB][NS], nb[CB][NS];
-    const bool more = grp + W < ngrp;
-    if (more) SKINNY_LOAD(na, nb, grp + W);
+  // One K group's MFMAs.
+  auto mfma_group = [&](const uint4 (&la)[RB][NS], const uint4 (&lb)[CB][NS]) {
 #pragma unroll
     for (int q = 0; q < NS; q++) {
       if constexpr (F16) {
@@ -1035,6 +958,129 @@ __global__ __launch_bounds__(64 * W) void gemm_skinny_kernel(GemmArgs g) {
             }
       }
     }
+  };
+
+  const int ngrp = g.K / GK;
+  uint4 la[RB][NS], lb[CB][NS];
+  int grp = wave;
+  if (!DMA && grp < ngrp) SKINNY_LOAD(la, lb, grp);
+  // The fp32 epilogue's residual input, loaded now (behind the first operand
+  // group) so its latency overlaps the main loop instead of following the
+  // reduction; each element is read and then written by this thread only.
+  fvec<FV> pre[NQ];
+  const bool vec = (g.ldc & (FV - 1)) == 0;
+  if constexpr (EPI == EPI_F32) {
+    const float *R = g.res ? g.res : (const float *)g.C;
+#pragma unroll
+    for (int k = 0; k < NQ; k++) {
+      pre[k] = 0.0f;
+      const int q = tid + NT * k;
+      const int r = q / (TC / FV), col = n0 + (q % (TC / FV)) * FV;
+      if (g.accumulate && vec && q < TEV && m0 + r < g.M && col + FV <= g.n_store)
+        pre[k] = *(const fvec<FV> *)(R + (size_t)(m0 + r) * g.ldc + col);
+    }
+  }
+  if constexpr (DMA) {
+    // Slab row r < TR is A row m0 + r, r >= TR the B row of tile column
+    // r - TR (the mapping of bp above). DMA load j of a group fills slab
+    // rows 8j .. 8j+7; lane l brings the 16-byte chunk (l % 8) ^ swz(row) of
+    // row 8j + l / 8 into LDS slot l % 8 of that row, so a row's logical
+    // chunk c sits in slot c ^ swz(row) (the XOR swizzle spreads the 16 rows
+    // a quarter-wave reads over distinct banks).
+    constexpr int LPG = (TR + TC) / 8;  // loads per group
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    const char *dsrc[LPG];
+#pragma unroll
+    for (int j = 0; j < LPG; j++) {
+      const int r = 8 * j + (lane >> 3);
+      const int c = (lane & 7) ^ swz<128>(r);
+      const T *row;
+      if (r < TR) {
+        row = (const T *)g.A + (size_t)min(m0 + r, g.M - 1) * g.lda;
+      } else {
+        const int cc = r - TR;
+        const int br = (EPI == EPI_GEGLU && NB == 1)
+                           ? (n0 & ~63) + (cc < 16 ? 0 : 32) + ((n0 >> 5) & 1) * 16 + (cc & 15)
+                           : n0 + cc;
+        row = (const T *)g.B + (size_t)br * g.ldb;
+      }
+      dsrc[j] = (const char *)(row + kz) + c * 16;
+    }
+    // The LDS reads are opaque to the compiler (lds_read8x16 / 4x16), so it
+    // adds no waits of its own for the DMA: the vmcnt waits below are the only
+    // ones.
+    auto issue = [&](int gi, int slot) {
+      char *dst = (char *)red + (wv * SLOTS + slot) * SLAB;
+      const size_t kb = (size_t)gi * GK * sizeof(T);
+#pragma unroll
+      for (int j = 0; j < LPG; j++)
+        __builtin_amdgcn_global_load_lds((gbl_void *)(dsrc[j] + kb), (lds_void *)(dst + j * 1024), 16, 0, 0);
+    };
+    // This wave's groups: wv, wv + W, ... (the register path's order).
+    const int myn = wv < ngrp ? (ngrp - 1 - wv) / W + 1 : 0;
+#pragma unroll
+    for (int i = 0; i < SLOTS; i++)
+      if (myn > i) issue(wv + i * W, i);
+    for (int i = 0; i < myn; i++) {
+      // Group i has landed once at most the next group's eight loads are
+      // outstanding (the residual loads above are older and count as done).
+      if (SLOTS == 2 && i + 1 < myn) wait_vmcnt<LPG>();
+      else wait_vmcnt<0>();
+      const char *sl = (const char *)red + (wv * SLOTS + i % SLOTS) * SLAB;
+      // The register path's rows and k chunks for this lane. When the reads
+      // return the fragments are in registers: the MFMAs may use them and the
+      // slot can be refilled with group i + SLOTS.
+      if constexpr (F16) {
+        const char *fp[8];
+        uint4 fr[8];
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+          const int c = (lane >> 4) + 4 * q;
+#pragma unroll
+          for (int b = 0; b < 2; b++) {
+            const int ra = 16 * b + (lane & 15), rb = 32 + ra;
+            fp[4 * q + b] = sl + ra * 128 + ((c ^ swz<128>(ra)) << 4);
+            fp[4 * q + 2 + b] = sl + rb * 128 + ((c ^ swz<128>(rb)) << 4);
+          }
+        }
+        lds_read8x16(fp, fr);
+#pragma unroll
+        for (int q = 0; q < NS; q++)
+#pragma unroll
+          for (int b = 0; b < 2; b++) {
+            la[b][q] = fr[4 * q + b];
+            lb[b][q] = fr[4 * q + 2 + b];
+          }
+      } else {
+#pragma unroll
+        for (int b = 0; b < MB + NB; b++) {
+          const int r = 32 * b + lr;
+          const char *fp[4];
+          uint4 fr[4];
+#pragma unroll
+          for (int q = 0; q < 4; q++) fp[q] = sl + r * 128 + (((lh + 2 * q) ^ swz<128>(r)) << 4);
+          lds_read4x16(fp, fr);
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            if (b < MB) la[b < MB ? b : 0][q] = fr[q];
+            else lb[b < MB ? 0 : b - MB][q] = fr[q];
+          }
+        }
+      }
+      if (i + SLOTS < myn) issue(wv + (i + SLOTS) * W, i % SLOTS);
+      mfma_group(la, lb);
+    }
+    // Every load has landed and every wave is done with its slab before the
+    // partial tiles reuse the memory.
+    wait_vmcnt<0>();
+    __syncthreads();
+    grp = ngrp;  // the register loop below does nothing
+  }
+  for (; grp < ngrp; grp += W) {
+    uint4 na[RB][NS], nb[CB][NS];
+    const bool more = grp + W < ngrp;
+    if (more) SKINNY_LOAD(na, nb, grp + W);
+    mfma_group(la, lb);
     if (more) {
 #pragma unroll
       for (int i = 0; i < RB; i++)
@@ -1165,33 +1211,38 @@ __global__ __launch_bounds__(64 * W) void gemm_skinny_kernel(GemmArgs g) {
 template <class T, int MB, int NB, int W>
 hipError_t launch_skinny_cfg(int epi, const GemmArgs &a, hipStream_t s, int splits = 1) {
   constexpr bool F = sizeof(T) == 2 && MB == 1 && NB == 1;
-  constexpr bool D = F && W == 8;  // the LDS operand path exists for these tiles
+  // The LDS operand path exists for these tiles.
+  constexpr bool D = W == 8 && (std::is_same<T, float>::value || (MB == 1 && NB == 1));
   dim3 grid(a.N / (32 * NB), (a.M + 32 * MB - 1) / (32 * MB), splits), block(64 * W);
-  const bool dma = D && !a.skinny_regs;
-#define SKINNY_LAUNCH(E)                                                                        \
-  do {                                                                                          \
-    if (dma)                                                                                    \
-      hipLaunchKernelGGL((gemm_skinny_kernel<T, MB, NB, E, W, F, D>), grid, block, 0, s, a);   \
-    else                                                                                        \
-      hipLaunchKernelGGL((gemm_skinny_kernel<T, MB, NB, E, W, F>), grid, block, 0, s, a);      \
-  } while (0)
+  auto go = [&](auto e) {
+    constexpr int E = decltype(e)::value;
+    if constexpr (D && std::is_same<T, float>::value) {
+      hipLaunchKernelGGL((gemm_skinny_kernel<T, MB, NB, E, W, F, true>), grid, block, 0, s, a);
+    } else if constexpr (D) {
+      if (a.skinny_regs) hipLaunchKernelGGL((gemm_skinny_kernel<T, MB, NB, E, W, F>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((gemm_skinny_kernel<T, MB, NB, E, W, F, true>), grid, block, 0, s, a);
+    } else {
+      hipLaunchKernelGGL((gemm_skinny_kernel<T, MB, NB, E, W, F>), grid, block, 0, s, a);
+    }
+  };
   switch (epi) {
     case EPI_F32:
-      SKINNY_LAUNCH(EPI_F32);
+      if constexpr (NB == 1 || std::is_same<T, float>::value) go(std::integral_constant<int, EPI_F32>{});
+      else return hipErrorInvalidValue;
       break;
     case EPI_STORE:
-      SKINNY_LAUNCH(EPI_STORE);
+      if constexpr (NB == 1 || std::is_same<T, float>::value) go(std::integral_constant<int, EPI_STORE>{});
+      else return hipErrorInvalidValue;
       break;
     case EPI_GEGLU:
-      SKINNY_LAUNCH(EPI_GEGLU);
+      if constexpr (MB == 1 || std::is_same<T, float>::value) go(std::integral_constant<int, EPI_GEGLU>{});
+      else return hipErrorInvalidValue;
       break;
     default:
-      if constexpr (NB == 2 && !std::is_same<T, f16>::value)
-        hipLaunchKernelGGL((gemm_skinny_kernel<T, MB, 2, EPI_GEGLU_KEEP, W, F>), grid, block, 0, s, a);
+      if constexpr (NB == 2 && !std::is_same<T, f16>::value) go(std::integral_constant<int, EPI_GEGLU_KEEP>{});
       else return hipErrorInvalidValue;
       break;
   }
-#undef SKINNY_LAUNCH
   return hipGetLastError();
 }
 
@@ -1199,32 +1250,42 @@ hipError_t launch_skinny_cfg(int epi, const GemmArgs &a, hipStream_t s, int spli
 // workgroup per CU (more workgroups for the few rows: cfg5 1.10 -> 0.92 ms,
 // cfg2 1.18 -> 1.06 ms against 64-row tiles everywhere), 64-row tiles
 // otherwise; 32 columns, or for GeGLU 32 (16 value + 16 gate rows) or 64
-// (32 + 32; training's kept pre-activation always).
+// (32 + 32; training's kept pre-activation always). fp32: 32 x 32 at any row
+// count, operands through LDS.
 template <class T>
 hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
-  if (epi == EPI_GEGLU || epi == EPI_GEGLU_KEEP) {
-    // Inference GeGLU on 32-column tiles (16 outputs each) while their grid
-    // fits one workgroup per CU (MI355X: 256): twice the workgroups of the
-    // 64-column tiles, a third less operand traffic per workgroup (cfg5
-    // 0.809 -> 0.789 ms; at 112 rows, 288 workgroups, 0.932 -> 0.951 ms).
-    if (a.M <= 128 && epi == EPI_GEGLU && (a.N / 32) * ((a.M + 31) / 32) <= 256)
-      return launch_skinny_cfg<T, 1, 1, 8>(epi, a, s);
+  constexpr bool f32 = std::is_same<T, float>::value;
+  if (epi == EPI_GEGLU_KEEP) {
     if (a.M <= 128) return launch_skinny_cfg<T, 1, 2, 8>(epi, a, s);
-    // fp32 inference GeGLU above 128 rows also on 32-row tiles (one 512-token
-    // fp32 forward 3.92 -> 3.80 ms against 64 x 64, bit-identical).
-    if (std::is_same<T, float>::value && epi == EPI_GEGLU) return launch_skinny_cfg<T, 1, 2, 8>(epi, a, s);
     return launch_skinny_cfg<T, 2, 2, 8>(epi, a, s);
   }
-  // 32-row tiles while their grid fits one workgroup per CU, else 64-row
-  // tiles (QKV at 112 rows: 288 -> 144 workgroups, cfg2 0.917 -> 0.901 ms).
-  if (a.M <= 128 && (a.N / 32) * ((a.M + 31) / 32) <= 256) return launch_skinny_cfg<T, 1, 1, 8>(epi, a, s);
-  // fp32 above 128 rows (the validation GEMM, the certification twin's
-  // forward): 32 x 32 tiles for outputs of 2048 columns or more, two
-  // workgroups per CU (512 x 2304 x 768: 39.6 -> 33.5 us; 1024 rows: 64.1 ->
-  // 55.6 us; bit-identical, the same K split over eight waves); the 768-wide
-  // outputs keep 64-row tiles (their 32 x 32 grid: 14.2 -> 15.4 us).
-  if (std::is_same<T, float>::value && a.M > 128 && a.N >= 2048) return launch_skinny_cfg<T, 1, 1, 8>(epi, a, s);
-  return launch_skinny_cfg<T, 2, 1, 8>(epi, a, s);
+  // 32 x 32 tiles while their grid fits one workgroup per CU (MI355X: 256):
+  // QKV at 112 rows as 144 workgroups of 64 rows instead of 288 took cfg2 0.917
+  // -> 0.901 ms, GeGLU on 32-column tiles there 0.932 -> 0.951 ms (cfg5 0.809
+  // -> 0.789 ms).
+  if constexpr (f32) {
+    // A CU's time is its 32 x 32 blocks of the busiest round; 32 x 64 tiles
+    // read a third less for the same blocks, so they are taken where they do
+    // not add any (K = 768, N = 2304, us, 32 x 32 / 32 x 64 / the register
+    // path: 203 rows 15.3 / 13.7 / 15.7, 300 rows 20.8 / 22.7 / 20.8, 512 rows
+    // 29.5 / 31.2 / 30.7; N = 768: 203 rows 7.4 / 12.0 / 13.2, 512 rows 13.8 /
+    // 12.2 / 13.6, 1,472 rows 28.8 / 32.2 / 101.7 on 256 x 128 tiles). Longer K
+    // at two blocks a CU keeps the register path (512 x 768 x 1152: 20.5 / 19.6 /
+    // 17.5).
+    const int c32 = (a.N / 32) * ((a.M + 31) / 32), c64 = c32 / 2;
+    const int r32 = (c32 + kCUs - 1) / kCUs, r64 = (c64 + kCUs - 1) / kCUs;
+    if (r32 == 2 && a.K > 768 && epi == EPI_F32) {
+      hipLaunchKernelGGL((gemm_skinny_kernel<float, 2, 1, EPI_F32, 8>), dim3(a.N / 32, (a.M + 63) / 64), dim3(512), 0, s, a);
+      return hipGetLastError();
+    }
+    if (2 * r64 <= r32) return launch_skinny_cfg<T, 1, 2, 8>(epi, a, s);
+  }
+  if (f32 || (a.N / 32) * ((a.M + 31) / 32) <= 256) return launch_skinny_cfg<T, 1, 1, 8>(epi, a, s);
+  if constexpr (!f32) {
+    if (epi == EPI_GEGLU) return launch_skinny_cfg<T, 1, 2, 8>(epi, a, s);
+    return launch_skinny_cfg<T, 2, 1, 8>(epi, a, s);
+  }
+  return hipErrorInvalidValue;
 }
 
 // Small-M split-K: a workgroup's time grows with the K it streams (~3.4 ns
@@ -1473,6 +1534,22 @@ hipError_t launch_gemm16(int epi, const GemmArgs &a, hipStream_t s, const LnFold
   return hipErrorInvalidValue;
 }
 
+// fp32 on the whole-K kernel (32 x 32 tiles, K split over eight waves, also
+// the smaller summation error: 1.8e-7 of the result against 5e-7) or on 256 x
+// 128 tiles, of which a round takes about as long as 20 rounds of 32 x 32 ones
+// on the 256 CUs (K = 768, N = 2304: 1,472 rows 70 against 104 us, 2,048 rows
+// 95 / 105, 3,000 rows 135 / 105, 4,000 rows 178 / 205; N = 768, 4,000 rows 64 /
+// 104). The two sum in different orders, so the parts of a two-stream forward
+// choose by the whole batch's rows.
+bool f32_small_tiles(int epi, const GemmArgs &a) {
+  if (epi == EPI_GEGLU_BWD) return false;
+  if (epi == EPI_GEGLU_KEEP) return a.M <= 1024;
+  const long long M = a.rows ? a.rows : a.M;
+  const long long r32 = ((M + 31) / 32 * (a.N / 32) + kCUs - 1) / kCUs;
+  const long long rt = ((M + 255) / 256 * (a.N / 128) + kCUs - 1) / kCUs;
+  return M <= 1024 || r32 <= 20 * rt;
+}
+
 template <class C>
 hipError_t launch_gemm_f32_tile(int epi, const GemmArgs &a, hipStream_t s) {
   switch (epi) {
@@ -1488,16 +1565,13 @@ hipError_t launch_gemm_f32_tile(int epi, const GemmArgs &a, hipStream_t s) {
 hipError_t launch_gemm(int precision, int epi, const GemmArgs &a, hipStream_t s, const LnFold *ln) {
   if (a.M <= 0) return hipSuccess;
   if (!gemm_epi_ok(precision, epi, a.M) || (epi == EPI_GEGLU_BWD && (!a.gin || a.ldc % 8))) return hipErrorInvalidValue;
-  // Small M goes to the whole-K kernel (grid: N/32 x M/64 workgroups). In
-  // fp32 (the scorer's dense layer over all [MASK] rows, the fp32 validation
-  // build) that pays up to M = 1024: the 64 x 128 tiles below would leave
-  // most CUs idle with a 24-step fp32 K loop each.
+  // Small M goes to the whole-K kernel.
   if (a.M <= 128)
     return precision == PREC_BF16  ? launch_skinny<bf16>(epi, a, s)
            : precision == PREC_F16 ? launch_skinny<f16>(epi, a, s)
                                    : launch_skinny<float>(epi, a, s);
   if (precision == PREC_BF16) return launch_gemm16<bf16>(epi, a, s, ln);
   if (precision == PREC_F16) return launch_gemm16<f16>(epi, a, s, ln);
-  if (a.M <= 1024) return launch_skinny<float>(epi, a, s);
+  if (f32_small_tiles(epi, a)) return launch_skinny<float>(epi, a, s);
   return launch_gemm_f32_tile<Tile<256, 128, 128, 3, 1, 2, 2>>(epi, a, s);
 }

@@ -193,6 +193,29 @@ def test_gemm_tile_boundaries(eng, prec, M, N, K, store):
     assert bool((dC[M] == 7.0).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(129, 2304, 32), (203, 2304, 768), (340, 768, 768), (352, 768, 768),
+                                   (512, 768, 1152), (1025, 768, 1152), (1500, 128, 96), (2049, 2304, 768),
+                                   (3000, 2304, 768)])
+def test_gemm_f32_device_tiles(eng, M, N, K):
+    """fp32 operands on both sides of the fp32 tile rules (32 x 32 and 32 x 64
+    through LDS, 64 x 32 through registers, 256 x 128): against float64 at the
+    fp32 bound, rows past M untouched, and accumulation into C."""
+    import torch
+
+    g = torch.Generator().manual_seed(M + K)
+    dA = torch.randn(M, K, generator=g).cuda()
+    dB = (torch.randn(N, K, generator=g) * 0.02).cuda()
+    dC = torch.full((M + 1, N), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    exact, bound = dA.double() @ dB.double().T, 1e-5 * (dA.double().abs() @ dB.double().abs().T)
+    eng.gemm_device("fp32", M, N, K, dA.data_ptr(), dB.data_ptr(), dC.data_ptr())
+    eng.synchronize()
+    assert bool(((dC[:M].double() - exact).abs() <= bound).all()) and bool((dC[M] == 7.0).all())
+    eng.gemm_device("fp32", M, N, K, dA.data_ptr(), dB.data_ptr(), dC.data_ptr(), accumulate=True)
+    eng.synchronize()
+    assert bool(((dC[:M].double() - 2 * exact).abs() <= 3 * bound).all()) and bool((dC[M] == 7.0).all())
+
+
 @pytest.mark.parametrize("prec", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("M,N,K", [(1, 2304, 768), (31, 768, 1152), (33, 384, 768), (64, 2304, 768),
                                    (65, 768, 768), (112, 768, 1152), (128, 2304, 64), (100, 128, 4096)])
