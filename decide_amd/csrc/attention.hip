@@ -26,8 +26,13 @@
 // Key tiles (64 keys) are visited in a list of the tiles some wave needs; the
 // next tile's K, V and RoPE factors are loaded into registers while the
 // current one is computed. K is rotated and stored key-major; V is stored
-// transposed (d-major) with two keys packed per 32-bit word so each wave's
-// LDS writes are contiguous.
+// transposed (d-major) with two keys packed per 32-bit word, its rows' chunks
+// swizzled. Q, K and V are all read whole rows at a time: eight lanes to a
+// row's 128 bytes, since the CU's address unit takes about a cycle per line a
+// load instruction touches (Q by MFMA fragment and V by key before: 64 x 512
+// tokens sliding-window layers 78.8 -> 69.5 us, 8 x ~2,800 tokens 69.5 -> 61.7;
+// global layers, bound by the softmax, 110 -> 108.5 and 249 -> 256 us; the
+// same values and sums).
 #include "common.hpp"
 
 namespace {
@@ -68,6 +73,11 @@ struct Staging<float, R> {
   uint32_t valid;  // bit j: K item j's key, 8+j: V item j's key exists (zeroed at the store)
   int info;
 };
+
+// The 16-byte chunk of V^T row d (64 keys of 16 bits, 128-byte rows) that holds
+// logical chunk c: the eight lanes that store one key pair's rows 8g .. 8g + 7
+// and the lanes that read 32 rows' equal chunks fall on distinct banks.
+__device__ __forceinline__ int vt_chunk(int d, int c) { return c ^ (((d >> 3) ^ d) & 7); }
 
 // ok ? v : 0, per component (a select of the whole vector can end up as an
 // indexed scratch access).
@@ -132,8 +142,8 @@ __device__ __forceinline__ void stage_load(Staging<T, R> &st, const T *qkv, int 
       st.s_hi[j] = *(const float4 *)(sin_t + p * 32 + 8 * c + 4);
     }
 #pragma unroll
-    for (int j = 0; j < R; j++) {  // V: key pair p = it % 32, d group g = it / 32
-      const int it = tid + NT * j, p = it & 31, g = it >> 5;
+    for (int j = 0; j < R; j++) {  // V: key pair p = it / 8, d group g = it % 8: eight lanes read a whole row
+      const int it = tid + NT * j, p = it >> 3, g = it & 7;
       const int k = k0 + 2 * p;
       st.v0[j] = *(const uint4 *)(qkv + (size_t)(unsigned)(base + min(k, n - 1)) * (unsigned)ld + 2 * H + head * D + 8 * g);
       st.v1[j] = *(const uint4 *)(qkv + (size_t)(unsigned)(base + min(k + 1, n - 1)) * (unsigned)ld + 2 * H + head * D +
@@ -206,20 +216,23 @@ __device__ __forceinline__ void stage_store(const Staging<T, R> &st, char *sK, c
     // Within each 16-key group the 4-key runs are stored in the order
     // 0-3, 8-11, 4-7, 12-15: the eight keys one lane feeds to a P.V step
     // (runs 4lh.. and 8+4lh.., the S^T accumulator order) are then one
-    // contiguous 16-byte read.
+    // contiguous 16-byte read, at chunk vt_chunk of the row.
 #pragma unroll
     for (int j = 0; j < R; j++) {
-      const int it = tid + NT * j, p = it & 31, g = it >> 5;
+      const int it = tid + NT * j, p = it >> 3, g = it & 7;
       const int lp = p & 7, q4 = lp >> 1;
       const int pw = (p & ~7) + ((((q4 & 1) << 1) | (q4 >> 1)) << 1) + (lp & 1);
+      int vx = (((pw >> 2) ^ g) << 4) + 4 * (pw & 3);
+      asm volatile("" : "+v"(vx));  // the eight store addresses are made from it here, not kept in registers
       const uint4 v0 = keep_if((st.valid >> (8 + j)) & 1, st.v0[j]), v1 = keep_if((st.valid >> (16 + j)) & 1, st.v1[j]);
       const uint32_t va[4] = {v0.x, v0.y, v0.z, v0.w};
       const uint32_t vb[4] = {v1.x, v1.y, v1.z, v1.w};
 #pragma unroll
       for (int w = 0; w < 4; w++) {
         // Byte permutes: (va & 0xffff) | (vb << 16) and (va >> 16) | (vb & 0xffff0000).
-        *(uint32_t *)(sV + (8 * g + 2 * w) * ROWV + 4 * pw) = __builtin_amdgcn_perm(vb[w], va[w], 0x05040100u);
-        *(uint32_t *)(sV + (8 * g + 2 * w + 1) * ROWV + 4 * pw) = __builtin_amdgcn_perm(vb[w], va[w], 0x07060302u);
+        *(uint32_t *)(sV + (8 * g + 2 * w) * ROWV + (vx ^ (32 * w))) = __builtin_amdgcn_perm(vb[w], va[w], 0x05040100u);
+        *(uint32_t *)(sV + (8 * g + 2 * w + 1) * ROWV + (vx ^ (32 * w + 16))) =
+            __builtin_amdgcn_perm(vb[w], va[w], 0x07060302u);
       }
     }
   } else {
@@ -272,14 +285,17 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
   static_assert(QT * QW <= 8, "tile codes hold 8 query chunks");
   using MF = Mfma<T>;
   typedef typename MF::frag frag;
-  constexpr int ROWK = D * sizeof(T) + 16;       // K tile row bytes (key-major)
-  constexpr int ROWV = KTILE * sizeof(T) + 16;   // V^T tile row bytes (d-major)
+  constexpr int ROWK = D * sizeof(T) + 16;  // K tile row bytes (key-major)
+  // V^T tile row bytes (d-major): 16-bit rows are swizzled (vt_chunk).
+  constexpr int ROWV = sizeof(T) == 2 ? KTILE * 2 : KTILE * 4 + 16;
   // 16-bit: two buffers, tile t is computed from one while tile t+1 is stored
   // into the other, with one barrier per tile. fp32 (the validation mode,
   // twice the bytes) keeps one buffer and a second barrier.
   constexpr int NBUF = sizeof(T) == 2 ? 2 : 1;
-  __shared__ __attribute__((aligned(16))) char sK[NBUF][KTILE * ROWK];
-  __shared__ __attribute__((aligned(16))) char sV[NBUF][D * ROWV];
+  constexpr int KV = KTILE * ROWK + D * ROWV;  // bytes of one buffer: K, then V^T
+  constexpr int ROWQ = D * sizeof(T), QROWS = 32 * QW * QT;  // the Q tile, before the first buffer is filled
+  constexpr int SMEM = NBUF * KV > QROWS * ROWQ ? NBUF * KV : QROWS * ROWQ;
+  __shared__ __attribute__((aligned(16))) char smem[SMEM];
   // Per staged key: option id (-1 prefix, -2 past the sequence end) and
   // position + half window, the fields the per-element mask tests.
   __shared__ __attribute__((aligned(16))) int sKo[NBUF][KTILE];
@@ -341,62 +357,82 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
     stage_load<T, R>(st, qkv, ld, H, head, base, n, kt * KTILE, a.cos_t, a.sin_t, ki, tid);
   }
 
-  // This lane's queries (one per query tile), their RoPE factors and the
-  // rotated Q^T operands (B operand: column = query, k = head dim).
+  // The work item's Q rows, rotated into LDS: thread items (row, 16-byte chunk
+  // pair (c, c + CPQ)), whole rows per load instruction. (Each wave loading
+  // its own MFMA fragments touched 32 rows with every instruction, which the
+  // CU's address unit serialises, and so did V's loads by key: together most
+  // of its work.)
   constexpr int NKS = D / MF::KSTEP;
-  frag qf[QT][NKS];
+  constexpr int EPC = 16 / (int)sizeof(T), CPQ = 32 / EPC, QI = QROWS * CPQ / NT;
+  auto q_token = [&](int idx, int &r) {  // token (in the sequence) and list row of query idx
+    if constexpr (LIST) {
+      r = a.rows[slot0 + (idx < cnt ? idx : 0)];
+      // a row token outside the sequence (flagged by the row gather) reads an in-bounds query
+      return min(max(a.row_tok[r] - base, 0), n - 1);
+    } else {
+      return min(q0 + idx, n - 1);
+    }
+  };
+  constexpr int QB = QI > 4 ? 4 : QI;  // items in flight
+  static_assert(QI % QB == 0, "Q items");
+#pragma clang loop unroll(disable)
+  for (int j0 = 0; j0 < QI; j0 += QB) {
+    uint4 ql[QB], qh[QB];
+    int qp[QB];
+#pragma unroll
+    for (int j = 0; j < QB; j++) {
+      const int it = tid + NT * (j0 + j), c = it % CPQ;
+      int r = 0;
+      const int qq = q_token(it / CPQ, r);
+      const T *row = LIST ? (const T *)a.q_rows + (size_t)r * H + head * D : qkv + (size_t)(base + qq) * ld + head * D;
+      qp[j] = a.kinfo[base + qq] & 0xffff;
+      ql[j] = *(const uint4 *)(row + EPC * c);
+      qh[j] = *(const uint4 *)(row + 32 + EPC * c);
+    }
+    typedef float FV __attribute__((ext_vector_type(EPC)));
+    FV qc[QB], qs[QB];
+#pragma unroll
+    for (int j = 0; j < QB; j++) {
+      const size_t o = (size_t)qp[j] * 32 + EPC * ((tid + NT * (j0 + j)) % CPQ);
+      qc[j] = *(const FV *)(a.cos_t + o);
+      qs[j] = *(const FV *)(a.sin_t + o);
+    }
+#pragma unroll
+    for (int j = 0; j < QB; j++) {
+      const int it = tid + NT * (j0 + j), row = it / CPQ, c = it % CPQ;
+      const uint32_t wl[4] = {ql[j].x, ql[j].y, ql[j].z, ql[j].w}, wh[4] = {qh[j].x, qh[j].y, qh[j].z, qh[j].w};
+      uint32_t ol[4], oh[4];
+#pragma unroll
+      for (int w = 0; w < 4; w++) {
+        if constexpr (sizeof(T) == 2) {
+          float a0 = lo16<T>(wl[w]), a1 = hi16<T>(wl[w]), b0 = lo16<T>(wh[w]), b1 = hi16<T>(wh[w]);
+          rope1(a0, b0, qc[j][2 * w], qs[j][2 * w]);
+          rope1(a1, b1, qc[j][2 * w + 1], qs[j][2 * w + 1]);
+          ol[w] = pack16<T>(a0, a1);
+          oh[w] = pack16<T>(b0, b1);
+        } else {
+          float x = __uint_as_float(wl[w]), y = __uint_as_float(wh[w]);
+          rope1(x, y, qc[j][w], qs[j][w]);
+          ol[w] = __float_as_uint(x);
+          oh[w] = __float_as_uint(y);
+        }
+      }
+      const int sw = row & (2 * CPQ - 1);  // chunk swizzle: reads of 32 rows' equal chunks spread over the banks
+      *(uint4 *)(smem + row * ROWQ + ((c ^ sw) << 4)) = make_uint4(ol[0], ol[1], ol[2], ol[3]);
+      *(uint4 *)(smem + row * ROWQ + (((c + CPQ) ^ sw) << 4)) = make_uint4(oh[0], oh[1], oh[2], oh[3]);
+    }
+  }
+  // This lane's queries (one per query tile).
   int qopt[QT], qpos[QT], qrow_r[QT];
   bool qvalid[QT];
 #pragma unroll
   for (int t = 0; t < QT; t++) {
-    int qq;
-    const T *qrow;
-    if constexpr (LIST) {
-      const int idx = (wave * QT + t) * 32 + lr;
-      qvalid[t] = idx < cnt;
-      const int r = a.rows[slot0 + (qvalid[t] ? idx : 0)];
-      qrow_r[t] = r;
-      // a row token outside the sequence (flagged by the row gather) reads an in-bounds query
-      qq = min(max(a.row_tok[r] - base, 0), n - 1);
-      qrow = (const T *)a.q_rows + (size_t)r * H + head * D;
-    } else {
-      const int q = q0 + (wave * QT + t) * 32 + lr;
-      qvalid[t] = q < n;
-      qq = qvalid[t] ? q : n - 1;
-      qrow = qkv + (size_t)(base + qq) * ld + head * D;
-    }
-    const int qinfo = a.kinfo[base + qq];
+    const int idx = (wave * QT + t) * 32 + lr;
+    qvalid[t] = LIST ? idx < cnt : q0 + idx < n;
+    qrow_r[t] = 0;
+    const int qinfo = a.kinfo[base + q_token(idx, qrow_r[t])];
     qopt[t] = (qinfo >> 16) - 1;
     qpos[t] = qinfo & 0xffff;
-    const float *cq = a.cos_t + (size_t)qpos[t] * 32, *sq = a.sin_t + (size_t)qpos[t] * 32;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ks++) qf[t][ks] = *(const frag *)(qrow + ks * MF::KSTEP + lh * MF::SLOTS);
-    // Pairs (i, i+32): step ks holds i = ks*KSTEP + lh*SLOTS + u, its partner
-    // is in step ks + NKS/2 at the same slot.
-#pragma unroll
-    for (int ks = 0; ks < NKS / 2; ks++)
-#pragma unroll
-      for (int u = 0; u < MF::SLOTS; u++) {
-#pragma clang fp contract(off)
-        const int i = ks * MF::KSTEP + lh * MF::SLOTS + u;
-        const float c = cq[i], sn = sq[i];
-        float x, y;
-        if constexpr (sizeof(T) == 2) {
-          x = (float)qf[t][ks][u];
-          y = (float)qf[t][ks + NKS / 2][u];
-        } else {
-          x = qf[t][ks];
-          y = qf[t][ks + NKS / 2];
-        }
-        const float x2 = x * c - y * sn, y2 = y * c + x * sn;
-        if constexpr (sizeof(T) == 2) {
-          qf[t][ks][u] = to_elem<T>(x2);
-          qf[t][ks + NKS / 2][u] = to_elem<T>(y2);
-        } else {
-          qf[t][ks] = x2;
-          qf[t][ks + NKS / 2] = y2;
-        }
-      }
   }
 
   f32x16 ot[QT][2];
@@ -411,7 +447,19 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
       for (int e = 0; e < 16; e++) ot[t][i][e] = 0.0f;
   }
 
-  __syncthreads();  // sCode visible
+  __syncthreads();  // sCode and the Q rows visible
+  frag qf[QT][NKS];  // Q^T operands (B operand: column = query, k = head dim)
+#pragma unroll
+  for (int t = 0; t < QT; t++) {
+    const int row = (wave * QT + t) * 32 + lr;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ks++) {
+      const int e = ks * MF::KSTEP + lh * MF::SLOTS;
+      qf[t][ks] = *(const frag *)(smem + row * ROWQ + (((e / EPC) ^ (row & (2 * CPQ - 1))) << 4) +
+                                  e % EPC * (int)sizeof(T));
+    }
+  }
+  __syncthreads();  // the Q rows read: the buffers may be filled
   auto next_tile = [&](int kt) {
     while (kt < nkt && sCode[kt] == 0) kt++;
     return kt;
@@ -424,7 +472,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
   // the key info of the one after that, one barrier.
   int kn = nkt, kn_next = nkt, b = 0;
   if (kt < nkt) {
-    if (stager) stage_store<T, R>(st, sK[0], sV[0], sKo[0], sKw[0], a.half_window, tid, ROWK, ROWV);
+    if (stager) stage_store<T, R>(st, smem, smem + KTILE * ROWK, sKo[0], sKw[0], a.half_window, tid, ROWK, ROWV);
     kn = next_tile(kt + 1);
     if (kn < nkt) {
       if (stager) {
@@ -438,7 +486,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
   }
   const unsigned win2 = (unsigned)(2 * a.half_window);
   while (kt < nkt) {
-    const char *sKb = sK[b], *sVb = sV[b];
+    const char *sKb = smem + b * KV, *sVb = sKb + KTILE * ROWK;
     const int *sKob = sKo[b], *sKwb = sKw[b];
     // This wave's classes: per query tile t and 32-key half i (uniform
     // across the wave).
@@ -540,6 +588,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
       // of tile i on lane half lh is key 32*i + 8*((r%16)/4) + 4*lh + r%4. A V
       // fragment read from LDS feeds every query tile that needs its half.
       constexpr int NPV = KTILE / MF::KSTEP;
+      int vsw = vt_chunk(lr, lh) << 4;
+      if constexpr (sizeof(T) == 2) asm volatile("" : "+v"(vsw));  // as vx in stage_store
 #pragma unroll
       for (int ks = 0; ks < NPV; ks++) {
         const int half = ks / (NPV / 2);
@@ -563,7 +613,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
           const char *vrow = sVb + (i * 32 + lr) * ROWV;
           frag vf;
           if constexpr (sizeof(T) == 2) {
-            vf = *(const frag *)(vrow + 32 * ks + 16 * lh);  // keys 16ks + {4lh..4lh+3, 8+4lh..8+4lh+3}
+            vf = *(const frag *)(vrow + (vsw ^ (32 * ks) ^ (64 * i)));  // keys 16ks + {4lh..4lh+3, 8+4lh..8+4lh+3}
           } else {
             const int r = ks & 15;
             const int key = 32 * (ks >> 4) + 8 * (r >> 2) + 4 * lh + (r & 3);
@@ -579,7 +629,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
     if (kn < nkt) {
       const int nb = NBUF == 2 ? b ^ 1 : 0;
       if constexpr (NBUF == 1) __syncthreads();  // every wave is done with the one buffer
-      if (stager) stage_store<T, R>(st, sK[nb], sV[nb], sKo[nb], sKw[nb], a.half_window, tid, ROWK, ROWV);
+      if (stager) stage_store<T, R>(st, smem + nb * KV, smem + nb * KV + KTILE * ROWK, sKo[nb], sKw[nb], a.half_window, tid, ROWK, ROWV);
       kn2 = kn_next;  // == next_tile(kn + 1); ki holds its key info
       if (kn2 < nkt) {
         if (stager) stage_load<T, R>(st, qkv, ld, H, head, base, n, kn2 * KTILE, a.cos_t, a.sin_t, ki, tid);
@@ -702,7 +752,7 @@ __device__ __forceinline__ void unit_load(UnitStage<T> &st, const T *qkv, int ld
   for (int j = 0; j < U::VI; j++) {
     const int it = lane + 64 * j;
     if constexpr (sizeof(T) == 2) {
-      const int k = k0 + 2 * (it & 15), g = it >> 4;
+      const int k = k0 + 2 * (it >> 3), g = it & 7;
       st.v0[j] = *(const uint4 *)(row(k) + 2 * H + 8 * g);
       st.v1[j] = *(const uint4 *)(row(k + 1) + 2 * H + 8 * g);
     } else {
@@ -754,7 +804,7 @@ __device__ __forceinline__ void unit_store(const UnitStage<T> &st, char *sK, cha
   for (int j = 0; j < U::VI; j++) {
     const int it = lane + 64 * j;
     if constexpr (sizeof(T) == 2) {
-      const int p = it & 15, g = it >> 4, lp = p & 7, q4 = lp >> 1;
+      const int p = it >> 3, g = it & 7, lp = p & 7, q4 = lp >> 1;
       const int pw = (p & ~7) + ((((q4 & 1) << 1) | (q4 >> 1)) << 1) + (lp & 1);
       const uint4 v0 = keep_if(k0 + 2 * p < n, st.v0[j]), v1 = keep_if(k0 + 2 * p + 1 < n, st.v1[j]);
       const uint32_t va[4] = {v0.x, v0.y, v0.z, v0.w}, vb[4] = {v1.x, v1.y, v1.z, v1.w};
