@@ -417,8 +417,8 @@ def train_bench(args) -> int:
         "loss_first_last": [round(losses[0], 5), round(losses[-1], 5)],
         "backward_probe_ms_per_launch": {k: round(v / max(nprobe, 1), 5) for k, v in probe.items()},
         "dgrad_qkv_tflops": round(qkv_flop / dg_s / 1e12, 2) if dg_s > 0 else None,
-        "roofline": {"kernel": "gemm_nt_kernel<bf16,64,128,128,5,EPI_F32> accumulating into the gradient (one "
-                               "split: 216 tiles): layer 1 dWqkv (weight-gradient stream, concurrent with the main "
+        "roofline": {"kernel": "gemm_nt_kernel<bf16,128,128,128,4,EPI_F32> accumulating into the gradient (one "
+                               "split: 108 tiles): layer 1 dWqkv (weight-gradient stream, concurrent with the main "
                                "stream)",
                      "bound": "mfma", "achieved": round(qkv_flop / wg_s / 1e12, 2) if wg_s > 0 else None,
                      "peak": PEAK[args.precision] / 1e12, "unit": "TFLOP/s",

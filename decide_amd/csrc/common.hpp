@@ -304,11 +304,11 @@ hipError_t launch_gemm_generic(int precision, int epi, const GemmArgs &a, hipStr
 // Whether launch_gemm takes this epilogue at M rows (EPI_GEGLU_BWD needs the
 // tiled kernel: M > 128 in bf16, M > 1024 in fp32).
 bool gemm_epi_ok(int precision, int epi, int M);
-// Split-K fp32-output GEMM: `splits` (1..16) partial products, each over a.K / splits
-// of K (a.K % (splits * 64) == 0), written to partial + split * M * N
-// (row-major, ldc = N), then summed in split order into C (M x N, ldc = N;
-// added to C when a.accumulate, else stored). partial holds splits * M * N floats.
-hipError_t launch_gemm_splitk(int precision, const GemmArgs &a, int splits, float *partial, hipStream_t s);
+// Weight-gradient GEMM into fp32 C (M x N, ldc = N; added to C when
+// a.accumulate, else stored): `splits` (1..16) partial products, each over a.K /
+// splits of K (a.K % (splits * 64) == 0), summed in split order. partial holds
+// splits * M * N floats for the shapes whose splits run as workgroups.
+hipError_t launch_gemm_wgrad(int precision, const GemmArgs &a, int splits, float *partial, hipStream_t s);
 // Small M (<= 128) split-K on the whole-K kernel, no reduction: workgroup z of
 // a tile multiplies K elements [z*K/splits, (z+1)*K/splits) and stores its
 // fp32 partial product at partial + z * M * N (row-major, ldc = N); a.C,

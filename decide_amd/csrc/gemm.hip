@@ -199,8 +199,12 @@ __device__ __forceinline__ float2 ln_fold_merge(const GemmArgs &g, const LnFold 
 // The body of gemm_nt_kernel and gemm_nt_ln_kernel (lf: the folded
 // LayerNorm's arguments, used by the EPI_*_LN forms only; PC: its statistics'
 // columns per part). PF: the main loop for small wave tiles (below).
-template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM, int WGN, bool PF, int PC>
-__device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf) {
+// SEG: the product is the sum of K / (seg stages) partial products, each
+// summed from zero and added in K order, to the bit what a split over
+// workgroups and a reduction in split order give.
+template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM, int WGN, bool PF, int PC, bool SEG = false>
+__device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf, int seg = 0) {
+  static_assert(!SEG || PF, "segments are summed in the operand-resident loop");
   using MF = Mfma<T>;
   typedef typename MF::frag frag;
   constexpr int NW = WGM * WGN, NT = 64 * NW;
@@ -341,6 +345,30 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
     // No scalar load in flight past here, so the compiler's waits in the loop
     // count LDS reads exactly.
     __builtin_amdgcn_s_waitcnt(0xc07f);
+    f32x16 total[SEG ? TM : 1][SEG ? TN : 1];
+    int left = seg;  // stages to the segment's end
+    if constexpr (SEG)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) total[i][j][e] = 0.0f;
+    auto end_stage = [&]() {
+      if constexpr (SEG)
+        if (--left == 0) {
+          left = seg;
+#pragma unroll
+          for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+              for (int e = 0; e < 16; e++) {
+                total[i][j][e] += acc[i][j][e];
+                acc[i][j][e] = 0.0f;
+              }
+        }
+    };
     int kt = 0, slot = 0;
     for (; kt + NSTAGE - 1 < nk; kt++) {
       const int nslot = slot + 1 == NSTAGE ? 0 : slot + 1, pslot = slot == 0 ? NSTAGE - 1 : slot - 1;
@@ -357,6 +385,7 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
         __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
         __builtin_amdgcn_sched_group_barrier(0x020, PER_KS, 0);
       }
+      end_stage();
       slot = nslot;
     }
     auto tail = [&](auto tc) {
@@ -372,6 +401,7 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
           mfmas(ks);
           if constexpr (TT < NSTAGE - 2) load_step(nslot, ks);
         }
+        end_stage();
         slot = nslot;
         kt++;
       }
@@ -381,6 +411,11 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
     tail(std::integral_constant<int, 1>{});
     if constexpr (NSTAGE > 3) tail(std::integral_constant<int, 2>{});
     if constexpr (NSTAGE > 4) tail(std::integral_constant<int, 3>{});
+    if constexpr (SEG)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = total[i][j];
   } else {
     // MFMA operands are double buffered across k steps: the fragments of step
     // ks+1 (or of the next stage's step 0) are read from LDS while the MFMAs of
@@ -758,6 +793,11 @@ template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM
 __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm_nt_kernel(GemmArgs g) {
   static_assert(EPI < EPI_F32_LN, "the folded-LayerNorm forms run as gemm_nt_ln_kernel");
   gemm_nt_tile<T, BM, BN, RB, NSTAGE, EPI, WPE, WGM, WGN, PF, 0>(g, LnFold{});
+}
+template <class T, int BM, int BN, int RB, int NSTAGE, int WPE, int WGM, int WGN>
+__global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm_nt_seg_kernel(GemmArgs g,
+                                                                                                             int seg) {
+  gemm_nt_tile<T, BM, BN, RB, NSTAGE, EPI_F32, WPE, WGM, WGN, true, 0, true>(g, LnFold{}, seg);
 }
 template <class T, int BM, int BN, int RB, int NSTAGE, int EPI, int WPE, int WGM, int WGN, bool PF, int PC>
 __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm_nt_ln_kernel(GemmArgs g,
@@ -1329,26 +1369,6 @@ __global__ void splitk_reduce_kernel(const float *part, int splits, size_t n, fl
 
 }  // namespace
 
-hipError_t launch_gemm_splitk(int precision, const GemmArgs &a0, int splits, float *partial, hipStream_t s) {
-  if (a0.M <= 0) return hipSuccess;
-  if (precision == PREC_F16) return hipErrorInvalidValue;  // training only
-  if (splits < 1 || splits > 16 || a0.K % (splits * 64) != 0 || a0.N % 128 != 0) return hipErrorInvalidValue;
-  GemmArgs a = a0;
-  a.K = a0.K / splits;
-  a.C = partial;
-  a.ldc = a0.N;
-  a.n_store = a0.N;
-  a.accumulate = 0;
-  a.c_split = (size_t)a0.M * a0.N;
-  const hipError_t e = precision == PREC_BF16 ? launch_tile<bf16, Tile<64, 128, 128, 5, 1, 2, 4, true>, EPI_F32>(a, s, nullptr, splits)
-                                              : launch_tile<float, Tile<128, 128, 128, 3, 1, 2, 2>, EPI_F32>(a, s, nullptr, splits);
-  if (e != hipSuccess) return e;
-  const size_t n = (size_t)a0.M * a0.N;
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, partial, splits,
-                     n, (float *)a0.C, a0.accumulate);
-  return hipGetLastError();
-}
-
 hipError_t launch_gemm_small_split(int precision, const GemmArgs &a, int splits, float *partial, hipStream_t s) {
   if (a.M <= 0) return hipSuccess;
   const int kt = prec16(precision) ? 64 : 32;
@@ -1457,20 +1477,27 @@ hipError_t launch_f32(const GemmArgs &a, hipStream_t s) {
   return launch_tile<T, F256x192, EPI_F32>(a, s);
 }
 
-// Operand-type outputs (store, GeGLU and their folded-LayerNorm forms), by
-// the same rule; past one round of 128 x 128, 256 x 128 tiles at two
-// workgroups per CU, whose epilogues and DMA stalls overlap the other's
+// Operand-type outputs (store, GeGLU, its backward and the folded-LayerNorm
+// forms), by the same rule; past the largest one-round tile, 256 x 128 tiles at
+// two workgroups per CU, whose epilogues and DMA stalls overlap the other's
 // MFMAs. N = 2304, K = 768, store / GeGLU, isolated launches as above (us):
 //   64 x 64 (two waves)  208 rows  5.8 /  6.1  (64 x 128:  6.8 /  7.1)
 //   128 x 64             600       7.0 /  7.4  (64 x 128:  8.1 /  8.5)
 //   128 x 128, 8 waves 1,500       9.4 /  9.8  (128 x 128, 64-byte stages: 12.5 / 13.0)
-//   256 x 128, 8 waves 3,000      15.8 / 16.2  (128 x 128, 64-byte stages: 18.3 / 18.5)
+//   192 x 128          2,046      12.6 / 13.3  (256 x 128, 8 waves: 14.4 / 15.6)
+//   256 x 128, 8 waves 3,000      16.3 / 17.0  (128 x 128, 64-byte stages: 19.3 / 19.9)
+//   192 x 256          3,840      21.8 / 23.7  (128 x 128, 64-byte stages: 26.1 / 26.5)
+//                      5,376      24.0 / 25.6  (256 x 128, two per CU: 27.9 / 28.9)
+//   256 x 256          7,000      30.4 / 31.0  (256 x 128, two per CU: 32.2 / 34.2)
 // At 64 x 64 the line lies at 160 workgroups: 252 of them (448 rows) took
 // 7.2 us against 6.8 for 128 x 64.
 typedef Tile<64, 64, 128, 5, 1, 2, 1, true> S64x64;
 typedef Tile<128, 64, 128, 4, 1, 4, 1, true> S128x64;
 typedef Tile<128, 128, 128, 4, 1, 4, 2, true> S128x128;
+typedef Tile<192, 128, 128, 3, 1, 2, 2> S192x128;
 typedef Tile<256, 128, 128, 3, 1, 4, 2> S256x128;
+typedef Tile<192, 256, 128, 2, 2, 2, 4> S192x256;
+typedef Tile<256, 256, 64, 5, 2, 2, 4, true> S256x256;
 typedef Tile<128, 128, 64, 3, 3, 2, 2> S128x128s;
 typedef Tile<256, 128, 64, 3, 2, 2, 2> S256x128s;
 
@@ -1481,8 +1508,12 @@ hipError_t launch_store(const GemmArgs &a, hipStream_t s, const LnFold *ln = nul
     if (S64x64::count(a) <= 160) return launch_tile<T, S64x64, EPI, PC>(a, s, ln);
     if (S128x64::count(a) <= kCUs) return launch_tile<T, S128x64, EPI, PC>(a, s, ln);
     if (S128x128::count(a) <= kCUs) return launch_tile<T, S128x128, EPI, PC>(a, s, ln);
+    if (S192x128::count(a) <= kCUs) return launch_tile<T, S192x128, EPI, PC>(a, s, ln);
     if (S256x128::count(a) <= kCUs) return launch_tile<T, S256x128, EPI, PC>(a, s, ln);
   }
+  if (a.N % 256 == 0 && S192x256::count(a) <= kCUs) return launch_tile<T, S192x256, EPI, PC>(a, s, ln);
+  if constexpr (EPI == EPI_STORE || EPI == EPI_GEGLU)
+    if (a.N % 256 == 0 && S256x256::count(a) <= kCUs) return launch_tile<T, S256x256, EPI, PC>(a, s, ln);
   if (a.M <= (gated ? 8192 : 4096)) return launch_tile<T, S128x128s, EPI, PC>(a, s, ln);
   return launch_tile<T, S256x128s, EPI, PC>(a, s, ln);
 }
@@ -1525,11 +1556,7 @@ hipError_t launch_gemm16(int epi, const GemmArgs &a, hipStream_t s, const LnFold
   }
   if constexpr (std::is_same<T, bf16>::value) {  // training: bf16 only
     if (epi == EPI_GEGLU_KEEP) return launch_store<T, EPI_GEGLU_KEEP>(a, s);
-    // GeGLU backward (N = 1152) at medium M: 64 x 192 at two workgroups per
-    // CU (3840 rows: 30.2 -> 25.8 us isolated).
-    if (a.M <= 1024) return launch_tile<T, Tile<64, 128, 128, 4, 1, 2, 2>, EPI_GEGLU_BWD>(a, s);
-    if (a.M <= 4096 && a.N % 192 == 0) return launch_tile<T, Tile<64, 192, 64, 4, 2, 2, 2>, EPI_GEGLU_BWD>(a, s);
-    return launch_tile<T, F128x128s, EPI_GEGLU_BWD>(a, s);
+    if (epi == EPI_GEGLU_BWD) return launch_store<T, EPI_GEGLU_BWD>(a, s);
   }
   return hipErrorInvalidValue;
 }
@@ -1574,4 +1601,42 @@ hipError_t launch_gemm(int precision, int epi, const GemmArgs &a, hipStream_t s,
   if (precision == PREC_F16) return launch_gemm16<f16>(epi, a, s, ln);
   if (f32_small_tiles(epi, a)) return launch_skinny<float>(epi, a, s);
   return launch_gemm_f32_tile<Tile<256, 128, 128, 3, 1, 2, 2>>(epi, a, s);
+}
+
+// Weight gradients: C (+)= A . B^T over the tokens (K) in `splits` partial
+// sums added in order. They run on the side stream beside the input-gradient
+// chain, so what they cost is the CU time they hold, not their own latency:
+// in bf16 a 128 x 128 tile walks its splits one after the other (half the
+// operand bytes per output of 64 x 128 tiles, and no partial outputs to write
+// and read; dWqkv at 3840 tokens: 108 workgroups for 25 us against 216 for 21
+// us; the backward of a step of 32 x 384 tokens in four micro-batches over 22
+// layers 22.7 -> 21.7 ms). Fewer than 32 such tiles (hidden sizes below 768) would leave the side
+// stream behind the chain and stay split over workgroups.
+hipError_t launch_gemm_wgrad(int precision, const GemmArgs &a0, int splits, float *partial, hipStream_t s) {
+  if (a0.M <= 0) return hipSuccess;
+  if (precision == PREC_F16) return hipErrorInvalidValue;  // training only
+  if (splits < 1 || splits > 16 || a0.K % (splits * 64) != 0 || a0.N % 128 != 0) return hipErrorInvalidValue;
+  const bool bf = precision == PREC_BF16;
+  GemmArgs a = a0;
+  a.ldc = a0.N;
+  a.n_store = a0.N;
+  if (bf && F128x128::count(a) >= 32) {
+    typedef F128x128 C;
+    if (splits == 1) return launch_tile<bf16, C, EPI_F32>(a, s);
+    hipLaunchKernelGGL((gemm_nt_seg_kernel<bf16, C::BM, C::BN, C::RB, C::NSTAGE, C::WPE, C::WGM, C::WGN>),
+                       dim3(C::count(a)), dim3(64 * C::WGM * C::WGN), 0, s, a, a.K / splits / 64);
+    return hipGetLastError();
+  }
+  if (splits == 1) return launch_gemm(precision, EPI_F32, a, s);
+  a.K = a0.K / splits;
+  a.C = partial;
+  a.accumulate = 0;
+  a.c_split = (size_t)a0.M * a0.N;
+  const hipError_t e = bf ? launch_tile<bf16, F64x128, EPI_F32>(a, s, nullptr, splits)
+                          : launch_tile<float, Tile<128, 128, 128, 3, 1, 2, 2>, EPI_F32>(a, s, nullptr, splits);
+  if (e != hipSuccess) return e;
+  const size_t n = (size_t)a0.M * a0.N;
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, partial, splits,
+                     n, (float *)a0.C, a0.accumulate);
+  return hipGetLastError();
 }

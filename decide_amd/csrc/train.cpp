@@ -14,8 +14,9 @@
 //   gWqkv += dqkv^T . n1           dn1 = dqkv . Wqkv
 //   dprev = dh1 + LNbwd(dn1)       (attn_norm; layer 0: dh1 + dn1)
 // Input-gradient GEMMs run on the forward GEMM kernel with a transposed copy
-// of the weights; weight-gradient GEMMs (a reduction over tokens) run split-K
-// on transposed operand copies, with partial products summed in split order.
+// of the weights; weight-gradient GEMMs (a reduction over tokens) run on
+// transposed operand copies, with partial products of token ranges summed in
+// order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -94,10 +95,9 @@ int refresh_wt(dn_ctx *c, const std::string &name, TensorSlot &t) {
 }
 
 // Splits of the token (K) dimension for a weight-gradient GEMM: about 200
-// workgroups of 64 x 128 (bf16) or 512 of 128 x 128 (fp32) in all, while each
-// split keeps at least 512 tokens of K; the partial outputs cost splits x M x N
-// floats of extra traffic. (Isolated bf16 launches at 3840 tokens: dWqkv
-// 36.7 us as 128 x 128 tiles x 4 splits, 24.8 us as 64 x 128 tiles unsplit.)
+// tiles of 64 x 128 (bf16) or 512 of 128 x 128 (fp32) in all, while each split
+// keeps at least 512 tokens of K. Where the splits go to workgroups of their
+// own the partial outputs cost splits x M x N floats of extra traffic.
 int split_count(int prec, int M, int N, int Tp) {
   const bool bf = prec == DN_PRECISION_BF16;
   const int tiles = ((M + (bf ? 63 : 127)) / (bf ? 64 : 128)) * (N / 128);
@@ -149,14 +149,7 @@ struct Bwd {
     a.N = N;
     a.K = Tp;
     a.accumulate = 1;
-    const int sp = split_count(prec, M, N, Tp);
-    if (sp == 1) {  // one split: accumulate straight into the gradient
-      a.ldc = N;
-      a.n_store = N;
-      HIPCHK(c, "gemm", launch_gemm(prec, EPI_F32, a, ws));
-      return DN_OK;
-    }
-    HIPCHK(c, "gemm(split-K)", launch_gemm_splitk(prec, a, sp, (float *)c->tr.part.p, ws));
+    HIPCHK(c, "gemm(wgrad)", launch_gemm_wgrad(prec, a, split_count(prec, M, N, Tp), (float *)c->tr.part.p, ws));
     return DN_OK;
   }
   // dst [cols x Tp] = src[T x cols]^T in the operand type (zero past T); with

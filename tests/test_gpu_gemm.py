@@ -162,9 +162,12 @@ def test_gemm_16bit_device_store(eng, prec, M, N, K):
     ("bf16", 129, 768, 64, False), ("bf16", 129, 768, 192, False), ("fp16", 1344, 768, 320, False),
     ("bf16", 1345, 768, 1152, False), ("bf16", 2689, 768, 768, False), ("fp16", 5377, 768, 768, False),
     ("bf16", 5441, 768, 1152, False), ("bf16", 8193, 768, 768, False), ("bf16", 200, 128, 256, False),
-    # stored outputs, N = 2304: 64 x 64, 128 x 64, 128 x 128, 256 x 128
+    # stored outputs, N = 2304: 64 x 64, 128 x 64, 128 x 128, 192 x 128, 256 x 128
+    # (N = 2176 keeps it above 3,584 rows), 192 x 256, 256 x 256, 256 x 128 in several rounds
     ("bf16", 129, 2304, 64, True), ("fp16", 256, 2304, 256, True), ("bf16", 257, 2304, 768, True),
     ("bf16", 897, 2304, 128, True), ("fp16", 1793, 2304, 768, True), ("bf16", 3585, 2304, 192, True),
+    ("fp16", 2689, 2304, 64, True), ("bf16", 3585, 2176, 768, True), ("fp16", 5376, 2304, 64, True),
+    ("bf16", 5377, 2304, 64, True), ("fp16", 7168, 2304, 768, True), ("bf16", 7169, 2304, 192, True),
     ("bf16", 4097, 128, 768, True)])
 def test_gemm_tile_boundaries(eng, prec, M, N, K, store):
     """Row counts on both sides of each tile rule and K from one stage up

@@ -411,6 +411,53 @@ def test_backward_matches_oracle_medium_rows(prec):
         check_grads(eng, want, prec, label="medium")
 
 
+@pytest.mark.parametrize("tokens", [1500, 3500, 5376, 5900, 8250])
+def test_backward_bit_equal_by_rows(tokens):
+    """One 768-wide layer in bf16 at row counts of each GeGLU-backward tile (128 x
+    64, 128 x 128, 192 x 128 at its last row count, 256 x 128 in one round and
+    in several) against the same sequences a few hundred rows at a time: a token
+    id that occurs once has the same embedding gradient to the bit, since no
+    tile or batch changes the order of a row's sums. Weight gradients are sums
+    over the tokens in another order: 2^-24 sqrt(tokens) of their norm is
+    5e-6, and 20 times that is allowed for cancellation."""
+    from decide_amd.nn import Config, build_sequence
+    from decide_amd.train import TrainEngine
+
+    cfg = Config(hidden=768, intermediate=1152, heads=12, layers=1, vocab=10001, half_window=64,
+                 layer_types=["full_attention"])
+    mask = cfg.vocab - 1
+    w = weights_for(cfg, seed=15, std=0.02)
+    rng = np.random.default_rng(16)
+    ids = rng.permutation(np.arange(3, mask)).astype(np.int32)
+    batch, used = [], 0
+    while used < tokens:
+        n = min(300, tokens - used)
+        seq = ids[used:used + n].copy()
+        seq[[n - 60, n - 40, n - 20]] = mask
+        batch.append(build_sequence(seq, mask, independent=len(batch) % 2 == 0))
+        used += n
+    once = np.setdiff1d(np.concatenate([s.ids for s in batch]), [mask])
+    dl = (rng.standard_normal(sum(len(s.mask_pos) for s in batch)) * 0.1).astype(np.float32)
+    print(f"case: one layer backward by rows, T={sum(len(s.ids) for s in batch)}", flush=True)
+    tok = "model.embeddings.tok_embeddings.weight"
+    got = []
+    with TrainEngine(cfg, w, precision="bf16") as eng:
+        for step in (len(batch), 1):
+            row = 0
+            for i in range(0, len(batch), step):
+                part = batch[i:i + step]
+                r = sum(len(s.mask_pos) for s in part)
+                eng.forward(part)
+                eng.backward(dl[row:row + r])
+                row += r
+            got.append({n: eng.download(n, "grad") for n in [tok] + [f"model.layers.0.{p}" for p in PROJ]})
+            eng.zero_grad()
+    assert np.any(got[0][tok][once]) and np.array_equal(got[0][tok][once], got[1][tok][once])
+    for name in got[0]:
+        a, b = got[0][name].astype(np.float64), got[1][name].astype(np.float64)
+        assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(a), name
+
+
 def test_backward_full_size_deterministic_and_linear():
     """At the trainer's micro-batch size (10 examples x 384 tokens under the
     4000-token budget, ModernBERT-base, bf16, embeddings trained): a second
