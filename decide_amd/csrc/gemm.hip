@@ -831,16 +831,17 @@ hipError_t launch_tile(const GemmArgs &a, hipStream_t s, const LnFold *ln = null
 // Workgroups of a launch that runs in one round on 256 CUs.
 constexpr int kCUs = 256;
 
-// Small-M GEMM (M <= 128 in bf16: one request; M <= 1024 in fp32: the
-// scorer's dense layer over every [MASK] row of a batch). Such
+// Small-M GEMM (M <= 128 in 16 bits: one request; fp32: f32_small_tiles, among
+// them the scorer's dense layer over every [MASK] row of a batch). Such
 // launches are bound by streaming the weights and by latency, and the
 // 128-wide tiles above would give only N/128 workgroups. Here a workgroup
 // owns a TR x TC output tile (TR = 32*MB rows, TC = 32*NB columns) and all
 // of K:
 //   * K is walked in groups of GK elements (four 16-byte loads per lane and
-//     operand row); the W waves take the groups round-robin and load their
-//     MFMA operands straight from global memory into registers (every
-//     operand is used by one wave only, so LDS staging buys nothing),
+//     operand row); the W waves take the groups round-robin, each through
+//     LDS of its own (DMA: whole rows a load, since the CU's address unit
+//     serialises loads that touch 32 rows) or, on the 64-row and 16-bit
+//     64-column tiles, straight from global memory into registers,
 //     prefetching the next group while the current one is multiplied.
 //   * The waves' partial tiles are summed through LDS in a fixed order, so
 //     results do not depend on timing, by the threads that store the
@@ -1378,7 +1379,8 @@ hipError_t launch_gemm_small_split(int precision, const GemmArgs &a, int splits,
                                  : launch_skinny_split<float>(a, splits, partial, s);
 }
 
-// All tile configs use BN = 128; K is staged 64 or 128 bytes per step.
+// Rows of B come in 128s (every tile width used divides N or is chosen only
+// where it does); K is staged 64 or 128 bytes per step.
 bool gemm_shape_ok(int precision, int N, int K) {
   const int kt = prec16(precision) ? 64 : 32;
   return N > 0 && K > 0 && N % 128 == 0 && K % kt == 0;
