@@ -1187,11 +1187,12 @@ struct RowStage {
   static constexpr int NI = sizeof(T) == 2 ? 1 : 2;
   uint4 lo[NI], hi[NI];
   float4 c0[NI], c1[NI], s0[NI], s1[NI];
+  int pos[NI];
 };
 
 template <class T, bool ROT>
 __device__ __forceinline__ void rows_load(RowStage<T> &st, const T *src, int ld, int base, int r0, int n,
-                                          const float *cos_t, const float *sin_t, const int *kinfo, int tid) {
+                                          const int *kinfo, int tid) {
   constexpr int EL = 16 / sizeof(T), CPH = 32 / EL;  // elements per chunk, chunks per half row
 #pragma unroll
   for (int j = 0; j < RowStage<T>::NI; j++) {
@@ -1201,14 +1202,22 @@ __device__ __forceinline__ void rows_load(RowStage<T> &st, const T *src, int ld,
     const T *p = src + tok * ld;
     st.lo[j] = keep_if(ok, *(const uint4 *)(p + EL * c));
     st.hi[j] = keep_if(ok, *(const uint4 *)(p + 32 + EL * c));
-    if constexpr (ROT) {
-      const size_t pos = (size_t)(kinfo[tok] & 0xffff);
-      st.c0[j] = *(const float4 *)(cos_t + pos * 32 + EL * c);
-      st.s0[j] = *(const float4 *)(sin_t + pos * 32 + EL * c);
-      if constexpr (sizeof(T) == 2) {
-        st.c1[j] = *(const float4 *)(cos_t + pos * 32 + EL * c + 4);
-        st.s1[j] = *(const float4 *)(sin_t + pos * 32 + EL * c + 4);
-      }
+    if constexpr (ROT) st.pos[j] = kinfo[tok] & 0xffff;
+  }
+}
+
+// The RoPE factors of the rows that rows_load<T, true> read.
+template <class T>
+__device__ __forceinline__ void rows_factors(RowStage<T> &st, const float *cos_t, const float *sin_t, int tid) {
+  constexpr int EL = 16 / sizeof(T), CPH = 32 / EL;
+#pragma unroll
+  for (int j = 0; j < RowStage<T>::NI; j++) {
+    const size_t o = (size_t)st.pos[j] * 32 + EL * ((tid + 256 * j) % CPH);
+    st.c0[j] = *(const float4 *)(cos_t + o);
+    st.s0[j] = *(const float4 *)(sin_t + o);
+    if constexpr (sizeof(T) == 2) {
+      st.c1[j] = *(const float4 *)(cos_t + o + 4);
+      st.s1[j] = *(const float4 *)(sin_t + o + 4);
     }
   }
 }
@@ -1264,13 +1273,16 @@ __device__ __forceinline__ void build_transposed(const char *R, char *TT, int ti
   constexpr int ROW = D * sizeof(T) + 16;
   if constexpr (sizeof(T) == 2) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int it = tid + 256 * j, p = it & 31, d = it >> 5;
-      const uint32_t lo = *(const uint16_t *)(R + (2 * p) * ROW + 2 * d);
-      const uint32_t hi = *(const uint16_t *)(R + (2 * p + 1) * ROW + 2 * d);
+    for (int j = 0; j < 4; j++) {
+      // Row pair p, columns d and d + 1: two words in, two out. A wave's lanes
+      // are 16 row pairs x 4 column pairs, two to a bank (32 pairs: four).
+      const int it = tid + 256 * j, p = (it & 15) | ((it >> 2) & 16), d = 2 * (((it >> 4) & 3) | ((it >> 7) << 2));
+      const uint32_t lo = *(const uint32_t *)(R + (2 * p) * ROW + 2 * d);
+      const uint32_t hi = *(const uint32_t *)(R + (2 * p + 1) * ROW + 2 * d);
       const int lp = p & 7, q4 = lp >> 1;
       const int pw = (p & ~7) + ((((q4 & 1) << 1) | (q4 >> 1)) << 1) + (lp & 1);
-      *(uint32_t *)(TT + d * ROW + 4 * pw) = lo | (hi << 16);
+      *(uint32_t *)(TT + d * ROW + 4 * pw) = (lo & 0xffffu) | (hi << 16);
+      *(uint32_t *)(TT + (d + 1) * ROW + 4 * pw) = (lo >> 16) | (hi & 0xffff0000u);
     }
   } else {
 #pragma unroll
@@ -1434,19 +1446,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
 
   __syncthreads();  // sCode
   const unsigned win2 = a.sliding ? (unsigned)(2 * a.half_window) : 0xffffffffu;
-  for (int kt = a.first[wi]; kt < nkt; kt++) {
-    if (sCode[kt] == 0) continue;
+  // 16-bit operands: the next needed tile is loaded into registers while this
+  // one is computed (a training micro-batch has about one workgroup per CU, so
+  // nothing else hides the loads). fp32 tiles take twice the registers, which
+  // would spill. With the transposed copies built from words: this kernel 31.9
+  // -> 30.6 us, the one below 56.2 -> 45.7 us, averaged over a step of 32 x 384
+  // tokens beside the weight-gradient stream (the step 32.55 -> 32.25 ms).
+  constexpr bool AHEAD = sizeof(T) == 2;
+  RowStage<T> sk, sv;
+  int info = 0;
+  auto load = [&](int kt) {
     const int k0 = kt * KTILE;
-    {
-      RowStage<T> sk, sv;
-      rows_load<T, true>(sk, qkv + H + head * D, ld, base, k0, n, a.cos_t, a.sin_t, a.kinfo, tid);
-      rows_load<T, false>(sv, qkv + 2 * H + head * D, ld, base, k0, n, nullptr, nullptr, nullptr, tid);
-      const int info = (tid < KTILE && k0 + tid < n) ? a.kinfo[base + k0 + tid] : 0;
-      __syncthreads();  // the previous tile's reads are done
-      rows_store<T, true>(sk, sK, tid);
-      rows_store<T, false>(sv, sV, tid);
-      if (tid < KTILE) sInfo[tid] = info;
-    }
+    rows_load<T, true>(sk, qkv + H + head * D, ld, base, k0, n, a.kinfo, tid);
+    rows_load<T, false>(sv, qkv + 2 * H + head * D, ld, base, k0, n, nullptr, tid);
+    rows_factors<T>(sk, a.cos_t, a.sin_t, tid);
+    info = (tid < KTILE && k0 + tid < n) ? a.kinfo[base + k0 + tid] : 0;
+  };
+  auto needed = [&](int kt) {  // the first needed tile from kt on
+    while (kt < nkt && __builtin_amdgcn_readfirstlane((int)sCode[kt]) == 0) kt++;
+    return kt;
+  };
+  int next = needed(a.first[wi]);
+  if (AHEAD && next < nkt) load(next);
+  while (next < nkt) {
+    const int kt = next, k0 = kt * KTILE;
+    if (!AHEAD) load(kt);
+    __syncthreads();  // the previous tile's reads are done
+    rows_store<T, true>(sk, sK, tid);
+    rows_store<T, false>(sv, sV, tid);
+    if (tid < KTILE) sInfo[tid] = info;
+    next = needed(kt + 1);
+    if (AHEAD && next < nkt) load(next);
     __syncthreads();
     build_transposed<T>(sK, sKT, tid);
     __syncthreads();
@@ -1586,11 +1616,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   const float c = a.scale_log2;
   const unsigned win2 = a.sliding ? (unsigned)(2 * a.half_window) : 0xffffffffu;
   const int nqt = (n + KTILE - 1) / KTILE;
-  for (int qt = 0; qt < nqt; qt++) {
-    const int q0 = qt * KTILE;
+  // Classes of query tile qt for this wave; false: no wave needs the tile.
+  auto classes = [&](int qt, int (&hcls)[2]) {
     const ChunkInfo qc0 = a.chunks[cbase + 2 * qt];
     const ChunkInfo qc1 = 2 * qt + 1 < nch ? a.chunks[cbase + 2 * qt + 1] : empty;
-    int any = 0, hcls[2] = {0, 0};
+    int any = 0;
+    hcls[0] = hcls[1] = 0;
 #pragma unroll
     for (int w = 0; w < 4; w++) {
       const int c0 = tile_class(qc0, kc[w], a.sliding, a.half_window);
@@ -1601,33 +1632,49 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
         hcls[1] = c1;
       }
     }
-    if (any == 0) continue;
-    // Staged one operand at a time after the barrier (fewer live registers:
-    // two workgroups per CU hide the load latency).
+    return any != 0;
+  };
+  // 16-bit operands: the next needed tile is loaded ahead as in the kernel
+  // above, its RoPE factors (16 registers) only when it is stored.
+  constexpr bool AHEAD = sizeof(T) == 2;
+  RowStage<T> sq, so;
+  int info = 0;
+  float lse = INFINITY, dd = 0.0f;
+  auto load = [&](int qt) {
+    const int q0 = qt * KTILE;
+    rows_load<T, true>(sq, qkv + head * D, ld, base, q0, n, a.kinfo, tid);
+    rows_load<T, false>(so, (const T *)a.dctx + head * D, H, base, q0, n, nullptr, tid);
+    info = 0;
+    lse = INFINITY;  // rows past the end: P = 2^-inf = 0
+    dd = 0.0f;
+    if (tid < KTILE && q0 + tid < n) {
+      const size_t t = (size_t)(base + q0 + tid);
+      info = a.kinfo[t];
+      lse = a.lse[t * a.heads + head];
+      dd = a.dsum[t * a.heads + head];
+    }
+  };
+  int next = 0, ncls[2] = {0, 0};
+  while (next < nqt && !classes(next, ncls)) next++;
+  if (AHEAD && next < nqt) load(next);
+  while (next < nqt) {
+    const int q0 = next * KTILE, hcls[2] = {ncls[0], ncls[1]};
+    if (AHEAD) rows_factors<T>(sq, a.cos_t, a.sin_t, tid);
     __syncthreads();  // the previous tile's reads are done
-    {
-      RowStage<T> sq;
-      rows_load<T, true>(sq, qkv + head * D, ld, base, q0, n, a.cos_t, a.sin_t, a.kinfo, tid);
-      rows_store<T, true>(sq, sQ, tid);
+    if (!AHEAD) {
+      load(next);
+      rows_factors<T>(sq, a.cos_t, a.sin_t, tid);
     }
-    {
-      RowStage<T> so;
-      rows_load<T, false>(so, (const T *)a.dctx + head * D, H, base, q0, n, nullptr, nullptr, nullptr, tid);
-      rows_store<T, false>(so, sO, tid);
-    }
+    rows_store<T, true>(sq, sQ, tid);
+    rows_store<T, false>(so, sO, tid);
     if (tid < KTILE) {
-      int info = 0;
-      float lse = INFINITY, dd = 0.0f;  // rows past the end: P = 2^-inf = 0
-      if (q0 + tid < n) {
-        const size_t t = (size_t)(base + q0 + tid);
-        info = a.kinfo[t];
-        lse = a.lse[t * a.heads + head];
-        dd = a.dsum[t * a.heads + head];
-      }
       sInfo[tid] = info;
       sL[tid] = lse;
       sD[tid] = dd;
     }
+    do next++;
+    while (next < nqt && !classes(next, ncls));
+    if (AHEAD && next < nqt) load(next);
     __syncthreads();
     build_transposed<T>(sQ, sQT, tid);
     build_transposed<T>(sO, sOT, tid);
