@@ -694,6 +694,16 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
 // ms, 2,044 tokens (16 items) 12.3 / 13.1 ms, 4 x 1024 17.0 / 17.1 ms: hence the
 // lines at 8 and 16 items.
 
+// Orders a wave's own LDS accesses where lanes read what others wrote (or
+// overwrite what others read). The hardware runs a wave's LDS operations in
+// order; the fences keep the compiler from moving them across (the barrier
+// alone is no memory operation) and emit nothing.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // One unit (32 keys) of a wave's staging, the items of Staging above spread
 // over 64 lanes.
 template <class T>
@@ -816,10 +826,10 @@ __device__ __forceinline__ void unit_store(const UnitStage<T> &st, char *sK, cha
     } else {
       const int key = it >> 4, g = it & 15;
       const uint4 v = keep_if(k0 + key < n, st.v[j]);
-      *(uint32_t *)(sV + (4 * g + 0) * ROWV + 4 * key) = v.x;
-      *(uint32_t *)(sV + (4 * g + 1) * ROWV + 4 * key) = v.y;
-      *(uint32_t *)(sV + (4 * g + 2) * ROWV + 4 * key) = v.z;
-      *(uint32_t *)(sV + (4 * g + 3) * ROWV + 4 * key) = v.w;
+      *(float *)(sV + (4 * g + 0) * ROWV + 4 * key) = __uint_as_float(v.x);
+      *(float *)(sV + (4 * g + 1) * ROWV + 4 * key) = __uint_as_float(v.y);
+      *(float *)(sV + (4 * g + 2) * ROWV + 4 * key) = __uint_as_float(v.z);
+      *(float *)(sV + (4 * g + 3) * ROWV + 4 * key) = __uint_as_float(v.w);
     }
   }
   if (lane < 32) {
@@ -924,8 +934,7 @@ __global__ __launch_bounds__(512) void attention_ks_kernel(AttnArgs a) {
       info = f.pi;
       if (nn >= 0) unit_info<T>(f, a.kinfo, base, n, 32 * (wave + QW * nn), lane);
     }
-    // Other lanes' rows: written and read by this wave alone, in order.
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();  // other lanes' rows, written and read by this wave alone
     f32x16 sT = {};
 #pragma unroll
     for (int ks = 0; ks < NKS; ks++)
@@ -984,7 +993,7 @@ __global__ __launch_bounds__(512) void attention_ks_kernel(AttnArgs a) {
         ot[i] = MF::mma(vf, pf, ot[i]);
       }
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();  // the rows read: the next unit, or the partial output, may replace them
     cur = nxt;
     nxt = nn;
   }
