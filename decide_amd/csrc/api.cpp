@@ -226,8 +226,7 @@ bool fold_geometry(const dn_ctx *c) {
 
 bool fold_eligible(const dn_ctx *c, int T) {
   const Config &g = c->cfg;
-  return (c->ln_fold || T <= kFoldSwitchTokens) && c->fold_cs.p && !g.generic &&
-         gemm_ln_fold_ok(g.precision, T, g.hidden, g.inter);
+  return c->ln_fold && c->fold_cs.p && !g.generic && gemm_ln_fold_ok(g.precision, T, g.hidden, g.inter);
 }
 
 size_t fold_bytes_per_token(const dn_ctx *c) { return fold_geometry(c) ? sizeof(float) * 2 : 0; }

@@ -213,9 +213,6 @@ struct dn_ctx {
 
 namespace dnh {
 
-// dn_set_ln_fold applies to forwards of more tokens than this; smaller ones
-// (above the small-M kernels' 128) always fold.
-constexpr int kFoldSwitchTokens = 1024;
 constexpr int kPositions = 65536;  // RoPE table rows: positions are validated / flagged to this range
 
 int fail(dn_ctx *c, int code, const std::string &msg);

@@ -219,11 +219,9 @@ int dn_set_row_tail(dn_ctx *ctx, int min_tokens);
  * i.e. LayerNorm(x).B^T, so the LayerNorm launches (a read of the fp32
  * residual stream each) disappear. The logits move by the bf16 rounding of
  * the operand (x - m) * w instead of the normalised row, the same size of
- * error. on = 0 runs the LayerNorm kernels in forwards (or parts of a
- * two-stream forward) of more than 1024 tokens; smaller ones always fold. The
- * default is on. No
- * counterpart in the reference (forward.go:289-294, :324 normalise, then
- * project). */
+ * error. on = 0 runs the LayerNorm kernels in every forward; the default is
+ * on. No counterpart in the reference (forward.go:289-294, :324 normalise,
+ * then project). */
 int dn_set_ln_fold(dn_ctx *ctx, int on);
 
 /* How the small-M GEMM kernel (batches of at most 128 tokens, 16-bit modes,

@@ -431,18 +431,19 @@ def test_cfg4_full_batch(base, engines):
 
 
 def test_ln_fold_matches_layernorm_kernels(base, engines):
-    """dn_set_ln_fold: bf16 forwards of more than 1024 tokens run attn_norm
+    """dn_set_ln_fold: 16-bit forwards of more than 128 tokens run attn_norm
     and mlp_norm inside the GEMMs around them (the residual GEMM writes the
-    norm's operand bf16((x - m) * w) and per-192-column row statistics; QKV
-    and Wi apply rstd and the mean through column sums of the weighted
-    projection). Against the same forward with the LayerNorm kernels and
-    against the oracle, at the bf16 bar, on batches that take each tile
-    configuration of the folded GEMMs: cfg3's 64 x 512 tokens (256 x 192
-    residual, 256 x 128 QKV / Wi tiles) on one stream and on two, one cfg4
-    sequence (2,816 tokens: 64 x 192 and 128 x 128 tiles), 4,097 and 6,001
-    tokens (256 x 192 residual, 256 x 128 QKV and 128 x 128 Wi tiles, the last
-    256-row tile holding 1 and 113 rows) and 1,025 tokens (the smallest batch
-    that folds; at 1,024 the switch changes nothing, bit for bit). The folded logits are not the unfolded ones (the fold ran).
+    norm's operand (x - m) * w in 16 bits and row statistics over parts of 64
+    columns, 192 above 5,376 tokens; QKV and Wi apply rstd and the mean through
+    column sums of the weighted projection). Against the same forward with the
+    LayerNorm kernels and against the oracle, at the bf16 bar, on batches that
+    take each tile configuration of the folded GEMMs above 1,024 tokens: cfg3's
+    64 x 512 tokens (256 x 192 residual, 256 x 128 QKV / Wi tiles) on one stream
+    and on two, one cfg4 sequence (2,816 tokens: 128 x 128 and 256 x 128 tiles),
+    4,097 tokens (128 x 128 and 192 x 256), 6,001 tokens (128 x 192 residual, 256
+    x 128 QKV and 128 x 128 Wi tiles, the last 256-row tile holding 113 rows) and
+    1,025 tokens (64 x 64 and 128 x 128). The folded logits are not the unfolded
+    ones (the fold ran). At 128 tokens the switch changes nothing, bit for bit.
     fp16 folds the same way (1,025 tokens); the fp32 mode does not fold."""
     from decide_amd.nn import build_sequence
     from decide_amd.synth import config_batch, pack_request
@@ -451,8 +452,8 @@ def test_ln_fold_matches_layernorm_kernels(base, engines):
     eng = engines["bf16"]
     rng = np.random.default_rng(91)
     b1025 = [build_sequence(pack_request(rng, p, [16] * 8, cfg.vocab), 50284, True) for p in (385, 384)]
-    b1024 = [build_sequence(pack_request(rng, 384, [16] * 8, cfg.vocab), 50284, True) for _ in range(2)]
-    assert sum(len(s.ids) for s in b1025) == 1025 and sum(len(s.ids) for s in b1024) == 1024
+    b128 = [build_sequence(pack_request(rng, 32, [16] * 2, cfg.vocab), 50284, True) for _ in range(2)]
+    assert sum(len(s.ids) for s in b1025) == 1025 and sum(len(s.ids) for s in b128) == 128
     b4097 = [build_sequence(pack_request(rng, p, [16] * 8, cfg.vocab), 50284, True) for p in [384] * 7 + [385]]
     b6001 = [build_sequence(pack_request(rng, p, [16] * 8, cfg.vocab), 50284, True) for p in [384] * 11 + [241]]
     assert sum(len(s.ids) for s in b4097) == 4097 and sum(len(s.ids) for s in b6001) == 6001
@@ -478,9 +479,9 @@ def test_ln_fold_matches_layernorm_kernels(base, engines):
                 want = orc.forward([batch[i]])
                 compare(folded[off[i]: off[i + 1]], want, [batch[i]], "bf16")
         eng.set_ln_fold(False)
-        plain = eng.forward(b1024)
+        plain = eng.forward(b128)
         eng.set_ln_fold(True)
-        assert np.array_equal(eng.forward(b1024), plain)
+        assert np.array_equal(eng.forward(b128), plain)
         # fp16 folds as bf16 does (checked at the 16-bit bar against its
         # LayerNorm kernels and the oracle); fp32 does not fold.
         for p in ("fp16", "fp32"):
