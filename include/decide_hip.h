@@ -207,8 +207,9 @@ int dn_set_stream_split(dn_ctx *ctx, int min_tokens);
  * (forward.go:212-243 runs every layer over all tokens, then gathers). */
 int dn_set_row_tail(dn_ctx *ctx, int min_tokens);
 
-/* bf16 and fp16 inference forwards of more than 128 tokens (hidden 768) run
- * attn_norm and mlp_norm folded into the GEMMs around them: the
+/* bf16 inference forwards of more than 128 tokens and fp16 ones of more than
+ * 1,024 (hidden 768) run attn_norm and mlp_norm folded into the GEMMs around
+ * them: the
  * residual GEMM before a LayerNorm (Wo, MlpWo) also writes the norm's operand
  * ((x - m) * w in the operand type) of the new residual row x, with m the row mean of the
  * previous LayerNorm and w the norm weight, and per part of 64 columns (192 in
@@ -219,7 +220,9 @@ int dn_set_row_tail(dn_ctx *ctx, int min_tokens);
  * i.e. LayerNorm(x).B^T, so the LayerNorm launches (a read of the fp32
  * residual stream each) disappear. The logits move by the bf16 rounding of
  * the operand (x - m) * w instead of the normalised row, the same size of
- * error. on = 0 runs the LayerNorm kernels in every forward; the default is
+ * error. In fp16 that operand overflows where a residual value times its norm
+ * weight exceeds 65,504 (the normalised row cannot, at ordinary weights).
+ * on = 0 runs the LayerNorm kernels in every forward; the default is
  * on. No counterpart in the reference (forward.go:289-294, :324 normalise,
  * then project). */
 int dn_set_ln_fold(dn_ctx *ctx, int on);
