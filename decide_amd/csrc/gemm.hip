@@ -22,9 +22,9 @@
 //     (row >> 1) & 7, so the 16 rows read by a quarter-wave fall in distinct
 //     banks (the swizzle is applied on the global side of the DMA).
 //   * Workgroup -> tile order is XCD-aware: consecutive workgroup ids go
-//     round-robin over the 8 XCDs; each XCD owns a contiguous range of the
-//     tiles in row order, so an A panel is read into one XCD's L2 (two at a
-//     range's ends) and B (at most 3.5 MB here) stays in it.
+//     round-robin over the 8 XCDs; while B fits an XCD's 4 MB L2 or little
+//     more, each XCD owns a contiguous range of the tiles in row order, so an A
+//     panel is read into one XCD's L2 (two at a range's ends) and B stays in it.
 //   * The epilogue stages the finished tile through LDS so global stores are
 //     full 16-byte-per-lane rows.
 #include <type_traits>
@@ -110,12 +110,23 @@ __device__ __forceinline__ void lds_read4x16(const char *const (&p)[4], uint4 (&
 // Row order over all workgroups, which ragged row counts took before, spread
 // each A panel over every XCD (3,840 x 768 x 2304, 128 x 128 tiles: 25.9 ->
 // 23.4 us; 3,840 x 2304 x 768: 25.7 -> 24.3 us).
+// A wide and large B would stream through every XCD's L2 for each of its
+// panels: from kRowOrderB bytes and kRowOrderN columns on, row order over all
+// workgroups, where an XCD sees every eighth column tile only (bf16, us, by
+// ranges / in row order: 20,000 x 8192 x 1024, B 16 MB, 396 / 382; 8,192 x 4096
+// x 4096 into fp32, 383 / 342; 20,000 x 4096 x 4096 725 / 675; 20,000 x 8192 x
+// 8192 2,770 / 2,627; 20,000 x 6144 x 1024, B 12 MB, 296 / 287; smaller or
+// narrower the other way or the same: 20,000 x 5248 x 1024, B 10.2 MB, 248 /
+// 259; 20,000 x 1024 x 8192 400 / 533; 20,000 x 2048 x 4096 356 / 355).
+constexpr size_t kRowOrderB = (size_t)12 << 20;
+constexpr int kRowOrderN = 4096;
 template <int BM, int BN>
 struct TileOrder {
   int m0, n0;
-  __device__ __forceinline__ TileOrder(int bid, int tiles_n) {
+  __device__ __forceinline__ TileOrder(int bid, int tiles_n, size_t b_bytes) {
+    const bool by_row = tiles_n * BN >= kRowOrderN && b_bytes >= kRowOrderB;
     const int nt = (int)gridDim.x, q = nt >> 3, r = nt & 7, xcd = bid & 7;
-    const int t = xcd * q + min(xcd, r) + (bid >> 3);
+    const int t = by_row ? bid : xcd * q + min(xcd, r) + (bid >> 3);
     m0 = (t / tiles_n) * BM;
     n0 = (t % tiles_n) * BN;
   }
@@ -239,7 +250,7 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
   const int wm = wave / WGN, wn = wave % WGN;
   const int lr = lane & 31, lh = lane >> 5;
 
-  const TileOrder<BM, BN> to(blockIdx.x, g.N / BN);
+  const TileOrder<BM, BN> to(blockIdx.x, g.N / BN, (size_t)g.N * g.K * sizeof(T));
   const int m0 = to.m0, n0 = to.n0;
   // Folded LayerNorm consumer: thread t < BM takes block row t's statistics
   // and thread t < BN column n0 + t's lcs (loaded here; merged after the

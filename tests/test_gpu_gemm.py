@@ -168,7 +168,9 @@ def test_gemm_16bit_device_store(eng, prec, M, N, K):
     ("bf16", 897, 2304, 128, True), ("fp16", 1793, 2304, 768, True), ("bf16", 3585, 2304, 192, True),
     ("fp16", 2689, 2304, 64, True), ("bf16", 3585, 2176, 768, True), ("fp16", 5376, 2304, 64, True),
     ("bf16", 5377, 2304, 64, True), ("fp16", 7168, 2304, 768, True), ("bf16", 7169, 2304, 192, True),
-    ("bf16", 4097, 128, 768, True)])
+    ("bf16", 4097, 128, 768, True),
+    # the row-ordered tiles of a B of 12 MB and 4,096 columns or more, ragged rows
+    ("bf16", 5001, 6144, 1024, True), ("bf16", 700, 4096, 1536, False)])
 def test_gemm_tile_boundaries(eng, prec, M, N, K, store):
     """Row counts on both sides of each tile rule and K from one stage up
     (fewer stages than the ring holds): every output against float64, at the
