@@ -1322,12 +1322,17 @@ hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
     // path: 203 rows 15.3 / 13.7 / 15.7, 300 rows 20.8 / 22.7 / 20.8, 512 rows
     // 29.5 / 31.2 / 30.7; N = 768: 203 rows 7.4 / 12.0 / 13.2, 512 rows 13.8 /
     // 12.2 / 13.6, 1,472 rows 28.8 / 32.2 / 101.7 on 256 x 128 tiles). Longer K
-    // at two blocks a CU keeps the register path (512 x 768 x 1152: 20.5 / 19.6 /
-    // 17.5).
+    // at two blocks a CU keeps the register path's 64 x 32 tiles while they run
+    // in one round (N = 768, K = 1152, 353 rows 19.8 / 20.1 / 17.5, 600 rows
+    // 20.4 / 21.0 / 17.7; K = 832, 512 rows 15.5 / 15.4 / 14.3; K = 2304, 512
+    // rows 38.6 / 37.1 / 29.7; N = 2304, K = 1152, 160 rows 20.4 / 19.7 / 17.6; N
+    // = 1536, K = 1536, 300 rows 26.5 / 25.6 / 21.8), not in two (N = 2304, K =
+    // 1152, 203 rows 20.7 / 20.2 / 26.2, K = 2304 39.4 / 38.4 / 48.0).
     const int c32 = (a.N / 32) * ((a.M + 31) / 32), c64 = c32 / 2;
     const int r32 = (c32 + kCUs - 1) / kCUs, r64 = (c64 + kCUs - 1) / kCUs;
-    if (r32 == 2 && a.K > 768 && epi == EPI_F32) {
-      hipLaunchKernelGGL((gemm_skinny_kernel<float, 2, 1, EPI_F32, 8>), dim3(a.N / 32, (a.M + 63) / 64), dim3(512), 0, s, a);
+    const dim3 regs(a.N / 32, (a.M + 63) / 64);
+    if (r32 == 2 && a.K > 768 && epi == EPI_F32 && regs.x * regs.y <= kCUs) {
+      hipLaunchKernelGGL((gemm_skinny_kernel<float, 2, 1, EPI_F32, 8>), regs, dim3(512), 0, s, a);
       return hipGetLastError();
     }
     if (2 * r64 <= r32) return launch_skinny_cfg<T, 1, 2, 8>(epi, a, s);
