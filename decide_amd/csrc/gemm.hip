@@ -111,22 +111,25 @@ __device__ __forceinline__ void lds_read4x16(const char *const (&p)[4], uint4 (&
 // each A panel over every XCD (3,840 x 768 x 2304, 128 x 128 tiles: 25.9 ->
 // 23.4 us; 3,840 x 2304 x 768: 25.7 -> 24.3 us).
 // A wide and large B would stream through every XCD's L2 for each of its
-// panels: from kRowOrderB bytes and kRowOrderN columns on, row order over all
-// workgroups, where an XCD sees every eighth column tile only (bf16, us, by
-// ranges / in row order: 20,000 x 8192 x 1024, B 16 MB, 396 / 382; 8,192 x 4096
-// x 4096 into fp32, 383 / 342; 20,000 x 4096 x 4096 725 / 675; 20,000 x 8192 x
-// 8192 2,770 / 2,627; 20,000 x 6144 x 1024, B 12 MB, 296 / 287; smaller or
-// narrower the other way or the same: 20,000 x 5248 x 1024, B 10.2 MB, 248 /
-// 259; 20,000 x 1024 x 8192 400 / 533; 20,000 x 2048 x 4096 356 / 355).
+// panels: from kRowOrderB bytes and kRowOrderN columns on, the grid is one row
+// of tiles after the other (blockIdx.y), whose column tiles go to the XCDs by
+// ranges, so an XCD sees an eighth of B (bf16, us, ranges over the whole grid /
+// this: 20,000 x 8192 x 1024, B 16 MB, 396 / 383; 8,192 x 4096 x 4096 into fp32,
+// 383 / 344; 20,000 x 4096 x 4096 725 / 679; 20,000 x 8192 x 8192 2,770 / 2,590;
+// 20,000 x 6144 x 1024, B 12 MB, 296 / 292; smaller or narrower B in row order
+// lose or gain nothing: 20,000 x 5248 x 1024, B 10.2 MB, 248 / 259; 20,000 x
+// 1024 x 8192 400 / 533; 20,000 x 2048 x 4096 356 / 355).
+// The order is the grid's shape: as a word of the arguments, or computed from
+// N and K, it cost every launch 0.1 to 0.25 us (a 512-token forward 932 -> 937
+// and 938 -> 960 us).
 constexpr size_t kRowOrderB = (size_t)12 << 20;
 constexpr int kRowOrderN = 4096;
 template <int BM, int BN>
 struct TileOrder {
   int m0, n0;
-  __device__ __forceinline__ TileOrder(int bid, int tiles_n, size_t b_bytes) {
-    const bool by_row = tiles_n * BN >= kRowOrderN && b_bytes >= kRowOrderB;
-    const int nt = (int)gridDim.x, q = nt >> 3, r = nt & 7, xcd = bid & 7;
-    const int t = by_row ? bid : xcd * q + min(xcd, r) + (bid >> 3);
+  __device__ __forceinline__ explicit TileOrder(int tiles_n) {
+    const int bid = blockIdx.x, nt = (int)gridDim.x, q = nt >> 3, r = nt & 7, xcd = bid & 7;
+    const int t = (int)blockIdx.y * nt + xcd * q + min(xcd, r) + (bid >> 3);
     m0 = (t / tiles_n) * BM;
     n0 = (t % tiles_n) * BN;
   }
@@ -250,7 +253,7 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
   const int wm = wave / WGN, wn = wave % WGN;
   const int lr = lane & 31, lh = lane >> 5;
 
-  const TileOrder<BM, BN> to(blockIdx.x, g.N / BN, (size_t)g.N * g.K * sizeof(T));
+  const TileOrder<BM, BN> to(g.N / BN);
   const int m0 = to.m0, n0 = to.n0;
   // Folded LayerNorm consumer: thread t < BM takes block row t's statistics
   // and thread t < BN column n0 + t's lcs (loaded here; merged after the
@@ -266,11 +269,11 @@ __device__ __forceinline__ void gemm_nt_tile(const GemmArgs &g, const LnFold &lf
     if (threadIdx.x < BM) ln_fold_load<NP>(g, lf, m0 + (int)threadIdx.x, ln_v, ln_mp);
     if (threadIdx.x < BN) ln_c = lf.lcs[n0 + threadIdx.x];
   }
-  // Split-K: blockIdx.y takes K elements [y*K, (y+1)*K) of A and B and writes
+  // Split-K: blockIdx.z takes K elements [z*K, (z+1)*K) of A and B and writes
   // its own partial output.
-  const size_t koff = (size_t)blockIdx.y * g.K;
+  const size_t koff = (size_t)blockIdx.z * g.K;
   const T *gA = (const T *)g.A + koff, *gB = (const T *)g.B + koff;
-  char *gC = (char *)g.C + (size_t)blockIdx.y * g.c_split * (F32OUT ? 4 : sizeof(T));
+  char *gC = (char *)g.C + (size_t)blockIdx.z * g.c_split * (F32OUT ? 4 : sizeof(T));
 
   // DMA sources: load i of this wave fills tile rows RPI*(wave + NW*i) .. +RPI-1;
   // lane l writes row RPI*(wave+NW*i) + l/CPR, LDS chunk slot l%CPR, which
@@ -829,7 +832,9 @@ struct Tile {
 template <class T, class C, int EPI, int PC = 0>
 hipError_t launch_tile(const GemmArgs &a, hipStream_t s, const LnFold *ln = nullptr, int splits = 1) {
   if (a.N % C::BN || a.K % (C::RB / (int)sizeof(T))) return hipErrorInvalidValue;
-  const dim3 grid(C::count(a), splits), block(64 * C::WGM * C::WGN);
+  const int tiles_n = a.N / C::BN, tiles_m = C::count(a) / tiles_n;
+  const bool rows = a.N >= kRowOrderN && (size_t)a.N * a.K * sizeof(T) >= kRowOrderB && tiles_m <= 65535;
+  const dim3 grid(rows ? tiles_n : tiles_n * tiles_m, rows ? tiles_m : 1, splits), block(64 * C::WGM * C::WGN);
   if constexpr (EPI >= EPI_F32_LN)
     hipLaunchKernelGGL((gemm_nt_ln_kernel<T, C::BM, C::BN, C::RB, C::NSTAGE, EPI, C::WPE, C::WGM, C::WGN, C::PF, PC>),
                        grid, block, 0, s, a, *ln);
