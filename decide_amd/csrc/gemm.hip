@@ -1517,8 +1517,10 @@ hipError_t launch_f32(const GemmArgs &a, hipStream_t s) {
 //   192 x 256          3,840      21.8 / 23.7  (128 x 128, 64-byte stages: 26.1 / 26.5)
 //                      5,376      24.0 / 25.6  (256 x 128, two per CU: 27.9 / 28.9)
 //   256 x 256          7,000      30.4 / 31.0  (256 x 128, two per CU: 32.2 / 34.2)
-// At 64 x 64 the line lies at 160 workgroups: 252 of them (448 rows) took
-// 7.2 us against 6.8 for 128 x 64.
+// At 64 x 64 the line lies at 224 workgroups (64 x 64 / 128 x 64: N = 2304, 317
+// rows 6.1 / 6.5, 381 rows, 216 of them, 6.4 / 6.6, 448 rows, 252, 7.2 / 6.8; K =
+// 1152, 381 rows 7.5 / 7.8; N = 1536, 573 rows 6.3 / 6.6; N = 768, 957 rows 5.7 /
+// 6.5, K = 2304 10.1 / 12.7).
 typedef Tile<64, 64, 128, 5, 1, 2, 1, true> S64x64;
 typedef Tile<128, 64, 128, 4, 1, 4, 1, true> S128x64;
 typedef Tile<128, 128, 128, 4, 1, 4, 2, true> S128x128;
@@ -1533,7 +1535,7 @@ template <class T, int EPI, int PC = 0>
 hipError_t launch_store(const GemmArgs &a, hipStream_t s, const LnFold *ln = nullptr) {
   constexpr bool gated = EPI == EPI_GEGLU || EPI == EPI_GEGLU_KEEP || EPI == EPI_GEGLU_LN;
   if constexpr (PC != kLnPartWide) {
-    if (S64x64::count(a) <= 160) return launch_tile<T, S64x64, EPI, PC>(a, s, ln);
+    if (S64x64::count(a) <= kCUs * 7 / 8) return launch_tile<T, S64x64, EPI, PC>(a, s, ln);
     if (S128x64::count(a) <= kCUs) return launch_tile<T, S128x64, EPI, PC>(a, s, ln);
     if (S128x128::count(a) <= kCUs) return launch_tile<T, S128x128, EPI, PC>(a, s, ln);
     if (S192x128::count(a) <= kCUs) return launch_tile<T, S192x128, EPI, PC>(a, s, ln);
