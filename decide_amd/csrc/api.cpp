@@ -420,7 +420,7 @@ struct Pass {
 // Whether attention splits a query chunk's keys over waves: batches of few work
 // items (attention.hip has both sides' times).
 bool attn_key_split(const Config &g, int nwork) {
-  return !g.generic && nwork <= (prec16(g.precision) ? kKeySplitItems16 : kKeySplitItems32);
+  return !g.generic && (long long)nwork * g.heads <= (prec16(g.precision) ? kKeySplitPairs16 : kKeySplitPairs32);
 }
 
 // Token info, 32-token chunk summaries, attention tile classes of both layer
@@ -977,9 +977,11 @@ int split_point(int nseq, const int32_t *seq_len, int T_total, int *first_tokens
   return cut;
 }
 
-// Smallest part of a split forward: above it every GEMM of a part runs the
-// tiled kernels of the single-stream forward (small M runs the small-M
-// kernels, whose summation order differs), so the logits are identical.
+// Smallest part of a split forward. Above it every 16-bit GEMM of a part sums
+// in the order of the single-stream forward's (at most 128 rows run the small-M
+// kernel, which does not), and the fold, its statistics' parts, the key-split
+// attention and the fp32 GEMM's kernel are chosen by the whole batch: the
+// logits are identical.
 constexpr int kMinPartTokens = 1025;
 
 int forward_split(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_ids, const int32_t *d_pos,
@@ -1009,8 +1011,8 @@ int forward_split(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_
   if (rc) return rc;
   rc = ensure_rope(c);
   if (rc) return rc;
-  // Each part's GEMMs fold when the part has more than 1024 tokens, as the
-  // single-stream forward of the whole batch does (kMinPartTokens).
+  // The parts (kMinPartTokens or more) fold as the single-stream forward of the
+  // whole batch does.
   const bool fold = fold_eligible(c, std::min(acc, T_total - acc));
   if (fold) {
     rc = ensure_fold_buffers(c, T);

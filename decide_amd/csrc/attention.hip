@@ -691,8 +691,13 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
 // 22-layer forwards, keys split against the tile walk: bf16 4 x 128 tokens
 // 886 against 979 us, 1,024 tokens 1,262 / 1,337, 4 x 256 tokens (8 work items)
 // 1,159 / 1,161, 8 x 184 (16 items) 1,390 / 1,284; fp32 8 x 184 11.18 / 11.32
-// ms, 2,044 tokens (16 items) 12.3 / 13.1 ms, 4 x 1024 17.0 / 17.1 ms: hence the
-// lines at 8 and 16 items.
+// ms, 2,044 tokens (16 items) 12.3 / 13.1 ms, 4 x 1024 17.0 / 17.1 ms. That is at
+// 12 heads; the grid is items x heads, and so are the lines, 96 and 192 pairs
+// (walk / split, us: bf16, 4 heads, 24 items 1,009 / 978 and 886 / 891, 48 items
+// 1,279 / 1,368; 8 heads, 12 items 1,082 / 1,055, 20 items 1,249 / 1,333; 16
+// heads, 6 items 1,648 / 1,615, 10 items 1,881 / 1,987; fp32, 4 heads, 48 items
+// 3,636 / 3,545; 8 heads, 24 items 5,284 / 5,194 and 4,795 / 4,838, 32 items
+// 6,217 / 6,364; 16 heads, 12 items 11,064 / 10,975, 16 items 10,437 / 10,755).
 
 // Orders a wave's own LDS accesses where lanes read what others wrote (or
 // overwrite what others read). The hardware runs a wave's LDS operations in
@@ -872,7 +877,7 @@ __global__ __launch_bounds__(512) void attention_ks_kernel(AttnArgs a) {
   const int u0 = wave + QW * lane;
   const uint32_t code = a.codes[(size_t)wi * ATTN_MAXKT + min(u0 >> 1, ATTN_MAXKT - 1)];
   // The chunk's Q rows, rotated once for every wave: thread t takes two
-  // element pairs (i, i + 32) of row t / 16 (or four of row t / 8).
+  // element pairs (i, i + 32) of row t / 16.
   constexpr int QE = 32 * 32 / (64 * QW);  // pairs per thread
   const int qr = tid / (32 / QE), qi = tid % (32 / QE) * QE, qq = min(q0 + qr, n - 1);
   const T *qrow = qkv + (size_t)(base + qq) * ld + head * D + qi;
@@ -1012,7 +1017,7 @@ __global__ __launch_bounds__(512) void attention_ks_kernel(AttnArgs a) {
       *(float4 *)(sO + lr * ROWO + i * 32 + 8 * g + 4 * lh) =
           make_float4(ot[i][4 * g], ot[i][4 * g + 1], ot[i][4 * g + 2], ot[i][4 * g + 3]);
   __syncthreads();
-  constexpr int DPT = 32 * D / (64 * QW);  // outputs per thread: 4 or 8 of one query
+  constexpr int DPT = 32 * D / (64 * QW);  // outputs per thread, of one query
   const int mq = tid / (D / DPT), d0 = tid % (D / DPT) * DPT;
   if (q0 + mq >= n) return;
   float m = -INFINITY;

@@ -93,9 +93,10 @@ struct TrainState {
 // the parts into the residual stream.
 constexpr int kSmallSplitMaxTokens = 128, kSmallSplitParts = 6, kSplitMaxWorkgroups = 256;
 
-// Batches of at most this many 128-query work items split the attention's keys
-// over waves (attention_ks_kernel, with the measurements at 12 heads).
-constexpr int kKeySplitItems16 = 8, kKeySplitItems32 = 16;
+// Batches of at most this many pairs of a 128-query work item and a head split
+// the attention's keys over waves (attention_ks_kernel has the measurements):
+// at 12 heads 8 work items in 16 bits and 16 in fp32.
+constexpr int kKeySplitPairs16 = 96, kKeySplitPairs32 = 192;
 
 // Device memory one forward works in beyond the weights: the activations,
 // the batch layout and the head's scratch. forward_core takes it from the
