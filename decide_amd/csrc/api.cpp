@@ -408,8 +408,7 @@ struct Pass {
   // split forward.
   bool fold = false;
   int ln_cols = kLnPartWide;
-  // Attention with the keys split over waves (attn_key_split), by the whole
-  // batch too.
+  // Attention with the keys split over waves (attn_key_split).
   bool key_split = false;
   int rows = 0;  // the whole batch's tokens
   Workspace w;
@@ -420,7 +419,9 @@ struct Pass {
 // Whether attention splits a query chunk's keys over waves: batches of few work
 // items (attention.hip has both sides' times).
 bool attn_key_split(const Config &g, int nwork) {
-  return !g.generic && (long long)nwork * g.heads <= (prec16(g.precision) ? kKeySplitPairs16 : kKeySplitPairs32);
+  const bool half = prec16(g.precision);
+  return !g.generic && nwork <= (half ? kKeySplitItems16 : kKeySplitItems32) &&
+         nwork * g.heads <= (half ? kKeySplitPairs16 : kKeySplitPairs32);
 }
 
 // Token info, 32-token chunk summaries, attention tile classes of both layer
@@ -979,10 +980,13 @@ int split_point(int nseq, const int32_t *seq_len, int T_total, int *first_tokens
 
 // Smallest part of a split forward. Above it every 16-bit GEMM of a part sums
 // in the order of the single-stream forward's (at most 128 rows run the small-M
-// kernel, which does not), and the fold, its statistics' parts, the key-split
-// attention and the fp32 GEMM's kernel are chosen by the whole batch: the
-// logits are identical.
+// kernel, which does not), the fold, its statistics' parts and the fp32 GEMM's
+// kernel are chosen by the whole batch, and attention's keys are never split:
+// the logits are identical.
 constexpr int kMinPartTokens = 1025;
+static_assert(2 * ((kMinPartTokens + ATTN_QUERIES - 1) / ATTN_QUERIES) > kKeySplitItems32 &&
+                  kKeySplitItems32 >= kKeySplitItems16,
+              "a split forward has more work items than the key-split attention takes");
 
 int forward_split(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_ids, const int32_t *d_pos,
                   const int32_t *d_opt, int R, const int32_t *d_row_tok, float *d_logits, int T_total, int cut,
@@ -1049,15 +1053,9 @@ int forward_split(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_
     ps[k].pos = d_pos + t0;
     ps[k].opt = d_opt ? d_opt + t0 : nullptr;
     ps[k].s = st[k];
-  }
-  const bool key_split = attn_key_split(g, ps[0].w.nwork + ps[1].w.nwork);
-  for (Pass &p : ps) {
-    p.key_split = key_split;
-    p.rows = T_total;
-    p.wide_global = !key_split;
-  }
-  for (Pass &p : ps) {
-    rc = enqueue_prologue(c, p, p.w.h, p.w.xn, nullptr, nullptr);
+    ps[k].rows = T_total;
+    ps[k].wide_global = true;
+    rc = enqueue_prologue(c, ps[k], ps[k].w.h, ps[k].w.xn, nullptr, nullptr);
     if (rc) return rc;
   }
   const bool rows_tail = tail_on_rows(c, T_total, R, false);

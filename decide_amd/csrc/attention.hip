@@ -691,13 +691,11 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
 // 22-layer forwards, keys split against the tile walk: bf16 4 x 128 tokens
 // 886 against 979 us, 1,024 tokens 1,262 / 1,337, 4 x 256 tokens (8 work items)
 // 1,159 / 1,161, 8 x 184 (16 items) 1,390 / 1,284; fp32 8 x 184 11.18 / 11.32
-// ms, 2,044 tokens (16 items) 12.3 / 13.1 ms, 4 x 1024 17.0 / 17.1 ms. That is at
-// 12 heads; the grid is items x heads, and so are the lines, 96 and 192 pairs
-// (walk / split, us: bf16, 4 heads, 24 items 1,009 / 978 and 886 / 891, 48 items
-// 1,279 / 1,368; 8 heads, 12 items 1,082 / 1,055, 20 items 1,249 / 1,333; 16
-// heads, 6 items 1,648 / 1,615, 10 items 1,881 / 1,987; fp32, 4 heads, 48 items
-// 3,636 / 3,545; 8 heads, 24 items 5,284 / 5,194 and 4,795 / 4,838, 32 items
-// 6,217 / 6,364; 16 heads, 12 items 11,064 / 10,975, 16 items 10,437 / 10,755).
+// ms, 2,044 tokens (16 items) 12.3 / 13.1 ms, 4 x 1024 17.0 / 17.1 ms: hence the
+// lines at 8 and 16 items. That is at 12 heads; the grid is items x heads, and
+// the lines are at most 96 and 192 pairs (walk / split, us: 16 heads, bf16, 6
+// items 1,648 / 1,615, 10 items 1,881 / 1,987; fp32, 12 items 11,064 / 10,975,
+// 16 items 10,437 / 10,755; 8 heads, fp32, 24 items 4,795 / 4,838).
 
 // Orders a wave's own LDS accesses where lanes read what others wrote (or
 // overwrite what others read). The hardware runs a wave's LDS operations in

@@ -93,9 +93,12 @@ struct TrainState {
 // the parts into the residual stream.
 constexpr int kSmallSplitMaxTokens = 128, kSmallSplitParts = 6, kSplitMaxWorkgroups = 256;
 
-// Batches of at most this many pairs of a 128-query work item and a head split
-// the attention's keys over waves (attention_ks_kernel has the measurements):
-// at 12 heads 8 work items in 16 bits and 16 in fp32.
+// Batches of at most this many 128-query work items, and pairs of an item and a
+// head (the grid is items x heads), split the attention's keys over waves
+// (attention_ks_kernel has the measurements). Fewer heads do not raise the
+// items: from 2,048 tokens the last layer's attention may run on the option
+// rows alone, which walks the tiles, and is then the full layer's bit for bit.
+constexpr int kKeySplitItems16 = 8, kKeySplitItems32 = 16;
 constexpr int kKeySplitPairs16 = 96, kKeySplitPairs32 = 192;
 
 // Device memory one forward works in beyond the weights: the activations,
