@@ -26,13 +26,16 @@
 // Key tiles (64 keys) are visited in a list of the tiles some wave needs; the
 // next tile's K, V and RoPE factors are loaded into registers while the
 // current one is computed. K is rotated and stored key-major; V is stored
-// transposed (d-major) with two keys packed per 32-bit word, its rows' chunks
-// swizzled. Q, K and V are all read whole rows at a time: eight lanes to a
-// row's 128 bytes, since the CU's address unit takes about a cycle per line a
-// load instruction touches (Q by MFMA fragment and V by key before: 64 x 512
-// tokens sliding-window layers 78.8 -> 69.5 us, 8 x ~2,800 tokens 69.5 -> 61.7;
-// global layers, bound by the softmax, 110 -> 108.5 and 249 -> 256 us; the
-// same values and sums).
+// transposed (d-major) with two keys packed per 32-bit word. K always, and Q
+// and V where that pays, are read whole rows at a time: eight lanes to a row's
+// 128 bytes, since the CU's address unit takes about a cycle per line a load
+// instruction touches. Q by MFMA fragment and V by key against both by rows,
+// 16 bits: 64 x 512 tokens, sliding-window layers 79 -> 71 us, 8 x 2,800
+// 59 -> 56. Layers bound by the softmax gain little, and lose at two query tiles
+// per wave: global layers in 256-query items, 8 x 2,800 tokens 294 -> 309 us,
+// 4 x 7,000 696 -> 736 (64 x 512 109 -> 107); the option rows' layer 94 -> 100
+// and 222 -> 232. So the 256-query items keep the former loads, the option rows
+// V's.
 #include "common.hpp"
 
 namespace {
@@ -113,7 +116,7 @@ __device__ __forceinline__ void key_info_load(KeyInfo<T, R> &f, const int *kinfo
 }
 
 // Loads one key tile (keys k0 .. k0+63) into registers; NT threads, R = 256/NT.
-template <class T, int R>
+template <class T, int R, bool VR>
 __device__ __forceinline__ void stage_load(Staging<T, R> &st, const T *qkv, int ld, int H, int head, int base, int n,
                                            int k0, const float *cos_t, const float *sin_t,
                                            const KeyInfo<T, R> &ki, int tid) {
@@ -142,8 +145,8 @@ __device__ __forceinline__ void stage_load(Staging<T, R> &st, const T *qkv, int 
       st.s_hi[j] = *(const float4 *)(sin_t + p * 32 + 8 * c + 4);
     }
 #pragma unroll
-    for (int j = 0; j < R; j++) {  // V: key pair p = it / 8, d group g = it % 8: eight lanes read a whole row
-      const int it = tid + NT * j, p = it >> 3, g = it & 7;
+    for (int j = 0; j < R; j++) {  // V: key pair p and d group g; VR: eight lanes read a whole row
+      const int it = tid + NT * j, p = VR ? it >> 3 : it & 31, g = VR ? it & 7 : it >> 5;
       const int k = k0 + 2 * p;
       st.v0[j] = *(const uint4 *)(qkv + (size_t)(unsigned)(base + min(k, n - 1)) * (unsigned)ld + 2 * H + head * D + 8 * g);
       st.v1[j] = *(const uint4 *)(qkv + (size_t)(unsigned)(base + min(k + 1, n - 1)) * (unsigned)ld + 2 * H + head * D +
@@ -184,7 +187,7 @@ __device__ __forceinline__ void rope1(float &a, float &b, float c, float s) {
   b = y;
 }
 
-template <class T, int R>
+template <class T, int R, bool VR>
 __device__ __forceinline__ void stage_store(const Staging<T, R> &st, char *sK, char *sV, int *sKo, int *sKw,
                                             int half_window, int tid, int ROWK, int ROWV) {
   constexpr int NT = 256 / R;
@@ -219,19 +222,19 @@ __device__ __forceinline__ void stage_store(const Staging<T, R> &st, char *sK, c
     // contiguous 16-byte read, at chunk vt_chunk of the row.
 #pragma unroll
     for (int j = 0; j < R; j++) {
-      const int it = tid + NT * j, p = it >> 3, g = it & 7;
+      const int it = tid + NT * j, p = VR ? it >> 3 : it & 31, g = VR ? it & 7 : it >> 5;
       const int lp = p & 7, q4 = lp >> 1;
       const int pw = (p & ~7) + ((((q4 & 1) << 1) | (q4 >> 1)) << 1) + (lp & 1);
-      int vx = (((pw >> 2) ^ g) << 4) + 4 * (pw & 3);
-      asm volatile("" : "+v"(vx));  // the eight store addresses are made from it here, not kept in registers
+      int vx = VR ? (((pw >> 2) ^ g) << 4) + 4 * (pw & 3) : 4 * pw;
+      if constexpr (VR) asm volatile("" : "+v"(vx));  // the eight store addresses are made from it here, not kept in registers
       const uint4 v0 = keep_if((st.valid >> (8 + j)) & 1, st.v0[j]), v1 = keep_if((st.valid >> (16 + j)) & 1, st.v1[j]);
       const uint32_t va[4] = {v0.x, v0.y, v0.z, v0.w};
       const uint32_t vb[4] = {v1.x, v1.y, v1.z, v1.w};
 #pragma unroll
       for (int w = 0; w < 4; w++) {
         // Byte permutes: (va & 0xffff) | (vb << 16) and (va >> 16) | (vb & 0xffff0000).
-        *(uint32_t *)(sV + (8 * g + 2 * w) * ROWV + (vx ^ (32 * w))) = __builtin_amdgcn_perm(vb[w], va[w], 0x05040100u);
-        *(uint32_t *)(sV + (8 * g + 2 * w + 1) * ROWV + (vx ^ (32 * w + 16))) =
+        *(uint32_t *)(sV + (8 * g + 2 * w) * ROWV + (VR ? vx ^ (32 * w) : vx)) = __builtin_amdgcn_perm(vb[w], va[w], 0x05040100u);
+        *(uint32_t *)(sV + (8 * g + 2 * w + 1) * ROWV + (VR ? vx ^ (32 * w + 16) : vx)) =
             __builtin_amdgcn_perm(vb[w], va[w], 0x07060302u);
       }
     }
@@ -286,8 +289,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
   using MF = Mfma<T>;
   typedef typename MF::frag frag;
   constexpr int ROWK = D * sizeof(T) + 16;  // K tile row bytes (key-major)
-  // V^T tile row bytes (d-major): 16-bit rows are swizzled (vt_chunk).
-  constexpr int ROWV = sizeof(T) == 2 ? KTILE * 2 : KTILE * 4 + 16;
+  // V read by whole rows (VR) or by key, with its tile's row bytes (d-major,
+  // swizzled by vt_chunk or padded).
+  constexpr bool VR = sizeof(T) == 2 && QT == 1 && !LIST;
+  constexpr int ROWV = VR ? KTILE * 2 : KTILE * (int)sizeof(T) + 16;
   // 16-bit: two buffers, tile t is computed from one while tile t+1 is stored
   // into the other, with one barrier per tile. fp32 (the validation mode,
   // twice the bytes) keeps one buffer and a second barrier.
@@ -354,14 +359,16 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
   const bool stager = tid < 256;
   if (kt < nkt && stager) {
     key_info_load<T, R>(ki, a.kinfo, base, n, kt * KTILE, tid);
-    stage_load<T, R>(st, qkv, ld, H, head, base, n, kt * KTILE, a.cos_t, a.sin_t, ki, tid);
+    stage_load<T, R, VR>(st, qkv, ld, H, head, base, n, kt * KTILE, a.cos_t, a.sin_t, ki, tid);
   }
 
-  // The work item's Q rows, rotated into LDS: thread items (row, 16-byte chunk
-  // pair (c, c + CPQ)), whole rows per load instruction. (Each wave loading
-  // its own MFMA fragments touched 32 rows with every instruction, which the
-  // CU's address unit serialises, and so did V's loads by key: together most
-  // of its work.)
+  // The work item's Q rows. QLDS: rotated into LDS by thread items (row,
+  // 16-byte chunk pair (c, c + CPQ)), whole rows per load instruction. (Each
+  // wave loading its own MFMA fragments touches 32 rows with every instruction,
+  // which the CU's address unit serialises, and so do V's loads by key:
+  // together most of its work in short key walks.) The wide 16-bit work items
+  // load fragments: they walk many tiles, and the registers that the compiler
+  // then has there are worth more (above).
   constexpr int NKS = D / MF::KSTEP;
   constexpr int EPC = 16 / (int)sizeof(T), CPQ = 32 / EPC, QI = QROWS * CPQ / NT;
   auto q_token = [&](int idx, int &r) {  // token (in the sequence) and list row of query idx
@@ -373,53 +380,57 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
       return min(q0 + idx, n - 1);
     }
   };
-  constexpr int QB = QI > 4 ? 4 : QI;  // items in flight
-  static_assert(QI % QB == 0, "Q items");
+  constexpr bool QLDS = QT == 1 || sizeof(T) == 4;
+  frag qf[QT][NKS];  // Q^T operands (B operand: column = query, k = head dim)
+  if constexpr (QLDS) {
+    constexpr int QB = QI > 4 ? 4 : QI;  // items in flight
+    static_assert(QI % QB == 0, "Q items");
 #pragma clang loop unroll(disable)
-  for (int j0 = 0; j0 < QI; j0 += QB) {
-    uint4 ql[QB], qh[QB];
-    int qp[QB];
+    for (int j0 = 0; j0 < QI; j0 += QB) {
+      uint4 ql[QB], qh[QB];
+      int qp[QB];
 #pragma unroll
-    for (int j = 0; j < QB; j++) {
-      const int it = tid + NT * (j0 + j), c = it % CPQ;
-      int r = 0;
-      const int qq = q_token(it / CPQ, r);
-      const T *row = LIST ? (const T *)a.q_rows + (size_t)r * H + head * D : qkv + (size_t)(base + qq) * ld + head * D;
-      qp[j] = a.kinfo[base + qq] & 0xffff;
-      ql[j] = *(const uint4 *)(row + EPC * c);
-      qh[j] = *(const uint4 *)(row + 32 + EPC * c);
-    }
-    typedef float FV __attribute__((ext_vector_type(EPC)));
-    FV qc[QB], qs[QB];
-#pragma unroll
-    for (int j = 0; j < QB; j++) {
-      const size_t o = (size_t)qp[j] * 32 + EPC * ((tid + NT * (j0 + j)) % CPQ);
-      qc[j] = *(const FV *)(a.cos_t + o);
-      qs[j] = *(const FV *)(a.sin_t + o);
-    }
-#pragma unroll
-    for (int j = 0; j < QB; j++) {
-      const int it = tid + NT * (j0 + j), row = it / CPQ, c = it % CPQ;
-      const uint32_t wl[4] = {ql[j].x, ql[j].y, ql[j].z, ql[j].w}, wh[4] = {qh[j].x, qh[j].y, qh[j].z, qh[j].w};
-      uint32_t ol[4], oh[4];
-#pragma unroll
-      for (int w = 0; w < 4; w++) {
-        if constexpr (sizeof(T) == 2) {
-          float a0 = lo16<T>(wl[w]), a1 = hi16<T>(wl[w]), b0 = lo16<T>(wh[w]), b1 = hi16<T>(wh[w]);
-          rope1(a0, b0, qc[j][2 * w], qs[j][2 * w]);
-          rope1(a1, b1, qc[j][2 * w + 1], qs[j][2 * w + 1]);
-          ol[w] = pack16<T>(a0, a1);
-          oh[w] = pack16<T>(b0, b1);
-        } else {
-          float x = __uint_as_float(wl[w]), y = __uint_as_float(wh[w]);
-          rope1(x, y, qc[j][w], qs[j][w]);
-          ol[w] = __float_as_uint(x);
-          oh[w] = __float_as_uint(y);
-        }
+      for (int j = 0; j < QB; j++) {
+        const int it = tid + NT * (j0 + j), c = it % CPQ;
+        int r = 0;
+        const int qq = q_token(it / CPQ, r);
+        const T *row = LIST ? (const T *)a.q_rows + (size_t)r * H + head * D : qkv + (size_t)(base + qq) * ld + head * D;
+        qp[j] = a.kinfo[base + qq] & 0xffff;
+        ql[j] = *(const uint4 *)(row + EPC * c);
+        qh[j] = *(const uint4 *)(row + 32 + EPC * c);
       }
-      const int sw = row & (2 * CPQ - 1);  // chunk swizzle: reads of 32 rows' equal chunks spread over the banks
-      *(uint4 *)(smem + row * ROWQ + ((c ^ sw) << 4)) = make_uint4(ol[0], ol[1], ol[2], ol[3]);
-      *(uint4 *)(smem + row * ROWQ + (((c + CPQ) ^ sw) << 4)) = make_uint4(oh[0], oh[1], oh[2], oh[3]);
+      typedef float FV __attribute__((ext_vector_type(EPC)));
+      FV qc[QB], qs[QB];
+#pragma unroll
+      for (int j = 0; j < QB; j++) {
+        const size_t o = (size_t)qp[j] * 32 + EPC * ((tid + NT * (j0 + j)) % CPQ);
+        qc[j] = *(const FV *)(a.cos_t + o);
+        qs[j] = *(const FV *)(a.sin_t + o);
+      }
+#pragma unroll
+      for (int j = 0; j < QB; j++) {
+        const int it = tid + NT * (j0 + j), row = it / CPQ, c = it % CPQ;
+        const uint32_t wl[4] = {ql[j].x, ql[j].y, ql[j].z, ql[j].w}, wh[4] = {qh[j].x, qh[j].y, qh[j].z, qh[j].w};
+        uint32_t ol[4], oh[4];
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+          if constexpr (sizeof(T) == 2) {
+            float a0 = lo16<T>(wl[w]), a1 = hi16<T>(wl[w]), b0 = lo16<T>(wh[w]), b1 = hi16<T>(wh[w]);
+            rope1(a0, b0, qc[j][2 * w], qs[j][2 * w]);
+            rope1(a1, b1, qc[j][2 * w + 1], qs[j][2 * w + 1]);
+            ol[w] = pack16<T>(a0, a1);
+            oh[w] = pack16<T>(b0, b1);
+          } else {
+            float x = __uint_as_float(wl[w]), y = __uint_as_float(wh[w]);
+            rope1(x, y, qc[j][w], qs[j][w]);
+            ol[w] = __float_as_uint(x);
+            oh[w] = __float_as_uint(y);
+          }
+        }
+        const int sw = row & (2 * CPQ - 1);  // chunk swizzle: reads of 32 rows' equal chunks spread over the banks
+        *(uint4 *)(smem + row * ROWQ + ((c ^ sw) << 4)) = make_uint4(ol[0], ol[1], ol[2], ol[3]);
+        *(uint4 *)(smem + row * ROWQ + (((c + CPQ) ^ sw) << 4)) = make_uint4(oh[0], oh[1], oh[2], oh[3]);
+      }
     }
   }
   // This lane's queries (one per query tile).
@@ -433,6 +444,22 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
     const int qinfo = a.kinfo[base + q_token(idx, qrow_r[t])];
     qopt[t] = (qinfo >> 16) - 1;
     qpos[t] = qinfo & 0xffff;
+    if constexpr (!QLDS) {
+      const T *qrow = qkv + (size_t)(base + min(q0 + idx, n - 1)) * ld + head * D + lh * MF::SLOTS;
+      const size_t o = (size_t)qpos[t] * 32 + lh * MF::SLOTS;
+      const float *cq = a.cos_t + o, *sq = a.sin_t + o;
+#pragma unroll
+      for (int ks = 0; ks < NKS; ks++) qf[t][ks] = *(const frag *)(qrow + ks * MF::KSTEP);
+#pragma unroll
+      for (int ks = 0; ks < NKS / 2; ks++)
+#pragma unroll
+        for (int u = 0; u < MF::SLOTS; u++) {
+          float x = (float)qf[t][ks][u], y = (float)qf[t][ks + NKS / 2][u];
+          rope1(x, y, cq[ks * MF::KSTEP + u], sq[ks * MF::KSTEP + u]);
+          qf[t][ks][u] = to_elem<T>(x);
+          qf[t][ks + NKS / 2][u] = to_elem<T>(y);
+        }
+    }
   }
 
   f32x16 ot[QT][2];
@@ -448,18 +475,19 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
   }
 
   __syncthreads();  // sCode and the Q rows visible
-  frag qf[QT][NKS];  // Q^T operands (B operand: column = query, k = head dim)
+  if constexpr (QLDS) {
 #pragma unroll
-  for (int t = 0; t < QT; t++) {
-    const int row = (wave * QT + t) * 32 + lr;
+    for (int t = 0; t < QT; t++) {
+      const int row = (wave * QT + t) * 32 + lr;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ks++) {
-      const int e = ks * MF::KSTEP + lh * MF::SLOTS;
-      qf[t][ks] = *(const frag *)(smem + row * ROWQ + (((e / EPC) ^ (row & (2 * CPQ - 1))) << 4) +
-                                  e % EPC * (int)sizeof(T));
+      for (int ks = 0; ks < NKS; ks++) {
+        const int e = ks * MF::KSTEP + lh * MF::SLOTS;
+        qf[t][ks] = *(const frag *)(smem + row * ROWQ + (((e / EPC) ^ (row & (2 * CPQ - 1))) << 4) +
+                                    e % EPC * (int)sizeof(T));
+      }
     }
+    __syncthreads();  // the Q rows read: the buffers may be filled
   }
-  __syncthreads();  // the Q rows read: the buffers may be filled
   auto next_tile = [&](int kt) {
     while (kt < nkt && sCode[kt] == 0) kt++;
     return kt;
@@ -472,12 +500,12 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
   // the key info of the one after that, one barrier.
   int kn = nkt, kn_next = nkt, b = 0;
   if (kt < nkt) {
-    if (stager) stage_store<T, R>(st, smem, smem + KTILE * ROWK, sKo[0], sKw[0], a.half_window, tid, ROWK, ROWV);
+    if (stager) stage_store<T, R, VR>(st, smem, smem + KTILE * ROWK, sKo[0], sKw[0], a.half_window, tid, ROWK, ROWV);
     kn = next_tile(kt + 1);
     if (kn < nkt) {
       if (stager) {
         key_info_load<T, R>(ki, a.kinfo, base, n, kn * KTILE, tid);
-        stage_load<T, R>(st, qkv, ld, H, head, base, n, kn * KTILE, a.cos_t, a.sin_t, ki, tid);
+        stage_load<T, R, VR>(st, qkv, ld, H, head, base, n, kn * KTILE, a.cos_t, a.sin_t, ki, tid);
       }
       kn_next = next_tile(kn + 1);
       if (kn_next < nkt && stager) key_info_load<T, R>(ki, a.kinfo, base, n, kn_next * KTILE, tid);
@@ -588,8 +616,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
       // of tile i on lane half lh is key 32*i + 8*((r%16)/4) + 4*lh + r%4. A V
       // fragment read from LDS feeds every query tile that needs its half.
       constexpr int NPV = KTILE / MF::KSTEP;
-      int vsw = vt_chunk(lr, lh) << 4;
-      if constexpr (sizeof(T) == 2) asm volatile("" : "+v"(vsw));  // as vx in stage_store
+      int vsw = VR ? vt_chunk(lr, lh) << 4 : 16 * lh;
+      if constexpr (VR) asm volatile("" : "+v"(vsw));  // as vx in stage_store
 #pragma unroll
       for (int ks = 0; ks < NPV; ks++) {
         const int half = ks / (NPV / 2);
@@ -613,7 +641,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
           const char *vrow = sVb + (i * 32 + lr) * ROWV;
           frag vf;
           if constexpr (sizeof(T) == 2) {
-            vf = *(const frag *)(vrow + (vsw ^ (32 * ks) ^ (64 * i)));  // keys 16ks + {4lh..4lh+3, 8+4lh..8+4lh+3}
+            vf = *(const frag *)(vrow + (VR ? vsw ^ (32 * ks) ^ (64 * i) : vsw + 32 * ks));  // keys 16ks + {4lh..4lh+3, 8+4lh..8+4lh+3}
           } else {
             const int r = ks & 15;
             const int key = 32 * (ks >> 4) + 8 * (r >> 2) + 4 * lh + (r & 3);
@@ -629,10 +657,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && QW == ATTN_WAVES ? 2 : QT =
     if (kn < nkt) {
       const int nb = NBUF == 2 ? b ^ 1 : 0;
       if constexpr (NBUF == 1) __syncthreads();  // every wave is done with the one buffer
-      if (stager) stage_store<T, R>(st, smem + nb * KV, smem + nb * KV + KTILE * ROWK, sKo[nb], sKw[nb], a.half_window, tid, ROWK, ROWV);
+      if (stager) stage_store<T, R, VR>(st, smem + nb * KV, smem + nb * KV + KTILE * ROWK, sKo[nb], sKw[nb], a.half_window, tid, ROWK, ROWV);
       kn2 = kn_next;  // == next_tile(kn + 1); ki holds its key info
       if (kn2 < nkt) {
-        if (stager) stage_load<T, R>(st, qkv, ld, H, head, base, n, kn2 * KTILE, a.cos_t, a.sin_t, ki, tid);
+        if (stager) stage_load<T, R, VR>(st, qkv, ld, H, head, base, n, kn2 * KTILE, a.cos_t, a.sin_t, ki, tid);
         kn_next = next_tile(kn2 + 1);
         if (kn_next < nkt && stager) key_info_load<T, R>(ki, a.kinfo, base, n, kn_next * KTILE, tid);
       }
