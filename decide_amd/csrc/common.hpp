@@ -307,7 +307,9 @@ bool gemm_epi_ok(int precision, int epi, int M);
 // Weight-gradient GEMM into fp32 C (M x N, ldc = N; added to C when
 // a.accumulate, else stored): `splits` (1..16) partial products, each over a.K /
 // splits of K (a.K % (splits * 64) == 0), summed in split order. partial holds
-// splits * M * N floats for the shapes whose splits run as workgroups.
+// gemm_wgrad_partial floats: splits * M * N for the shapes whose splits run as
+// workgroups, else none.
+size_t gemm_wgrad_partial(int precision, int M, int N, int splits);
 hipError_t launch_gemm_wgrad(int precision, const GemmArgs &a, int splits, float *partial, hipStream_t s);
 // Small M (<= 128) split-K on the whole-K kernel, no reduction: workgroup z of
 // a tile multiplies K elements [z*K/splits, (z+1)*K/splits) and stores its

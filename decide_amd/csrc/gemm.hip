@@ -1640,17 +1640,27 @@ hipError_t launch_gemm(int precision, int epi, const GemmArgs &a, hipStream_t s,
 // operand bytes per output of 64 x 128 tiles, and no partial outputs to write
 // and read; dWqkv at 3840 tokens: 108 workgroups for 25 us against 216 for 21
 // us; the backward of a step of 32 x 384 tokens in four micro-batches over 22
-// layers 22.7 -> 21.7 ms). Fewer than 32 such tiles (hidden sizes below 768) would leave the side
-// stream behind the chain and stay split over workgroups.
+// layers 22.7 -> 21.7 ms). Fewer than 32 such tiles (hidden sizes below 768)
+// would leave the side stream behind the chain and stay split over workgroups.
+static bool wgrad_walks_splits(int precision, int M, int N) {
+  GemmArgs a{};
+  a.M = M;
+  a.N = N;
+  return precision == PREC_BF16 && F128x128::count(a) >= 32;
+}
+
+size_t gemm_wgrad_partial(int precision, int M, int N, int splits) {
+  return splits == 1 || wgrad_walks_splits(precision, M, N) ? 0 : (size_t)splits * M * N;
+}
+
 hipError_t launch_gemm_wgrad(int precision, const GemmArgs &a0, int splits, float *partial, hipStream_t s) {
   if (a0.M <= 0) return hipSuccess;
   if (precision == PREC_F16) return hipErrorInvalidValue;  // training only
   if (splits < 1 || splits > 16 || a0.K % (splits * 64) != 0 || a0.N % 128 != 0) return hipErrorInvalidValue;
-  const bool bf = precision == PREC_BF16;
   GemmArgs a = a0;
   a.ldc = a0.N;
   a.n_store = a0.N;
-  if (bf && F128x128::count(a) >= 32) {
+  if (wgrad_walks_splits(precision, a.M, a.N)) {
     typedef F128x128 C;
     if (splits == 1) return launch_tile<bf16, C, EPI_F32>(a, s);
     hipLaunchKernelGGL((gemm_nt_seg_kernel<bf16, C::BM, C::BN, C::RB, C::NSTAGE, C::WPE, C::WGM, C::WGN>),
@@ -1662,8 +1672,9 @@ hipError_t launch_gemm_wgrad(int precision, const GemmArgs &a0, int splits, floa
   a.C = partial;
   a.accumulate = 0;
   a.c_split = (size_t)a0.M * a0.N;
-  const hipError_t e = bf ? launch_tile<bf16, F64x128, EPI_F32>(a, s, nullptr, splits)
-                          : launch_tile<float, Tile<128, 128, 128, 3, 1, 2, 2>, EPI_F32>(a, s, nullptr, splits);
+  const hipError_t e = precision == PREC_BF16
+                           ? launch_tile<bf16, F64x128, EPI_F32>(a, s, nullptr, splits)
+                           : launch_tile<float, Tile<128, 128, 128, 3, 1, 2, 2>, EPI_F32>(a, s, nullptr, splits);
   if (e != hipSuccess) return e;
   const size_t n = (size_t)a0.M * a0.N;
   hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, partial, splits,

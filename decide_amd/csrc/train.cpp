@@ -247,10 +247,11 @@ int backward_impl(dn_ctx *c, const float *dlogits) {
     HIPCHK(c, "hipEventRecord", hipEventRecord(tr.ev_trans[q], tr.side));
   }
   HIPCHK(c, "hipMalloc", ensure(tr.dsum, 4 * (size_t)T * g.heads));
-  // split-K partials: weight gradients (<= 16 splits) and input gradients (<= 4 splits of T x max(H, I))
-  HIPCHK(c, "hipMalloc", ensure(tr.part, 4 * std::max((size_t)16 * std::max({(size_t)3 * H * H, (size_t)2 * I * H,
-                                                                             (size_t)H * I}),
-                                                        (size_t)4 * T * std::max(H, I))));
+  // Split-K partials of the weight gradients that write them, at the most splits.
+  size_t part = 0;
+  for (const auto &mn : {std::pair<int, int>{H, I}, {2 * I, H}, {H, H}, {3 * H, H}})
+    part = std::max(part, gemm_wgrad_partial(prec, mn.first, mn.second, 16));
+  if (part) HIPCHK(c, "hipMalloc", ensure(tr.part, sizeof(float) * part));
   // LayerNorm weight-gradient partials: one slot per (layer parity, norm);
   // their column sums run on the weight-gradient stream.
   const size_t lnslot = (size_t)ln_bwd_blocks(std::max(T, R)) * H;

@@ -458,6 +458,35 @@ def test_backward_bit_equal_by_rows(tokens):
         assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(a), name
 
 
+def test_backward_workspace_without_unused_partials():
+    """bf16 weight gradients at 768 columns sum their token splits in registers and
+    write no partial outputs: the first step's workspace holds none (16 x 3 x 768^2
+    floats, 108 MiB, would). What it does hold at 64 tokens is some 56 buffers of a
+    2 MiB page each."""
+    import torch
+
+    from decide_amd.nn import Config, build_sequence
+    from decide_amd.train import TrainEngine
+
+    cfg = Config(hidden=768, intermediate=1152, heads=12, layers=1, vocab=1000, half_window=64,
+                 layer_types=["full_attention"])
+    w = weights_for(cfg, seed=3, std=0.02)
+    ids = np.random.default_rng(3).integers(3, 990, size=64).astype(np.int32)
+    ids[[20, 40]] = 999
+    batch = [build_sequence(ids, 999, independent=True)]
+    used = []
+    for _ in range(2):  # the first engine loads the kernels
+        with TrainEngine(cfg, w, precision="bf16") as eng:
+            torch.cuda.synchronize()
+            free = torch.cuda.mem_get_info()[0]
+            eng.forward(batch)
+            eng.backward(np.array([0.5, -0.5], np.float32))
+            eng.grad_norm()
+            used.append(free - torch.cuda.mem_get_info()[0])
+    print(f"case: workspace of the first step {used[1] / 2**20:.1f} MB", flush=True)
+    assert used[1] < 160 << 20
+
+
 def test_backward_full_size_deterministic_and_linear():
     """At the trainer's micro-batch size (10 examples x 384 tokens under the
     4000-token budget, ModernBERT-base, bf16, embeddings trained): a second
