@@ -264,7 +264,21 @@ int ensure_fold_cs(dn_ctx *c, hipStream_t s) {
   }
   const int rc = flush();
   if (rc) return rc;
-  c->fold_gen = c->wgen;
+  // Recorded into a graph, the sums are there from its first replay on.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIPCHK(c, "hipStreamIsCapturing", hipStreamIsCapturing(s, &cap));
+  if (cap == hipStreamCaptureStatusNone) c->fold_gen = c->wgen;
+  return DN_OK;
+}
+
+// New weights: once a forward has folded, its sums are rebuilt with the weights
+// and not by the next forward, so a captured forward's replays have them too.
+int weights_changed(dn_ctx *c) {
+  c->wgen++;
+  if (!c->fold_gen) return DN_OK;
+  const int rc = ensure_fold_cs(c, c->stream);
+  if (rc) return rc;
+  HIPCHK(c, "hipStreamSynchronize", hipStreamSynchronize(c->stream));
   return DN_OK;
 }
 
@@ -1288,8 +1302,7 @@ int upload_f32(dn_ctx *c, TensorSlot &t, const float *data, int64_t n) {
     HIPCHK(c, "hipMemcpy", hipMemcpy(t.buf.p, data, bytes, hipMemcpyHostToDevice));
   }
   t.set = true;
-  c->wgen++;
-  return DN_OK;
+  return weights_changed(c);
 }
 // Validation (forward.go:142-196) and staging of a host batch.
 int stage_batch(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *ids, const int32_t *pos,
@@ -1582,8 +1595,7 @@ static int upload_bf16_impl(dn_ctx *c, const char *name, const uint16_t *bits, i
     HIPCHK(c, "hipMemcpy", hipMemcpy(t->buf.p, bits, (size_t)n * 2, hipMemcpyHostToDevice));
   }
   t->set = true;
-  c->wgen++;
-  return DN_OK;
+  return weights_changed(c);
 }
 
 int dn_upload_tensor_bf16(dn_ctx *c, const char *name, const uint16_t *bits, int64_t n) {

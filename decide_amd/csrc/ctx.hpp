@@ -255,10 +255,12 @@ int ensure_rope(dn_ctx *c);
 void set_work2(Workspace &w, int nwork2);
 int ensure_err_flag(dn_ctx *c);
 // Folded LayerNorm: whether a forward of T tokens on this context takes it,
-// and the column sums brought up to date with the weights (a kernel per
-// projection on stream s when they changed; no allocation).
+// and the column sums brought up to date with the weights (one launch on
+// stream s when they changed; no allocation). weights_changed: after every
+// change of a weight.
 bool fold_eligible(const dn_ctx *c, int T);
 int ensure_fold_cs(dn_ctx *c, hipStream_t s);
+int weights_changed(dn_ctx *c);
 // Bytes of the folded LayerNorm's per-token statistics (0 when the context
 // never folds).
 size_t fold_bytes_per_token(const dn_ctx *c);

@@ -178,3 +178,57 @@ def test_key_split_line_follows_heads(prec, tokens):
     oracle.set_workers(WORKERS)
     with Engine(cfg, w, precision=prec) as eng:
         compare(eng.forward(batch), oracle.OracleModel(cfg, w).forward(batch), batch, prec)
+
+
+def test_captured_forward_follows_new_weights():
+    """A captured dn_forward_device of a batch that folds the LayerNorm (300 tokens
+    in bf16): every replay gives the eager logits, and after an upload of other
+    weights the replays give theirs, the folded column sums among them. The
+    program's own eager forwards run between the replays."""
+    import torch
+
+    from decide_amd import Engine
+    from decide_amd.nn import Config, flatten, row_tokens
+    from decide_amd.synth import random_weights
+
+    cfg = Config(hidden=768, intermediate=1152, heads=12, layers=3, vocab=50368, half_window=64,
+                 layer_types=["full_attention", "sliding_attention", "full_attention"])
+    w, w2 = random_weights(cfg, seed=1), random_weights(cfg, seed=2)
+    batch = batch_with_total(300, cfg.vocab, np.random.default_rng(5))
+    seq_len, ids, pos, opt, _, _ = flatten(batch)
+    rows = row_tokens(batch)
+    ids, pos, opt, rows = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (ids, pos, opt, rows))
+    out = torch.zeros(len(rows), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with Engine(cfg, w, precision="bf16") as eng:
+        eng.set_stream(s.cuda_stream)
+
+        def forward():
+            eng.forward_device(seq_len, ids.data_ptr(), pos.data_ptr(), opt.data_ptr(), len(rows), rows.data_ptr(),
+                               out.data_ptr())
+
+        def eager():
+            forward()
+            eng.synchronize()
+            return out.cpu().numpy()
+
+        def replay():
+            out.fill_(7.0)
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            return out.cpu().numpy()
+
+        first = eager()
+        with torch.cuda.graph(g, stream=s):
+            forward()
+        for _ in range(3):
+            assert np.array_equal(replay(), first)
+            assert np.array_equal(eager(), first)
+        eng.load(w2)
+        second = [replay() for _ in range(2)]
+        want = eager()
+        assert not np.array_equal(want, first)
+        for got in second + [replay()]:
+            assert np.array_equal(got, want)
