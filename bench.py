@@ -386,10 +386,10 @@ def train_bench(args) -> int:
     probe, nprobe = eng.read_probe_backward()
     eng.set_probe(-1)
     # Roofline kernel: layer 1's QKV weight-gradient GEMM (dWqkv += dqkv^T . n1,
-    # 2 * 2304 * 768 flop per token; 2304 x 768 output in 64 x 128 tiles, run
-    # unsplit over the tokens), timed with HIP events on
-    # the weight-gradient stream; it shares the GPU with the main stream's
-    # kernels while it runs.
+    # 2 * 2304 * 768 flop per token; 2304 x 768 output in 128 x 128 tiles,
+    # run unsplit over the tokens), timed with HIP events on the
+    # weight-gradient stream; it shares the GPU with the main stream's kernels
+    # while it runs.
     qkv_flop = 2.0 * (3 * H) * H * sum(len(s.ids) for s in ex) * args.steps
     wg_s = probe["wgrad_qkv"] * 1e-3
     dg_s = probe["dgrad_qkv"] * 1e-3
@@ -570,7 +570,8 @@ def main() -> int:
     ap.add_argument("--row-tail", type=int, default=2048, metavar="TOKENS",
                     help="dn_set_row_tail: batches of at least TOKENS finish the last layer on the option rows (0: off)")
     ap.add_argument("--ln-fold", type=int, default=1, choices=(0, 1),
-                    help="dn_set_ln_fold: bf16 and fp16 batches of more than 1024 tokens run the LayerNorms inside the GEMMs")
+                    help="dn_set_ln_fold: bf16 batches of more than 128 tokens and fp16 ones of more than 1024 run the "
+                         "LayerNorms inside the GEMMs")
     ap.add_argument("--copy-calibration", type=int, default=0, metavar="MIB",
                     help="run one device copy of MIB MiB first (reference kernel for HBM counters)")
     ap.add_argument("--tokenizer", action="store_true",
@@ -685,24 +686,27 @@ def main() -> int:
     # Per-launch roofline views. The kernel with the largest share of GPU
     # time at cfg3 is the fp32-residual GEMM (Wo and MlpWo share its symbol):
     # algorithmic bytes per launch are A, the weights, and the fp32 residual
-    # read and written (T x H each way); with the folded LayerNorm (16-bit,
-    # T > 1024) also the next norm's 16-bit operand (T x H) and the row
-    # statistics (8 bytes per row and 192 columns) it writes. By the roofline
-    # model it is bound by HBM (its bytes take longer at 8 TB/s than its flops
-    # at the MFMA peak).
-    fold = bool(args.ln_fold) and prec in ("bf16", "fp16") and T > 1024
+    # read and written (T x H each way); with the folded LayerNorm (bf16 above
+    # 128 tokens, fp16 above 1024) also the next norm's 16-bit operand (T x H)
+    # and the row statistics (8 bytes per row and part of 192 columns, 64 up to
+    # 5,376 tokens) it writes. By the roofline model it is bound by HBM (its
+    # bytes take longer at 8 TB/s than its flops at the MFMA peak).
+    fold = bool(args.ln_fold) and T > {"bf16": 128, "fp16": 1024}.get(prec, T)
     res_s = (avg["gemm_wo"] + avg["gemm_mlpwo"]) * 1e-3
     res_bytes = esz * (T * H + H * H) + esz * (T * I + H * I) + 2 * 2 * 4 * T * H
     if fold:
-        res_bytes += 2 * (esz * T * H + 8 * T * (H // 192))
+        res_bytes += 2 * (esz * T * H + 8 * T * (H // (64 if T <= 5376 else 192)))
     res_flop = 2.0 * T * H * (H + I)
     wi_flop = 2.0 * T * (2 * I) * H
     wi_bytes = esz * (T * H + 2 * I * H + T * I)
     wi_s = avg["gemm_wi"] * 1e-3
     traffic = read_traffic(args.config, prec, fold)
-    res_name = (f"gemm_nt_kernel<{tname},256,192,128,2,EPI_F32_LN,2,4,2> (Wo and MlpWo + fp32 residual + the next "
-                "LayerNorm's operand and statistics)" if fold else
-                f"gemm_nt_kernel<{tname},256,192,128,2,EPI_F32,2,4,2> (Wo and MlpWo + fp32 residual)")
+    # The tiles are those of more than 8,192 tokens (16 bits); smaller batches take others.
+    res_tile, wi_tile = ((",256,192,128,2", ",2,4,2"), (",256,128,64,3", ",2,2,2")) if T > 8192 and prec != "fp32" else \
+        (("", ""), ("", ""))
+    res_name = (f"gemm_nt_ln_kernel<{tname}{res_tile[0]},EPI_F32_LN{res_tile[1]}> (Wo and MlpWo + fp32 residual + the "
+                "next LayerNorm's operand and statistics)" if fold else
+                f"gemm_nt_kernel<{tname}{res_tile[0]},EPI_F32{res_tile[1]}> (Wo and MlpWo + fp32 residual)")
     if hbm_bound:
         # small M (cfg2, cfg5): the skinny kernel streams the weights; the Wi
         # launch (the largest weight matrix) is the line
@@ -760,7 +764,7 @@ def main() -> int:
         result["projection_gemm_frac_attainable"] = round(gemm_tflops / attain["changing_operands_tflops"], 4)
     if not hbm_bound:
         result["roofline_wi_gemm"] = {
-            "kernel": f"gemm_nt_kernel<{tname},256,128,64,3,{'EPI_GEGLU_LN' if fold else 'EPI_GEGLU'},2,2,2> "
+            "kernel": f"gemm_nt{'_ln' if fold else ''}_kernel<{tname}{wi_tile[0]},EPI_GEGLU{'_LN' if fold else ''}{wi_tile[1]}> "
                       f"(Wi projection + fused GeGLU{' + folded mlp_norm' if fold else ''}), layer %d"
                       % args.probe_layer,
             "bound": "mfma", "achieved": round(wi_flop / wi_s / 1e12, 2), "peak": PEAK[prec] / 1e12,
@@ -966,7 +970,7 @@ def extra_configs(eng, cfg, dev, stream, args) -> dict:
 # 32768): the residual GEMMs (N = 768) and the Wi GEMM (N = 2 x 1152).
 ROOF_TILES = {"residual": [256, 192, 128, 2, 0, 2, 4, 2], "wi": [256, 128, 64, 3, 2, 2, 2, 2],
               "qkv": [256, 128, 64, 3, 1, 2, 2, 2]}
-# With the folded LayerNorm (the default 16-bit forward above 1024 tokens) the
+# With the folded LayerNorm (the default 16-bit forward above 1024 tokens at least) the
 # same tiles run the EPI_F32_LN / EPI_GEGLU_LN / EPI_STORE_LN epilogues.
 FOLD_EPI = {"residual": 5, "wi": 7, "qkv": 6}
 

@@ -213,10 +213,8 @@ int upload_layout(dn_ctx *c, const HostLayout &hl, const Workspace &w, int nseq,
   return DN_OK;
 }
 
-// The context's own workspace: layout arrays (re-uploaded only when the batch
-// layout changes) and activation buffers for T tokens and R rows.
-// Folded LayerNorm: attn_norm and mlp_norm of the large-batch bf16 forward
-// run inside the GEMMs around them (LnFold, the EPI_*_LN forms): the residual GEMM
+// Folded LayerNorm: attn_norm and mlp_norm of a 16-bit forward run inside the
+// GEMMs around them (LnFold, the EPI_*_LN forms; gemm_ln_fold_ok): the residual GEMM
 // before the norm writes its operand and row statistics, the GEMM after it
 // applies the row and column terms, and the LayerNorm launch disappears.
 bool fold_geometry(const dn_ctx *c) {
@@ -288,6 +286,8 @@ int ensure_fold_buffers(dn_ctx *c, size_t T) {
   return DN_OK;
 }
 
+// The context's own workspace: layout arrays (re-uploaded only when the batch
+// layout changes) and activation buffers for T tokens and R rows.
 int ctx_workspace(dn_ctx *c, int nseq, const int32_t *seq_len, int R, Workspace *w) {
   std::vector<int> len(seq_len, seq_len + nseq);
   const bool same = len == c->lay_len && c->d_seq_off.p;

@@ -289,7 +289,8 @@ enum { EPI_F32 = 0, EPI_STORE = 1, EPI_GEGLU = 2, EPI_GEGLU_KEEP = 3, EPI_GEGLU_
 enum { EPI_F32_LN = 5, EPI_STORE_LN = 6, EPI_GEGLU_LN = 7 };
 // The folded LayerNorm's row width, and the columns per statistics part
 // written by EPI_F32_LN (LnFold::lparts tells which): narrow for forwards of
-// up to kLnNarrowTokens tokens.
+// up to kLnNarrowTokens tokens, whose one-round tiles are 64 and 128 columns
+// wide (launch_fold).
 constexpr int kLnHidden = 768, kLnPartNarrow = 64, kLnPartWide = 192, kLnNarrowTokens = 5376;
 // Whether the folded LayerNorm runs for a 16-bit model of this geometry at M
 // rows (the configurations launch_gemm tiles for EPI_*_LN).

@@ -113,7 +113,7 @@ struct Workspace {
   // [kSmallSplitParts x T x H] split-K partial products of the residual
   // GEMMs for batches of at most kSmallSplitMaxTokens tokens; null otherwise.
   float *part = nullptr;
-  // Folded LayerNorm (bf16 / fp16, more than 128 tokens): the row means of a
+  // Folded LayerNorm (fold_eligible): the row means of a
   // layer's attn_norm and mlp_norm ([T] each); null: no fold.
   float *lmean1 = nullptr, *lmean2 = nullptr;
   int *seq_off = nullptr, *seq_len = nullptr, *chunk_off = nullptr, *first = nullptr;
@@ -180,7 +180,7 @@ struct dn_ctx {
   // Folded LayerNorm (dn_set_ln_fold): the column sums of the LayerNorm-
   // weighted QKV and Wi weights per layer ([L x (3H + 2I)] floats, allocated
   // by dn_set_config), rebuilt when the weights' generation (bumped by every
-  // upload and optimizer step) has moved; the forwards' statistics buffers.
+  // upload and optimizer step) has moved; the forwards' row means.
   DevBuf fold_cs, fold_mean;
   uint64_t wgen = 1, fold_gen = 0;
   bool ln_fold = true;

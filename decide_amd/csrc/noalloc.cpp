@@ -8,7 +8,7 @@
 // kScratchBytes. The call makes no hipMalloc / hipFree and uses no
 // allocating library routine; the RoPE tables, the error flag and the
 // folded LayerNorm's column-sum array come from set-up (dn_set_config; the
-// column sums are refilled by a kernel when the weights have changed).
+// column sums are refilled by one launch when the weights have changed).
 //
 // Every call on a GPU shares that GPU's array and it keeps the last call's
 // contents: calls that overlap on one GPU (two contexts, two streams) race.

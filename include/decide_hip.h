@@ -201,8 +201,9 @@ int dn_set_stream_split(dn_ctx *ctx, int min_tokens);
  * attention output and residual rows are gathered, and Wo, mlp_norm, Wi and
  * MlpWo run on R rows instead of T. Every step after attention is row-wise and
  * the scorer head reads only those rows, so the logits are those of the full
- * layer up to the summation order of the smaller GEMMs' kernels. 0 turns it
- * off; the default is 2048. While the kernel probe times the last layer
+ * layer up to the summation order of the smaller GEMMs' kernels (and, where
+ * min_tokens is set below 1025, of the attention that splits a small batch's
+ * keys over waves). 0 turns it off; the default is 2048. While the kernel probe times the last layer
  * (dn_set_probe) forwards run the full layer. No counterpart in the reference
  * (forward.go:212-243 runs every layer over all tokens, then gathers). */
 int dn_set_row_tail(dn_ctx *ctx, int min_tokens);
