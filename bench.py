@@ -700,7 +700,7 @@ def main() -> int:
     wi_flop = 2.0 * T * (2 * I) * H
     wi_bytes = esz * (T * H + 2 * I * H + T * I)
     wi_s = avg["gemm_wi"] * 1e-3
-    traffic = read_traffic(args.config, prec, fold)
+    traffic = read_traffic(args.config, prec, fold) if args.nseq is None else {}
     # The tiles are those of more than 8,192 tokens (16 bits); smaller batches take others.
     res_tile, wi_tile = ((",256,192,128,2", ",2,4,2"), (",256,128,64,3", ",2,2,2")) if T > 8192 and prec != "fp32" else \
         (("", ""), ("", ""))

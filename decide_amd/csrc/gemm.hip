@@ -22,9 +22,12 @@
 //     (row >> 1) & 7, so the 16 rows read by a quarter-wave fall in distinct
 //     banks (the swizzle is applied on the global side of the DMA).
 //   * Workgroup -> tile order is XCD-aware: consecutive workgroup ids go
-//     round-robin over the 8 XCDs; while B fits an XCD's 4 MB L2 or little
-//     more, each XCD owns a contiguous range of the tiles in row order, so an A
-//     panel is read into one XCD's L2 (two at a range's ends) and B stays in it.
+//     round-robin over the 8 XCDs; up to a B of 12 MB each XCD owns a
+//     contiguous range of the tiles in row order, so an A panel is read into
+//     one XCD's L2 (two at a range's ends). A B of up to ~2 MB stays there too;
+//     a larger one is read again for every few panels, out of the memory-side
+//     cache (32,768 x 2304 x 768: 293 MB fetched against 224 with the N tiles
+//     in groups of 2 MB of B, both 142 to 144 us).
 //   * The epilogue stages the finished tile through LDS so global stores are
 //     full 16-byte-per-lane rows.
 #include <type_traits>
