@@ -1520,6 +1520,9 @@ hipError_t launch_f32(const GemmArgs &a, hipStream_t s) {
 //   192 x 256          3,840      21.8 / 23.7  (128 x 128, 64-byte stages: 26.1 / 26.5)
 //                      5,376      24.0 / 25.6  (256 x 128, two per CU: 27.9 / 28.9)
 //   256 x 256          7,000      30.4 / 31.0  (256 x 128, two per CU: 32.2 / 34.2)
+// N = 768, store, K = 768 / 2304: 192 x 256 at 16,000 rows 23.2 / 55.2 (256 x 256
+// 24.1 / 60.5, 128 x 128 with 64-byte stages 27.3 / 76.2), 256 x 256 at 21,000 rows
+// 28.5 / 67.0 (35.8 / 93.2).
 // At 64 x 64 the line lies at 224 workgroups (64 x 64 / 128 x 64: N = 2304, 317
 // rows 6.1 / 6.5, 381 rows, 216 of them, 6.4 / 6.6, 448 rows, 252, 7.2 / 6.8; K =
 // 1152, 381 rows 7.5 / 7.8; N = 1536, 573 rows 6.3 / 6.6; N = 768, 957 rows 5.7 /
