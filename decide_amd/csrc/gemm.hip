@@ -1329,19 +1329,29 @@ hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
     // not add any (K = 768, N = 2304, us, 32 x 32 / 32 x 64 / the register
     // path: 203 rows 15.3 / 13.7 / 15.7, 300 rows 20.8 / 22.7 / 20.8, 512 rows
     // 29.5 / 31.2 / 30.7; N = 768: 203 rows 7.4 / 12.0 / 13.2, 512 rows 13.8 /
-    // 12.2 / 13.6, 1,472 rows 28.8 / 32.2 / 101.7 on 256 x 128 tiles). Longer K
-    // at two blocks a CU keeps the register path's 64 x 32 tiles while they run
-    // in one round (N = 768, K = 1152, 353 rows 19.8 / 20.1 / 17.5, 600 rows
-    // 20.4 / 21.0 / 17.7; K = 832, 512 rows 15.5 / 15.4 / 14.3; K = 2304, 512
-    // rows 38.6 / 37.1 / 29.7; N = 2304, K = 1152, 160 rows 20.4 / 19.7 / 17.6; N
-    // = 1536, K = 1536, 300 rows 26.5 / 25.6 / 21.8), not in two (N = 2304, K =
-    // 1152, 203 rows 20.7 / 20.2 / 26.2, K = 2304 39.4 / 38.4 / 48.0).
+    // 12.2 / 13.6, 1,472 rows 28.8 / 32.2 / 101.7 on 256 x 128 tiles).
+    // Longer K past one round: workgroups that share a CU cover each other's
+    // loads, and the operands go straight into registers, on 64 x 32 tiles where
+    // those take half the rounds, else 32 x 32 (us, 32 x 32 and 32 x 64 through
+    // LDS / 32 x 32 and 64 x 32 in registers: 512 x 768 x 1152 20.8, 20.2 / 20.1,
+    // 17.8; 203 x 2304 x 1152 20.7, 20.2 / 20.2, 26.1; 1,000 x 768 x 1152 30.2,
+    // 35.4 / 29.1, 33.5; 1,000 x 1024 x 2304 77.7, 70.8 / 67.7, 58.2; 777 x 2304 x
+    // 2304 142, 129 / 125, 114; 900 x 768 x 4096 102, 116 / 89, 95), at K = 1024
+    // only in one round of the 64 x 32 ones (512 x 1024 18.6, 16.9 / 18.3, 16.6;
+    // 1,300 x 1024 44.8, 43.1 / 45.6, 46.1).
     const int c32 = (a.N / 32) * ((a.M + 31) / 32), c64 = c32 / 2;
     const int r32 = (c32 + kCUs - 1) / kCUs, r64 = (c64 + kCUs - 1) / kCUs;
-    const dim3 regs(a.N / 32, (a.M + 63) / 64);
-    if (r32 == 2 && a.K > 768 && epi == EPI_F32 && regs.x * regs.y <= kCUs) {
-      hipLaunchKernelGGL((gemm_skinny_kernel<float, 2, 1, EPI_F32, 8>), regs, dim3(512), 0, s, a);
-      return hipGetLastError();
+    if (epi == EPI_F32 && a.K > 768 && r32 > 1) {
+      const dim3 tall(a.N / 32, (a.M + 63) / 64), square(a.N / 32, (a.M + 31) / 32);
+      const int rtall = ((int)(tall.x * tall.y) + kCUs - 1) / kCUs;
+      if (2 * rtall <= r32 && (rtall == 1 || a.K >= 1152)) {
+        hipLaunchKernelGGL((gemm_skinny_kernel<float, 2, 1, EPI_F32, 8>), tall, dim3(512), 0, s, a);
+        return hipGetLastError();
+      }
+      if (a.K >= 1152) {
+        hipLaunchKernelGGL((gemm_skinny_kernel<float, 1, 1, EPI_F32, 8>), square, dim3(512), 0, s, a);
+        return hipGetLastError();
+      }
     }
     if (2 * r64 <= r32) return launch_skinny_cfg<T, 1, 2, 8>(epi, a, s);
   }
@@ -1602,7 +1612,8 @@ hipError_t launch_gemm16(int epi, const GemmArgs &a, hipStream_t s, const LnFold
 // 128 tiles, of which a round takes about as long as 20 rounds of 32 x 32 ones
 // on the 256 CUs (K = 768, N = 2304: 1,472 rows 70 against 104 us, 2,048 rows
 // 95 / 105, 3,000 rows 135 / 105, 4,000 rows 178 / 205; N = 768, 4,000 rows 64 /
-// 104). The two sum in different orders, so the parts of a two-stream forward
+// 104), for longer K 18 (K = 1152, 1,700 rows 130 / 149, 2,200 rows 163 / 151; K =
+// 1536, 2,200 rows 204 / 197). The two sum in different orders, so the parts of a two-stream forward
 // choose by the whole batch's rows.
 bool f32_small_tiles(int epi, const GemmArgs &a) {
   if (epi == EPI_GEGLU_BWD) return false;
@@ -1610,7 +1621,7 @@ bool f32_small_tiles(int epi, const GemmArgs &a) {
   const long long M = a.rows ? a.rows : a.M;
   const long long r32 = ((M + 31) / 32 * (a.N / 32) + kCUs - 1) / kCUs;
   const long long rt = ((M + 255) / 256 * (a.N / 128) + kCUs - 1) / kCUs;
-  return M <= 1024 || r32 <= 20 * rt;
+  return M <= 1024 || r32 <= (a.K > 768 ? 18 : 20) * rt;
 }
 
 template <class C>

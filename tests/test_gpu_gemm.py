@@ -199,7 +199,8 @@ def test_gemm_tile_boundaries(eng, prec, M, N, K, store):
 
 
 @pytest.mark.parametrize("M,N,K", [(129, 2304, 32), (203, 2304, 768), (160, 2304, 1152), (203, 2304, 1152),
-                                   (641, 768, 1152), (340, 768, 768), (352, 768, 768),
+                                   (641, 768, 1152), (777, 1024, 2304), (1000, 768, 1216), (650, 1024, 1120),
+                                   (1700, 2304, 1152), (1825, 2304, 1152), (340, 768, 768), (352, 768, 768),
                                    (512, 768, 1152), (1025, 768, 1152), (1500, 128, 96), (2049, 2304, 768),
                                    (3000, 2304, 768)])
 def test_gemm_f32_device_tiles(eng, M, N, K):
