@@ -424,7 +424,7 @@ struct Pass {
   int ln_cols = kLnPartWide;
   // Attention with the keys split over waves (attn_key_split).
   bool key_split = false;
-  int rows = 0;  // the whole batch's tokens
+  int rows = 0;  // the whole batch's tokens (inference)
   Workspace w;
   const int32_t *ids, *pos, *opt;
   hipStream_t s;
@@ -1173,6 +1173,7 @@ int forward_core(dn_ctx *c, int nseq, const int32_t *seq_len, const int32_t *d_i
   ps.pos = d_pos;
   ps.opt = d_opt;
   ps.s = c->stream;
+  ps.rows = train ? 0 : T;
   ps.fold = !train && w.lmean1 && fold_eligible(c, T);
   ps.ln_cols = T <= kLnNarrowTokens ? kLnPartNarrow : kLnPartWide;
   // Training keeps the tile walk in bf16: its gradients cancel over a

@@ -1613,11 +1613,17 @@ hipError_t launch_gemm16(int epi, const GemmArgs &a, hipStream_t s, const LnFold
 // on the 256 CUs (K = 768, N = 2304: 1,472 rows 70 against 104 us, 2,048 rows
 // 95 / 105, 3,000 rows 135 / 105, 4,000 rows 178 / 205; N = 768, 4,000 rows 64 /
 // 104), for longer K 18 (K = 1152, 1,700 rows 130 / 149, 2,200 rows 163 / 151; K =
-// 1536, 2,200 rows 204 / 197). The two sum in different orders, so the parts of a two-stream forward
-// choose by the whole batch's rows.
+// 1536, 2,200 rows 204 / 197). A forward of 8,192 tokens or more runs as two
+// parts that share the CUs, where CU time counts and the large tiles take three
+// fifths of the small ones' (N = 768 on small / large: 4 x 2,800 tokens 34.9 /
+// 33.1 ms, 11 x 1,000 29.8 / 26.7, 26 x 512 31.4 / 29.2). The two sum in
+// different orders, so a forward chooses by the whole batch's rows, in parts or
+// not.
+constexpr int kF32SharedRows = 8192;
 bool f32_small_tiles(int epi, const GemmArgs &a) {
   if (epi == EPI_GEGLU_BWD) return false;
   if (epi == EPI_GEGLU_KEEP) return a.M <= 1024;
+  if (a.rows >= kF32SharedRows) return false;
   const long long M = a.rows ? a.rows : a.M;
   const long long r32 = ((M + 31) / 32 * (a.N / 32) + kCUs - 1) / kCUs;
   const long long rt = ((M + 255) / 256 * (a.N / 128) + kCUs - 1) / kCUs;
